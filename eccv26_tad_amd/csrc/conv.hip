@@ -176,11 +176,32 @@ extern "C" int svtad_fwd(const void* x, const int32_t* nbr, const void* weight, 
     return launch_status();
 }
 
+// The words that the scan for entries without their symmetric partner writes
+// after svtad_bwd_in_workspace_bytes (rounded up to 16).
+static size_t bwd_in_scan_at(int dtype, int c_in, int c_out) { return cdiv(bwd_in_ws(dtype, c_in, c_out), 16) * 16; }
+
+extern "C" size_t svtad_bwd_in_ex_workspace_bytes(int64_t n, int c_in, int c_out, int dtype) {
+    if (!dtype_ok(dtype) || c_in <= 0 || c_out <= 0 || n < 0) return 0;
+    return bwd_in_scan_at(dtype, c_in, c_out) + (size_t)cdiv(n, kOrphanScanRows) * 4;
+}
+
+static int check_table_flags(const char* what, unsigned flags);
+
 extern "C" int svtad_bwd_in(const void* grad_out, const int32_t* nbr, const void* weight,
                             void* grad_in, void* workspace, size_t workspace_bytes, int64_t n,
                             int c_in, int c_out, int64_t tokens_per_batch, int dtype, void* stream) {
+    return svtad_bwd_in_ex(grad_out, nbr, weight, grad_in, workspace, workspace_bytes, n, c_in, c_out,
+                           tokens_per_batch, dtype, 0u, stream);
+}
+
+extern "C" int svtad_bwd_in_ex(const void* grad_out, const int32_t* nbr, const void* weight,
+                               void* grad_in, void* workspace, size_t workspace_bytes, int64_t n,
+                               int c_in, int c_out, int64_t tokens_per_batch, int dtype,
+                               unsigned table_flags, void* stream) {
     int st = check_common("bwd_in", n, c_in, c_out, tokens_per_batch, dtype);
+    if (!st) st = check_table_flags("bwd_in", table_flags);
     if (st) return st;
+    const bool sym = table_flags & SVTAD_TABLE_SYMMETRIC;
     const size_t need = bwd_in_ws(dtype, c_in, c_out);
     if (need && (!workspace || workspace_bytes < need))
         return set_error(SVTAD_ERR_WORKSPACE, "bwd_in: workspace smaller than svtad_bwd_in_workspace_bytes()");
@@ -194,12 +215,24 @@ extern "C" int svtad_bwd_in(const void* grad_out, const int32_t* nbr, const void
     if (gg_mfma_supported(dtype, c_out, c_in) && al16(grad_out) && al16(weight) && al16(grad_in) &&
         (!need || al16(workspace)))
         flagged = gg_mfma(dtype, MODE_BWDIN, grad_out, nbr, weight, nullptr, 0, grad_in, n, c_out, c_in,
-                          tokens_per_batch, need ? workspace : nullptr, false, flag, s);
+                          tokens_per_batch, need ? workspace : nullptr, false, flag, s, sym);
     else
         gg_valu(dtype, MODE_BWDIN, grad_out, nbr, weight, nullptr, 0, grad_in, n, c_out, c_in,
                 tokens_per_batch, s);
-    orphans(dtype, false, grad_out, nbr, weight, grad_in, n, c_in, c_out, tokens_per_batch,
-            flagged ? flag : nullptr, s);
+    if (sym) return launch_status();  // no entries without a partner
+    // kernels that keep no flag: a scan of the table over the whole chip sets
+    // one word per block where the workspace has room for them (see k_orphans)
+    int64_t n_flags = 1;
+    if (!flagged) {
+        flag = nullptr;
+        if (workspace && workspace_bytes >= svtad_bwd_in_ex_workspace_bytes(n, c_in, c_out, dtype) &&
+            ((uintptr_t)workspace & 3) == 0) {
+            flag = (uint32_t*)((char*)workspace + bwd_in_scan_at(dtype, c_in, c_out));
+            n_flags = cdiv(n, kOrphanScanRows);
+            orphan_scan(nbr, n, tokens_per_batch, flag, s);
+        }
+    }
+    orphans(dtype, false, grad_out, nbr, weight, grad_in, n, c_in, c_out, tokens_per_batch, flag, s, n_flags);
     return launch_status();
 }
 

@@ -119,17 +119,44 @@ __global__ __launch_bounds__(256) void k_gg_valu(const T* __restrict__ src,
 // not in the table are not covered by the transposed gather; the rows they
 // reach are recomputed here (after the gather kernel has stored gi) by one
 // workgroup, in fp32 with one rounding and a fixed order (orphan_exact).
-// Tables built from a keep mask have none: with the flag the launch returns
-// at once, without it the workgroup only scans the table.
+// Tables built from a keep mask have none: with the flag words (one of the
+// backward-input kernel, or one per workgroup of k_orphan_scan) all 0 the
+// launch returns at once, without them the workgroup scans the table itself,
+// one dependent pair of loads per 256 entries (775 us at 21952 rows).
 // ---------------------------------------------------------------------------
 template <typename T, bool DEPTHWISE>
 __global__ __launch_bounds__(256) void k_orphans(const T* __restrict__ go,
                                                  const int32_t* __restrict__ nbr,
                                                  const T* __restrict__ w, T* __restrict__ gi,
                                                  int64_t n, int c_in, int c_out, int64_t tpb,
-                                                 const uint32_t* __restrict__ flag) {
-    if (flag && *flag == 0u) return;  // no entry without a symmetric partner
+                                                 const uint32_t* __restrict__ flag, int64_t n_flags) {
+    if (flag) {  // no entry without a symmetric partner: done
+        int any = 0;
+        for (int64_t q = threadIdx.x; q < n_flags; q += 256) any |= flag[q] != 0u ? 1 : 0;
+        if (__syncthreads_or(any) == 0) return;
+    }
     orphan_exact<T, DEPTHWISE, 256>(go, nbr, w, gi, n, c_in, c_out, tpb);
+}
+
+// flags[b] = whether one of rows [256 b, 256 b + 256) has an entry without its
+// symmetric partner (written by every launch: no clearing). Bound by two
+// dependent reads of the table (36 N bytes and their partners).
+__global__ __launch_bounds__(256) void k_orphan_scan(const int32_t* __restrict__ nbr, int64_t n, int64_t tpb,
+                                                     uint32_t* __restrict__ flags) {
+    const int64_t e0 = (int64_t)blockIdx.x * (kOrphanScanRows * 9);
+    const int64_t e1 = min<int64_t>(n * 9, e0 + kOrphanScanRows * 9);
+    int any = 0;
+#pragma unroll
+    for (int q = 0; q < kOrphanScanRows * 9 / 256; ++q) {
+        const int64_t e = e0 + q * 256 + threadIdx.x;
+        if (e >= e1) break;
+        const int64_t i = e / 9;
+        const int k = (int)(e - i * 9);
+        const int64_t j = src_row(nbr, i, k, n, tpb);
+        any |= j >= 0 && src_row(nbr, j, 8 - k, n, tpb) != i ? 1 : 0;
+    }
+    const int r = __syncthreads_or(any);
+    if (threadIdx.x == 0) flags[blockIdx.x] = r ? 1u : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -717,25 +744,29 @@ void gg_valu(int dtype, int mode, const void* src, const int32_t* nbr, const voi
 
 template <typename T>
 static void launch_orphans(bool dw, const void* go, const int32_t* nbr, const void* w, void* gi,
-                           int64_t n, int c_in, int c_out, int64_t tpb, const uint32_t* flag,
+                           int64_t n, int c_in, int c_out, int64_t tpb, const uint32_t* flag, int64_t n_flags,
                            hipStream_t s) {
     // one workgroup (the pass is exact and ordered, orphan_exact)
     dim3 grid(1);
     if (dw)
         hipLaunchKernelGGL((k_orphans<T, true>), grid, dim3(256), 0, s, (const T*)go, nbr,
-                           (const T*)w, (T*)gi, n, c_in, c_out, tpb, flag);
+                           (const T*)w, (T*)gi, n, c_in, c_out, tpb, flag, n_flags);
     else
         hipLaunchKernelGGL((k_orphans<T, false>), grid, dim3(256), 0, s, (const T*)go, nbr,
-                           (const T*)w, (T*)gi, n, c_in, c_out, tpb, flag);
+                           (const T*)w, (T*)gi, n, c_in, c_out, tpb, flag, n_flags);
+}
+
+void orphan_scan(const int32_t* nbr, int64_t n, int64_t tpb, uint32_t* flags, hipStream_t s) {
+    hipLaunchKernelGGL(k_orphan_scan, dim3((unsigned)cdiv(n, kOrphanScanRows)), dim3(256), 0, s, nbr, n, tpb, flags);
 }
 
 void orphans(int dtype, bool dw, const void* go, const int32_t* nbr, const void* w, void* gi,
-             int64_t n, int c_in, int c_out, int64_t tpb, const uint32_t* flag, hipStream_t s) {
+             int64_t n, int c_in, int c_out, int64_t tpb, const uint32_t* flag, hipStream_t s, int64_t n_flags) {
     switch (dtype) {
-        case SVTAD_F32: launch_orphans<float>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, s); break;
-        case SVTAD_F16: launch_orphans<f16>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, s); break;
-        case SVTAD_BF16: launch_orphans<bf16>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, s); break;
-        case SVTAD_F64: launch_orphans<double>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, s); break;
+        case SVTAD_F32: launch_orphans<float>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, n_flags, s); break;
+        case SVTAD_F16: launch_orphans<f16>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, n_flags, s); break;
+        case SVTAD_BF16: launch_orphans<bf16>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, n_flags, s); break;
+        case SVTAD_F64: launch_orphans<double>(dw, go, nbr, w, gi, n, c_in, c_out, tpb, flag, n_flags, s); break;
     }
 }
 

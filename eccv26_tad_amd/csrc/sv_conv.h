@@ -27,11 +27,14 @@ void gg_valu(int dtype, int mode, const void* src, const int32_t* nbr, const voi
              int64_t tpb, hipStream_t s);
 // Backward-input contributions of table entries (i, k) -> j whose symmetric
 // partner (j, 8-k) -> i is absent (the gathered kernels cannot see them),
-// added with atomics. With a non-NULL flag the pass returns at once when the
-// flag is 0 (the wide backward-input kernel sets it when it meets such an
-// entry; the pack kernels clear it).
+// added with atomics. With a non-NULL flag the pass returns at once when its
+// n_flags words are 0 (the wide backward-input kernel sets its one word when
+// it meets such an entry, and the pack kernels clear it; orphan_scan writes
+// one word per kOrphanScanRows rows).
 void orphans(int dtype, bool dw, const void* go, const int32_t* nbr, const void* w, void* gi,
-             int64_t n, int c_in, int c_out, int64_t tpb, const uint32_t* flag, hipStream_t s);
+             int64_t n, int c_in, int c_out, int64_t tpb, const uint32_t* flag, hipStream_t s, int64_t n_flags = 1);
+constexpr int kOrphanScanRows = 256;
+void orphan_scan(const int32_t* nbr, int64_t n, int64_t tpb, uint32_t* flags, hipStream_t s);
 void bw_valu(int dtype, const BwPlan& p, const void* go, const void* x, const int32_t* nbr,
              void* gw, void* gb, void* ws, int64_t n, int c_in, int c_out, int64_t tpb,
              hipStream_t s);

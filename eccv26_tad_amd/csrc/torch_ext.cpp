@@ -202,10 +202,12 @@ at::Tensor op_fwd_packed(const at::Tensor& x_in, const at::Tensor& nbr_in, const
     return out;
 }
 
-// bwd_in(grad_output, neighbor_indices, weight, n_kept, C_in, tokens_per_batch)
-// -> [n_kept, C_in] in grad_output's dtype (2d_sparse_v3.cu:824-835)
-at::Tensor op_bwd_in(const at::Tensor& go_in, const at::Tensor& nbr_in, const at::Tensor& w_in,
-                     int64_t n_kept, int64_t c_in, int64_t tpb) {
+// table_flags from the `symmetric` keyword of the backward ops: the caller's
+// promise that every table entry has its partner (SVTAD_TABLE_SYMMETRIC)
+static unsigned table_flags(bool symmetric) { return symmetric ? (unsigned)SVTAD_TABLE_SYMMETRIC : 0u; }
+
+static at::Tensor bwd_in_raw(const at::Tensor& go_in, const at::Tensor& nbr_in, const at::Tensor& w_in,
+                             int64_t n_kept, int64_t c_in, int64_t tpb, bool symmetric) {
     check_gpu(go_in, "grad_output");
     check_gpu(w_in, "weight");
     at::Tensor go = rows_view(go_in);
@@ -219,19 +221,23 @@ at::Tensor op_bwd_in(const at::Tensor& go_in, const at::Tensor& nbr_in, const at
     c10::DeviceGuard g(go.device());
     at::Tensor gi = at::empty({n_kept, c_in}, go.options());
     const int dt = dtype_code(go);
-    const size_t ws_bytes = svtad_bwd_in_workspace_bytes((int)c_in, (int)c_out, dt);
+    const size_t ws_bytes = symmetric ? svtad_bwd_in_workspace_bytes((int)c_in, (int)c_out, dt)
+                                      : svtad_bwd_in_ex_workspace_bytes(n_kept, (int)c_in, (int)c_out, dt);
     at::Tensor ws;
     if (ws_bytes && n_kept > 0) ws = at::empty({(int64_t)ws_bytes}, go.options().dtype(at::kByte));
-    const int st = svtad_bwd_in(go.data_ptr(), nbr.data_ptr<int32_t>(), w.data_ptr(), gi.data_ptr(),
-                                ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, n_kept, (int)c_in,
-                                (int)c_out, tpb, dt, stream_of(go));
+    const int st = svtad_bwd_in_ex(go.data_ptr(), nbr.data_ptr<int32_t>(), w.data_ptr(), gi.data_ptr(),
+                                   ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, n_kept, (int)c_in,
+                                   (int)c_out, tpb, dt, table_flags(symmetric), stream_of(go));
     check_status(st, "bwd_in");
     return gi;
 }
 
-// table_flags from the `symmetric` keyword of the backward ops: the caller's
-// promise that every table entry has its partner (SVTAD_TABLE_SYMMETRIC)
-static unsigned table_flags(bool symmetric) { return symmetric ? (unsigned)SVTAD_TABLE_SYMMETRIC : 0u; }
+// bwd_in(grad_output, neighbor_indices, weight, n_kept, C_in, tokens_per_batch)
+// -> [n_kept, C_in] in grad_output's dtype (2d_sparse_v3.cu:824-835)
+at::Tensor op_bwd_in(const at::Tensor& go, const at::Tensor& nbr, const at::Tensor& w, int64_t n_kept,
+                     int64_t c_in, int64_t tpb) {
+    return bwd_in_raw(go, nbr, w, n_kept, c_in, tpb, false);
+}
 
 // bwd_in_packed(grad_output, neighbor_indices, weight, packed_bwd, n_kept, C_in,
 // tokens_per_batch, symmetric=False): bwd_in with a weight packed by
@@ -240,7 +246,7 @@ static unsigned table_flags(bool symmetric) { return symmetric ? (unsigned)SVTAD
 at::Tensor op_bwd_in_packed(const at::Tensor& go_in, const at::Tensor& nbr_in, const at::Tensor& w_in,
                             const at::Tensor& packed, int64_t n_kept, int64_t c_in, int64_t tpb,
                             bool symmetric) {
-    if (packed.numel() == 0) return op_bwd_in(go_in, nbr_in, w_in, n_kept, c_in, tpb);
+    if (packed.numel() == 0) return bwd_in_raw(go_in, nbr_in, w_in, n_kept, c_in, tpb, symmetric);
     check_gpu(go_in, "grad_output");
     at::Tensor go = rows_view(go_in);
     const int64_t c_out = go.size(-1);
@@ -258,7 +264,7 @@ at::Tensor op_bwd_in_packed(const at::Tensor& go_in, const at::Tensor& nbr_in, c
     const int st = svtad_bwd_in_packed_ex(go.data_ptr(), nbr.data_ptr<int32_t>(), w.data_ptr(),
                                           packed.data_ptr(), gi.data_ptr(), n_kept, (int)c_in,
                                           (int)c_out, tpb, dt, table_flags(symmetric), stream_of(go));
-    if (st == SVTAD_ERR_UNSUPPORTED) return op_bwd_in(go_in, nbr_in, w_in, n_kept, c_in, tpb);
+    if (st == SVTAD_ERR_UNSUPPORTED) return bwd_in_raw(go_in, nbr_in, w_in, n_kept, c_in, tpb, symmetric);
     check_status(st, "bwd_in_packed");
     return gi;
 }

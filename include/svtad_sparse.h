@@ -120,6 +120,16 @@ int svtad_bwd_in(const void* grad_out, const int32_t* nbr, const void* weight, v
                  void* workspace, size_t workspace_bytes, int64_t n, int c_in, int c_out,
                  int64_t tokens_per_batch, int dtype, void* stream);
 
+/* svtad_bwd_in with table_flags (svtad_table_flags; 0 = the same call). A
+ * workspace of svtad_bwd_in_ex_workspace_bytes() (at least
+ * svtad_bwd_in_workspace_bytes(), plus a word per 256 rows) lets the check for
+ * entries without their symmetric partner run over the whole GPU in the
+ * shapes whose kernels do not make it; both calls take either size. */
+size_t svtad_bwd_in_ex_workspace_bytes(int64_t n, int c_in, int c_out, int dtype);
+int svtad_bwd_in_ex(const void* grad_out, const int32_t* nbr, const void* weight, void* grad_in,
+                    void* workspace, size_t workspace_bytes, int64_t n, int c_in, int c_out,
+                    int64_t tokens_per_batch, int dtype, unsigned table_flags, void* stream);
+
 /*
  * Pre-packed weights (no counterpart in the reference; the autograd wrapper
  * packs once per forward and reuses the backward layout, where the entry

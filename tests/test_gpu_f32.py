@@ -1,0 +1,86 @@
+"""The float32 layer's kernels against a float64 scatter over the table's
+entries, at row counts and widths around the kernels' blocks and tiles."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import random_mask
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def sv():
+    import eccv26_tad_amd as sv
+
+    return sv
+
+
+def _table(rng, n, one_way):
+    """Symmetric table [n, 9] (int32) of a random mask cut to n rows, with
+    ``one_way`` entries whose partner is removed."""
+    import eccv26_tad_amd as sv
+
+    side = 1 + int(np.ceil(np.sqrt(n / 0.5 / 4)))
+    mask = np.zeros((1, 4, side, side), dtype=np.uint8)
+    while mask.sum() < n:
+        mask = random_mask(rng, 1, 4, side, side, min(1.0, 0.6))
+        side += 1
+    t = sv.build_neighbor_table(torch.from_numpy(mask).cuda()).cpu().numpy()[:n]
+    t[t >= n] = -1
+    pairs = np.argwhere((t >= 0) & (np.arange(9) != 4))
+    for i, k in pairs[rng.permutation(len(pairs))[:one_way]]:
+        t[t[i, k], 8 - k] = -1
+    if one_way:  # the last row too: the last, partly filled block
+        t[n - 1, 0], t[0, 8] = 0, -1
+    return t
+
+
+def _exact(t, x, w, b, go):
+    """(y, gi, gw, gb, and the same sums of absolute terms) in float64."""
+    n = len(x)
+    out = []
+    for f in (lambda v: v, np.abs):
+        x_, w_, go_, b_ = f(x), f(w), f(go), f(b)
+        y = np.tile(b_, (n, 1))
+        gi = np.zeros_like(x_)
+        gw = np.zeros_like(w_)
+        for k in range(9):
+            i = np.nonzero(t[:, k] >= 0)[0]
+            j = t[i, k]
+            y[i] += x_[j] @ w_[k]
+            np.add.at(gi, j, go_[i] @ w_[k].T)
+            gw[k] = x_[j].T @ go_[i]
+        out.append((y, gi, gw, go_.sum(0)))
+    return out
+
+
+def _check(name, got, exact, mag, terms):
+    # an fp32 sum of `terms` products in any order: each addition rounds by at
+    # most 2^-24 of the sum of absolute terms
+    err = np.abs(got.double().cpu().numpy() - exact)
+    bar = 2.0 ** -24 * (terms + 2) * mag + 1e-30
+    assert (err <= bar).all(), (name, float((err / bar).max()))
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1000])
+@pytest.mark.parametrize("one_way", [0, 3])
+@pytest.mark.parametrize("dname", ["f32", "f64"])
+def test_backward_input_finds_one_way_entries(sv, n, one_way, dname):
+    rng = np.random.default_rng(n + one_way)
+    t = _table(rng, n, one_way)
+    ci, co = 8, 12
+    dt = {"f32": torch.float32, "f64": torch.float64}[dname]
+    x, w, go, b = (rng.standard_normal(s).astype(np.float32).astype(np.float64)
+                   for s in ((n, ci), (9, ci, co), (n, co), (co,)))
+    (_, gi, _, _), (_, mag, _, _) = _exact(t, x, w, b, go)
+    dev = [torch.from_numpy(v).to("cuda", dt) for v in (go, w)]
+    tab = torch.from_numpy(t).cuda()
+    got = sv.ops.bwd_in(dev[0], tab, dev[1], n, ci, 0)
+    _check("gi", got, gi, mag, 9 * co)
+    if not one_way:
+        empty = torch.empty(0, dtype=torch.uint8, device="cuda")
+        same = sv.ops.bwd_in_packed(dev[0], tab, dev[1], empty, n, ci, 0, symmetric=True)
+        assert torch.equal(same, got)
