@@ -170,6 +170,10 @@ extern "C" int svtad_fwd(const void* x, const int32_t* nbr, const void* weight, 
         (!need || al16(workspace)))
         gg_mfma(dtype, MODE_FWD, x, nbr, weight, bias, bias_mode, out, n, c_in, c_out,
                 tokens_per_batch, need ? workspace : nullptr, false, nullptr, s);
+    else if (dtype == SVTAD_F32 && gg_f32_supported(n, c_in, c_out) && al16(x) && al16(weight) && al16(out))
+        // every bias mode adds the fp32 bias to the fp32 sum
+        gg_f32(MODE_FWD, x, nbr, weight, bias_mode == SVTAD_BIAS_NONE ? nullptr : bias, out, n, c_in, c_out,
+               tokens_per_batch, false, s);
     else
         gg_valu(dtype, MODE_FWD, x, nbr, weight, bias, bias_mode, out, n, c_in, c_out,
                 tokens_per_batch, s);
@@ -216,6 +220,9 @@ extern "C" int svtad_bwd_in_ex(const void* grad_out, const int32_t* nbr, const v
         (!need || al16(workspace)))
         flagged = gg_mfma(dtype, MODE_BWDIN, grad_out, nbr, weight, nullptr, 0, grad_in, n, c_out, c_in,
                           tokens_per_batch, need ? workspace : nullptr, false, flag, s, sym);
+    else if (dtype == SVTAD_F32 && gg_f32_supported(n, c_out, c_in) && al16(grad_out) && al16(weight) &&
+             al16(grad_in))
+        gg_f32(MODE_BWDIN, grad_out, nbr, weight, nullptr, grad_in, n, c_out, c_in, tokens_per_batch, sym, s);
     else
         gg_valu(dtype, MODE_BWDIN, grad_out, nbr, weight, nullptr, 0, grad_in, n, c_out, c_in,
                 tokens_per_batch, s);

@@ -25,6 +25,12 @@ struct BwPlan {
 void gg_valu(int dtype, int mode, const void* src, const int32_t* nbr, const void* w,
              const void* bias, int bias_mode, void* out, int64_t n, int c_red, int n_out,
              int64_t tpb, hipStream_t s);
+// float32 gathered GEMM on the matrix cores: the widths and row counts it
+// takes (16-byte aligned operands besides), and the launch. bias may be NULL;
+// sym as for gg_mfma.
+bool gg_f32_supported(int64_t n, int c_red, int n_out);
+void gg_f32(int mode, const void* src, const int32_t* nbr, const void* w, const void* bias, void* out, int64_t n,
+            int c_red, int n_out, int64_t tpb, bool sym, hipStream_t s);
 // Backward-input contributions of table entries (i, k) -> j whose symmetric
 // partner (j, 8-k) -> i is absent (the gathered kernels cannot see them),
 // added with atomics. With a non-NULL flag the pass returns at once when its

@@ -84,3 +84,24 @@ def test_backward_input_finds_one_way_entries(sv, n, one_way, dname):
         empty = torch.empty(0, dtype=torch.uint8, device="cuda")
         same = sv.ops.bwd_in_packed(dev[0], tab, dev[1], empty, n, ci, 0, symmetric=True)
         assert torch.equal(same, got)
+
+
+@pytest.mark.parametrize("n,ci,co", [(1, 4, 4), (15, 16, 32), (33, 48, 48), (129, 20, 36), (200, 64, 40),
+                                     (257, 100, 128), (300, 128, 96), (1500, 36, 200), (4099, 64, 64)])
+@pytest.mark.parametrize("one_way", [0, 2])
+def test_layer_matches_float64(sv, n, ci, co, one_way):
+    """Forward with bias and backward-input in float32."""
+    rng = np.random.default_rng(n + ci + one_way)
+    t = _table(rng, n, one_way)
+    x, w, go, b = (rng.standard_normal(s).astype(np.float32).astype(np.float64)
+                   for s in ((n, ci), (9, ci, co), (n, co), (co,)))
+    (y, gi, gw, gb), (my, mgi, mgw, mgb) = _exact(t, x, w, b, go)
+    X, W, GO, B = (torch.from_numpy(v).to("cuda", torch.float32) for v in (x, w, go, b))
+    tab = torch.from_numpy(t).cuda()
+    for mode in (1, 2):
+        _check("y", sv.ops.fwd_bias(X, tab, W, B, 0, mode), y, my, 9 * ci + 1)
+    _check("y - b", sv.ops.fwd(X, tab, W, co, 0), y - b, my, 9 * ci + 1)
+    _check("gi", sv.ops.bwd_in(GO, tab, W, n, ci, 0), gi, mgi, 9 * co)
+    if not one_way:
+        empty = torch.empty(0, dtype=torch.uint8, device="cuda")
+        _check("gi", sv.ops.bwd_in_packed(GO, tab, W, empty, n, ci, 0, symmetric=True), gi, mgi, 9 * co)
