@@ -46,6 +46,13 @@ static int check_common(const char* who, int64_t n, int c_in, int c_out, int64_t
 // rows.
 static BwPlan plan_bw(int64_t n, int c_in, int c_out, int dtype) {
     BwPlan p;
+    if (dtype == SVTAD_F32 && n > 0 && bw_f32_supported(n, c_in, c_out)) {
+        p.path = 2;
+        p.rows_per_split = bw_f32_rows_per_split(n, c_in, c_out);
+        p.splits = (int)cdiv(n, p.rows_per_split);
+        p.ws_bytes = (size_t)p.splits * ((size_t)9 * c_in * c_out + c_out) * 4;
+        return p;
+    }
     p.path = bw_mfma_supported(dtype, n, c_in, c_out) ? 1 : 0;
     int tm = 64, tn = 64;
     bool big = false;
@@ -365,7 +372,8 @@ extern "C" int svtad_bwd_w(const void* grad_out, const void* x, const int32_t* n
     // grad_w NULL: only the row-split partial sums are written (to workspace)
     if (!workspace || (n > 0 && (!grad_out || !x || !nbr)))
         return set_error(SVTAD_ERR_INVALID, "bwd_w: null pointer");
-    if (p.path == 1 && !(al16(grad_out) && al16(x))) p.path = 0;  // same workspace layout
+    if (p.path != 0 && !(al16(grad_out) && al16(x))) p.path = 0;  // same workspace layout
+    if (p.path == 2 && !(al16(workspace) && al16(grad_w) && al16(grad_bias))) p.path = 0;
     if (workspace_bytes < p.ws_bytes)
         return set_error(SVTAD_ERR_WORKSPACE, "bwd_w: workspace smaller than svtad_bwd_w_workspace_bytes()");
     hipStream_t s = (hipStream_t)stream;
@@ -374,7 +382,9 @@ extern "C" int svtad_bwd_w(const void* grad_out, const void* x, const int32_t* n
         st = bw_mfma(dtype, p, grad_out, x, nbr, grad_w, grad_bias, workspace, workspace_bytes, n, c_in, c_out,
                      tokens_per_batch, nullptr, &unused, s);
         if (st) return st;
-    } else
+    } else if (p.path == 2)
+        bw_f32(p, grad_out, x, nbr, grad_w, grad_bias, workspace, n, c_in, c_out, tokens_per_batch, s);
+    else
         bw_valu(dtype, p, grad_out, x, nbr, grad_w, grad_bias, workspace, n, c_in, c_out,
                 tokens_per_batch, s);
     return launch_status();

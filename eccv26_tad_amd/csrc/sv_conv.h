@@ -15,7 +15,7 @@ enum { MODE_FWD = 0, MODE_BWDIN = 1 };
 // [splits][9][c_in][c_out] (+ [splits][c_out] for the bias) in the
 // accumulator type.
 struct BwPlan {
-    int path;                 // 0 = VALU, 1 = MFMA
+    int path;                 // 0 = VALU, 1 = MFMA (f16 / bf16), 2 = float32 MFMA
     int splits;
     int64_t rows_per_split;
     size_t ws_bytes;
@@ -31,6 +31,13 @@ void gg_valu(int dtype, int mode, const void* src, const int32_t* nbr, const voi
 bool gg_f32_supported(int64_t n, int c_red, int n_out);
 void gg_f32(int mode, const void* src, const int32_t* nbr, const void* w, const void* bias, void* out, int64_t n,
             int c_red, int n_out, int64_t tpb, bool sym, hipStream_t s);
+// float32 backward-weight on the matrix cores (n >= 1): the shapes it takes
+// (16-byte aligned operands besides), its splits, and the launch (gw NULL:
+// partials only; gb NULL: no bias).
+bool bw_f32_supported(int64_t n, int c_in, int c_out);
+int64_t bw_f32_rows_per_split(int64_t n, int c_in, int c_out);
+void bw_f32(const BwPlan& p, const void* go, const void* x, const int32_t* nbr, void* gw, void* gb, void* ws, int64_t n,
+            int c_in, int c_out, int64_t tpb, hipStream_t s);
 // Backward-input contributions of table entries (i, k) -> j whose symmetric
 // partner (j, 8-k) -> i is absent (the gathered kernels cannot see them),
 // added with atomics. With a non-NULL flag the pass returns at once when its

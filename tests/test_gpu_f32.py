@@ -90,7 +90,7 @@ def test_backward_input_finds_one_way_entries(sv, n, one_way, dname):
                                      (257, 100, 128), (300, 128, 96), (1500, 36, 200), (4099, 64, 64)])
 @pytest.mark.parametrize("one_way", [0, 2])
 def test_layer_matches_float64(sv, n, ci, co, one_way):
-    """Forward with bias and backward-input in float32."""
+    """Forward with bias, backward-input and backward-weight in float32."""
     rng = np.random.default_rng(n + ci + one_way)
     t = _table(rng, n, one_way)
     x, w, go, b = (rng.standard_normal(s).astype(np.float32).astype(np.float64)
@@ -102,6 +102,11 @@ def test_layer_matches_float64(sv, n, ci, co, one_way):
         _check("y", sv.ops.fwd_bias(X, tab, W, B, 0, mode), y, my, 9 * ci + 1)
     _check("y - b", sv.ops.fwd(X, tab, W, co, 0), y - b, my, 9 * ci + 1)
     _check("gi", sv.ops.bwd_in(GO, tab, W, n, ci, 0), gi, mgi, 9 * co)
+    for bias in (True, False):
+        got_w, got_b = sv.ops.bwd_w_bias(GO, X, tab, ci, 0, bias)
+        _check("gw", got_w, gw, mgw, n)
+        if bias:
+            _check("gb", got_b, gb, mgb, n)
     if not one_way:
         empty = torch.empty(0, dtype=torch.uint8, device="cuda")
         _check("gi", sv.ops.bwd_in_packed(GO, tab, W, empty, n, ci, 0, symmetric=True), gi, mgi, 9 * co)
