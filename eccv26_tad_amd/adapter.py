@@ -87,6 +87,7 @@ the unfused chain in the reference's op order.
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -255,7 +256,7 @@ class SparseConvAdapterFunction(Function):
 
     @staticmethod
     def forward(ctx, x, w_d, b_d, w_c, b_c, w_u, b_u, gamma, nbr, n_special, tpb, hm_rows=None, hm_gate=None,
-                packed=None, cd=None):
+                packed=None, cd=None, keep_packed=None):
         S = int(n_special)
         ctx.symmetric = is_symmetric_table(nbr)
         cd = x.dtype if cd is None else cd
@@ -263,40 +264,70 @@ class SparseConvAdapterFunction(Function):
         # the heatmap gate keep their dtype, as in the reference chain
         params = (w_d, b_d, w_c, b_c, w_u, b_u, gamma, hm_gate)
         ctx.dtypes = tuple(None if t is None else t.dtype for t in (x,) + params)
-        xc = _cast(x, cd)
-        w_d, b_d, w_c, b_c, w_u, b_u = (_cast(t, cd) for t in (w_d, b_d, w_c, b_c, w_u, b_u))
-        pre, sp, pa = _ops.adapter_down(xc, w_d, b_d, S)
-        if hm_rows is not None:
-            # heatmap injection on the SparseConv2D input (in place)
-            _ops.heatmap_add_(pa, sp, hm_rows, hm_gate)
+        need_bwd = any(ctx.needs_input_grad)
         c_in = w_c.shape[1]
         if c_in % 4 != 0:
             raise ValueError(f"C_in ({c_in}) must be divisible by 4 for optimized kernel.")
         mode = BIAS_NONE if b_c is None else (BIAS_FP32 if c_in >= IMPLICIT_GEMM_MIN_CIN else BIAS_AFTER)
-        need_bwd = any(ctx.needs_input_grad)
-        if packed is None or (need_bwd and packed[1] is None):
-            packed = _ops.pack_weight(w_c, True, need_bwd)
-        pf, pb = packed
-        processed = _ops.fwd_packed(pa, nbr, w_c, pf, b_c, tpb, mode)
+        has_bd = b_d is not None
         # z * gamma + x: float32 when gamma is a float32 parameter (the
         # reference's dtype promotion under autocast), else in cd
-        out = _ops.adapter_up(sp, processed, w_u, b_u, gamma, x, gamma.dtype == torch.float32 and cd != gamma.dtype)
-        ctx.save_for_backward(xc, w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma, hm_rows, hm_gate)
-        ctx.flags = (S, int(tpb), b_d is not None)
+        out32 = gamma.dtype == torch.float32 and cd != gamma.dtype
+        rows = w_c.shape[2] == c_in and _ops.adapter_rows_ok(x.shape[-1], c_in)
+        w_dt = w_ut = None
+        if rows:
+            pack = packed is None or (need_bwd and packed[1] is None)
+            wd, b_d, wu, b_u_c, b_c_c, w_c, w_u_c, w_dt, w_ut, pf, pb = _ops.adapter_prep(
+                w_d, b_d, w_c, b_c, w_u, b_u, gamma, cd == torch.bfloat16, need_bwd, pack)
+            if not pack:
+                pf, pb = packed
+            elif keep_packed is not None:
+                keep_packed(pf, pb if need_bwd else None)
+            w_u, b_c = w_u_c, (None if b_c is None else b_c_c)
+            pre, sp, pa, xc = _ops.adapter_rows_down(x, wd, b_d, c_in, S, need_bwd)
+            if x.dtype == cd:
+                xc = x
+        else:
+            xc = _cast(x, cd)
+            w_d, b_d, w_c, b_c, w_u, b_u = (_cast(t, cd) for t in (w_d, b_d, w_c, b_c, w_u, b_u))
+            pre, sp, pa = _ops.adapter_down(xc, w_d, b_d, S)
+            if packed is None or (need_bwd and packed[1] is None):
+                packed = _ops.pack_weight(w_c, True, need_bwd)
+            pf, pb = packed
+        if hm_rows is not None:
+            # heatmap injection on the SparseConv2D input (in place)
+            _ops.heatmap_add_(pa, sp, hm_rows, hm_gate)
+        processed = _ops.fwd_packed(pa, nbr, w_c, pf, b_c, tpb, mode)
+        if rows:
+            out = _ops.adapter_rows_res(sp, processed, wu, b_u_c, gamma, x, out32)
+            b_u = None if b_u is None else b_u_c
+        else:
+            out = _ops.adapter_up(sp, processed, w_u, b_u, gamma, x, out32)
+        if need_bwd:
+            ctx.save_for_backward(xc, None if rows else w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma,
+                                  hm_rows, hm_gate, w_dt, w_ut)
+        ctx.flags = (S, int(tpb), has_bd)
         return out
 
     @staticmethod
     def backward(ctx, go):
-        x, w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma, hm_rows, hm_gate = ctx.saved_tensors
+        (x, w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma, hm_rows, hm_gate, w_dt,
+         w_ut) = ctx.saved_tensors
         S, tpb, has_bd = ctx.flags
         x_dt, wd_dt, bd_dt, wc_dt, bc_dt, wu_dt, bu_dt, _, _ = ctx.dtypes
         need = ctx.needs_input_grad
         B, N, n = go.shape
-        k = w_u.shape[1]
-        cd = x.dtype
+        k = pre.shape[-1]
+        cd = pre.dtype
         go = go.contiguous()
         go_res = go  # the residual's gradient (float32 under autocast)
-        go = _cast(go, cd)
+        if w_ut is not None:
+            # (go * gamma) W_u with go cast on the way (its cast is kept for
+            # the weight gradients) and the two kinds of rows stored apart
+            g_sp, g_pa, gc = _ops.adapter_rows_split(go, w_ut, k, S, True)
+            go = gc if go.dtype != cd else go
+        else:
+            go = _cast(go, cd)
         go2 = go.reshape(-1, n)
         # up projection: G = go^T cat(sp, processed) without the cat, in fp32
         G = _up_wgrad(go, B, N, S, sp, processed)
@@ -306,9 +337,10 @@ class SparseConvAdapterFunction(Function):
         g_gamma = g_gamma.view(gamma.shape) if need[7] else None
         gw_u = gw_u if need[5] else None
         gb_u = gb_u if b_u is not None and need[6] else None
-        dc = torch.matmul(go, w_u_g)  # [B, N, k]: (go * gamma) W_u
-        g_sp = dc[:, :S]
-        g_pa = dc[:, S:].reshape(-1, k)
+        if w_ut is None:
+            dc = torch.matmul(go, w_u_g)  # [B, N, k]: (go * gamma) W_u
+            g_sp = dc[:, :S]
+            g_pa = dc[:, S:].reshape(-1, k)
         # SparseConv2D
         need_bc = b_c is not None and need[4]
         gi_pa, gw_c, gb_c = _ops.bwd_packed(g_pa, pa, nbr, w_c, pb, w_c.shape[1], tpb, need_bc,
@@ -334,7 +366,11 @@ class SparseConvAdapterFunction(Function):
         x2 = x.reshape(-1, x.shape[-1])
         gx = None
         if need[0]:
-            if x_dt == cd:
+            if w_dt is not None:
+                # du W_d plus the residual's gradient, one rounding
+                gx = _ops.adapter_rows_res(None, du, w_dt, du.new_empty(0), None, go_res if x_dt != cd else go,
+                                           x_dt != cd)
+            elif x_dt == cd:
                 gx = torch.addmm(go2, du2, w_d).view(x.shape)
             else:
                 # float32 x under autocast: the down projection's gradient
@@ -344,7 +380,7 @@ class SparseConvAdapterFunction(Function):
         gb_d = _colsum(du2).to(bd_dt) if has_bd and need[2] else None
         return (gx, gw_d, gb_d, gw_c.to(wc_dt) if need[3] else None,
                 gb_c.to(bc_dt) if need_bc else None, _cast(gw_u, wu_dt), _cast(gb_u, bu_dt), g_gamma,
-                None, None, None, None, g_gate, None, None)
+                None, None, None, None, g_gate, None, None, None)
 
 
 def _trunc_normal_init(layer, std):
@@ -488,12 +524,18 @@ class SparseConvAdapter(nn.Module):
                 hm_rows = (base + cells).reshape(-1).to(torch.int32)
                 hm_gate = self.heatmap_gate
             cache = conv.packed_weight_cache
-            packed = None
+            packed = keep_packed = None
             if cache is not None:
-                packed = cache.get(conv.weight, _cast(conv.weight, cd), torch.is_grad_enabled())
+                if _ops.adapter_rows_ok(self.embed_dims, self.hidden_dims):
+                    # packed with the other parameters' preparation when not current
+                    packed = cache.peek(conv.weight, cd, torch.is_grad_enabled())
+                    keep_packed = functools.partial(cache.put, conv.weight, cd)
+                else:
+                    packed = cache.get(conv.weight, _cast(conv.weight, cd), torch.is_grad_enabled())
             return SparseConvAdapterFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight,
                                                    conv.bias, self.up_proj.weight, self.up_proj.bias, self.gamma,
-                                                   nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd)
+                                                   nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd,
+                                                   keep_packed)
         sp, pa = AdapterDownFunction.apply(x, self.down_proj.weight, self.down_proj.bias, S, cd)
         processed = conv(pa, nbr, tokens_per_batch=tokens_per_batch)
         x_comb = torch.cat([sp, processed.view(B, N - S, -1)], dim=1)

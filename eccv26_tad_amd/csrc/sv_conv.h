@@ -7,6 +7,8 @@
 
 #include <algorithm>
 
+#include "../../include/svtad_sparse.h"
+
 namespace svtad {
 
 enum { MODE_FWD = 0, MODE_BWDIN = 1 };
@@ -66,6 +68,8 @@ void dw_bw(int dtype, const BwPlan& p, const void* go, const void* x, const int3
 bool dw_bwd_fused(int dtype, const BwPlan& p, const void* go, const void* x, const int32_t* nbr, const void* w,
                   void* gi, void* gw, void* gb, void* ws, uint32_t* flags, int64_t n, int c, int64_t tpb,
                   hipStream_t s, bool sym = false);
+
+constexpr int kMaxPrepJobs = SVTAD_MAX_PREP_JOBS;
 
 // out[e] = T(sum_s part[s][e]) for e < count; partials in the accumulator type.
 void split_reduce(int dtype, const void* part, int64_t count, int splits, void* out, hipStream_t s);

@@ -959,6 +959,214 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> op_up_proj_grads(
     return {out, w_sc, g_sc, gs_sc};
 }
 
+// ---------------------------------------------------------------------------
+// The adapter's GEMMs over whole token tiles (svtad_adapter_prep / _rows)
+// ---------------------------------------------------------------------------
+
+// whether the adapter of these widths runs on svtad_adapter_rows
+bool op_adapter_rows_ok(int64_t embed, int64_t hidden) {
+    return svtad_adapter_rows_ok(SVTAD_ROWS_GELU, (int)embed, (int)hidden) &&
+           svtad_adapter_rows_ok(SVTAD_ROWS_SPLIT, (int)embed, (int)hidden) &&
+           svtad_adapter_rows_ok(SVTAD_ROWS_RES, (int)hidden, (int)embed);
+}
+
+// adapter_prep(w_d, b_d, w_c, b_c, w_u, b_u, gamma, bf16, train, pack_conv)
+//   -> [wd, b_d, wu, b_u, b_c, w_c, w_u, wdT, wuT, packed_fwd, packed_bwd]
+// One launch: the parameters (f32 or the compute type) cast, wd / wu in the
+// fragment order of the down / up projection, and with train wdT / wuT in that
+// of the input gradient / the up projection's backward (scaled by gamma), w_u
+// as is; with pack_conv the SparseConv2D layouts of w_c (packed_bwd with
+// train). An item that is not wanted, or a missing bias, is empty.
+std::vector<at::Tensor> op_adapter_prep(const at::Tensor& w_d_in, const c10::optional<at::Tensor>& b_d,
+                                        const at::Tensor& w_c_in, const c10::optional<at::Tensor>& b_c,
+                                        const at::Tensor& w_u_in, const c10::optional<at::Tensor>& b_u,
+                                        const at::Tensor& gamma_in, bool bf16, bool train, bool pack_conv) {
+    const at::ScalarType t = bf16 ? at::kBFloat16 : at::kHalf;
+    const int dt = bf16 ? SVTAD_BF16 : SVTAD_F16;
+    check_gpu(w_d_in, "w_d");
+    auto param = [&](const at::Tensor& p) {
+        TORCH_CHECK(p.is_cuda() && p.device() == w_d_in.device(), "adapter_prep: parameters must share the GPU");
+        TORCH_CHECK(p.scalar_type() == t || p.scalar_type() == at::kFloat,
+                    "adapter_prep: parameters take the compute type or float32, got ", p.scalar_type());
+        return p.contiguous();
+    };
+    at::Tensor w_d = param(w_d_in), w_c = param(w_c_in), w_u = param(w_u_in), gm = param(gamma_in);
+    TORCH_CHECK(w_d.dim() == 2 && w_u.dim() == 2 && w_c.dim() == 3 && w_c.size(0) == 9 && gm.numel() == 1 &&
+                    w_u.size(0) == w_d.size(1) && w_u.size(1) == w_d.size(0) && w_c.size(1) == w_d.size(0) &&
+                    w_c.size(2) == w_d.size(0),
+                "adapter_prep: w_d [h, E], w_c [9, h, h], w_u [E, h] and a gamma of one element");
+    const int64_t h = w_d.size(0), E = w_d.size(1);
+    c10::DeviceGuard g(w_d.device());
+    const auto opt = w_d.options().dtype(t);
+    std::vector<svtad_prep_job> jobs;
+    std::vector<at::Tensor> keep;
+    auto add = [&](int kind, const at::Tensor& src, int off, int64_t n, int64_t k, bool pair, bool scaled, int64_t extra) {
+        at::Tensor dst = at::empty({(int64_t)off * n * k + extra}, opt);
+        jobs.push_back(svtad_prep_job{src.data_ptr(), dst.data_ptr(), scaled ? gm.data_ptr() : nullptr, kind, off, (int)n,
+                                      (int)k, src.scalar_type() == at::kFloat, gm.scalar_type() == at::kFloat, pair});
+        keep.push_back(src);
+        return dst;
+    };
+    auto cast = [&](const at::Tensor& p) {
+        if (p.scalar_type() == t) return ((uintptr_t)p.data_ptr() & 15) ? p.clone() : p;
+        if (p.numel() % 8) return p.to(t);
+        return add(SVTAD_PREP_CAST, p, 1, 1, p.numel(), false, false, 0).view(p.sizes());
+    };
+    auto bias = [&](const c10::optional<at::Tensor>& b, int64_t n) {
+        if (!bias_present(b)) return at::empty({0}, opt);
+        TORCH_CHECK(b->numel() == n, "adapter_prep: a bias must have ", n, " elements");
+        return cast(param(*b));
+    };
+    const at::Tensor none = at::empty({0}, opt), noneb = at::empty({0}, opt.dtype(at::kByte));
+    std::vector<at::Tensor> out(11, none);
+    out[0] = add(SVTAD_PREP_ROWS, w_d, 1, h, E, true, false, 0);
+    out[1] = bias(b_d, h);
+    out[2] = add(SVTAD_PREP_ROWS, w_u, 1, E, h, false, false, 0);
+    out[3] = bias(b_u, E);
+    out[4] = bias(b_c, h);
+    out[5] = cast(w_c);
+    if (train) {
+        out[6] = cast(w_u);
+        out[7] = add(SVTAD_PREP_COLS, w_d, 1, E, h, false, false, 0);
+        out[8] = add(SVTAD_PREP_COLS, w_u, 1, h, E, true, true, 0);
+    }
+    out[9] = out[10] = noneb;
+    if (pack_conv) {
+        const size_t bf = svtad_fwd_workspace_bytes((int)h, (int)h, dt), bb = svtad_bwd_in_workspace_bytes((int)h, (int)h, dt);
+        if (bf == (size_t)9 * h * h * 2) out[9] = add(SVTAD_PREP_CONV_FWD, w_c, 9, h, h, false, false, 0).view(at::kByte);
+        if (train && bb > bf && bf)
+            out[10] = add(SVTAD_PREP_CONV_BWD, w_c, 9, h, h, false, false, (int64_t)(bb - bf) / 2).view(at::kByte);
+    }
+    check_status(svtad_adapter_prep(jobs.data(), (int)jobs.size(), dt, stream_of(w_d)), "adapter_prep");
+    return out;
+}
+
+// x contiguous; a float32 x (whose cast once gave a fresh buffer) on 16 bytes
+static at::Tensor rows_input(const at::Tensor& x) {
+    at::Tensor c = x.contiguous();
+    return c.scalar_type() == at::kFloat && ((uintptr_t)c.data_ptr() & 15) ? c.clone() : c;
+}
+
+static svtad_rows_args rows_args(int kind, int64_t B, int64_t N, int64_t S, int64_t k, int64_t n) {
+    svtad_rows_args a = {};
+    a.kind = kind;
+    a.batch = B;
+    a.n_tokens = N;
+    a.n_special = S;
+    a.k = (int)k;
+    a.n = (int)n;
+    return a;
+}
+
+static void rows_check(const at::Tensor& a, const at::Tensor& w, int64_t k, int64_t n, const char* what) {
+    check_gpu(a, what);
+    check_gpu(w, "w");
+    TORCH_CHECK(w.scalar_type() == at::kHalf || w.scalar_type() == at::kBFloat16, "adapter_rows: w must be f16 / bf16");
+    TORCH_CHECK(w.numel() == n * k && w.is_contiguous(), "adapter_rows: w does not match ", n, " x ", k);
+    TORCH_CHECK(a.scalar_type() == w.scalar_type() || a.scalar_type() == at::kFloat,
+                "adapter_rows: ", what, " takes the type of w or float32");
+}
+
+// adapter_rows_down(x [B, N, k], wd, bias or empty, n, n_special, copy) ->
+//   (pre_act [B, N, n], act_special [B, S, n], act_patch [B * (N - S), n], x in the compute type if copy, else empty)
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> op_adapter_rows_down(const at::Tensor& x_in, const at::Tensor& w,
+                                                                                const at::Tensor& bias, int64_t n,
+                                                                                int64_t S, bool copy) {
+    TORCH_CHECK(x_in.dim() == 3, "x must be [B, N, C]");
+    const int64_t B = x_in.size(0), N = x_in.size(1), k = x_in.size(2);
+    rows_check(x_in, w, k, n, "x");
+    TORCH_CHECK(S >= 0 && S <= N, "n_special out of range");
+    at::Tensor x = rows_input(x_in);
+    c10::DeviceGuard g(x.device());
+    const auto opt = w.options();
+    at::Tensor pre = at::empty({B, N, n}, opt), sp = at::empty({B, S, n}, opt), pa = at::empty({B * (N - S), n}, opt);
+    const bool f32 = x.scalar_type() == at::kFloat;
+    at::Tensor xc = copy && f32 ? at::empty({B, N, k}, opt) : at::empty({0}, opt);
+    svtad_rows_args a = rows_args(SVTAD_ROWS_GELU, B, N, S, k, n);
+    a.a0 = x.data_ptr();
+    a.w = w.data_ptr();
+    a.bias = opt_ptr(bias, n, w);
+    a.a_copy = xc.numel() ? xc.data_ptr() : nullptr;
+    a.out0 = pre.data_ptr();
+    a.out1 = sp.numel() ? sp.data_ptr() : nullptr;
+    a.out2 = pa.numel() ? pa.data_ptr() : nullptr;
+    a.a_f32 = f32;
+    check_status(svtad_adapter_rows(&a, dtype_code(w), stream_of(x)), "adapter_rows_down");
+    return {pre, sp, pa, xc};
+}
+
+// adapter_rows_split(go [B, N, k], wuT, n, n_special, copy) ->
+//   (special [B, S, n], patch [B * (N - S), n], go in the compute type if copy, else empty)
+std::tuple<at::Tensor, at::Tensor, at::Tensor> op_adapter_rows_split(const at::Tensor& go_in, const at::Tensor& w, int64_t n,
+                                                                     int64_t S, bool copy) {
+    TORCH_CHECK(go_in.dim() == 3, "go must be [B, N, C]");
+    const int64_t B = go_in.size(0), N = go_in.size(1), k = go_in.size(2);
+    rows_check(go_in, w, k, n, "go");
+    TORCH_CHECK(S >= 0 && S <= N, "n_special out of range");
+    at::Tensor go = rows_input(go_in);
+    c10::DeviceGuard g(go.device());
+    const auto opt = w.options();
+    at::Tensor sp = at::empty({B, S, n}, opt), pa = at::empty({B * (N - S), n}, opt);
+    const bool f32 = go.scalar_type() == at::kFloat;
+    at::Tensor gc = copy && f32 ? at::empty({B, N, k}, opt) : at::empty({0}, opt);
+    svtad_rows_args a = rows_args(SVTAD_ROWS_SPLIT, B, N, S, k, n);
+    a.a0 = go.data_ptr();
+    a.w = w.data_ptr();
+    a.a_copy = gc.numel() ? gc.data_ptr() : nullptr;
+    a.out1 = sp.numel() ? sp.data_ptr() : nullptr;
+    a.out2 = pa.numel() ? pa.data_ptr() : nullptr;
+    a.a_f32 = f32;
+    check_status(svtad_adapter_rows(&a, dtype_code(w), stream_of(go)), "adapter_rows_split");
+    return {sp, pa, gc};
+}
+
+// adapter_rows_res(a_special [B, S, k] or None, a, w, bias or empty, gamma or None, residual [B, N, n], out_float32)
+//   -> [B, N, n]: adapter_up with a fragment-ordered weight, or without gamma A W^T + residual
+// a holds the patch rows [B * (N - S), k] beside a_special, else all rows.
+at::Tensor op_adapter_rows_res(const c10::optional<at::Tensor>& sp_in, const at::Tensor& a_in, const at::Tensor& w,
+                               const at::Tensor& bias, const c10::optional<at::Tensor>& gamma_in,
+                               const at::Tensor& res_in, bool out_float32) {
+    TORCH_CHECK(res_in.dim() == 3, "residual must be [B, N, C]");
+    const int64_t B = res_in.size(0), N = res_in.size(1), n = res_in.size(2), k = a_in.size(-1);
+    rows_check(res_in, w, k, n, "residual");
+    check_gpu(a_in, "a");
+    TORCH_CHECK(a_in.scalar_type() == w.scalar_type(), "a and w dtypes differ");
+    const bool split = sp_in.has_value() && sp_in->defined();
+    int64_t S = 0;
+    at::Tensor sp;
+    if (split) {
+        check_gpu(*sp_in, "a_special");
+        TORCH_CHECK(sp_in->dim() == 3 && sp_in->size(0) == B && sp_in->size(2) == k && sp_in->scalar_type() == w.scalar_type(),
+                    "a_special must be [B, S, k]");
+        S = sp_in->size(1);
+        sp = sp_in->contiguous();
+    }
+    TORCH_CHECK(S <= N && a_in.numel() == B * (N - S) * k, "a does not match the residual's rows");
+    at::Tensor a = a_in.contiguous(), res = rows_input(res_in), gm;
+    c10::DeviceGuard g(res.device());
+    at::Tensor out = at::empty({B, N, n}, out_float32 ? res.options().dtype(at::kFloat) : w.options());
+    svtad_rows_args r = rows_args(SVTAD_ROWS_RES, B, N, S, k, n);
+    if (gamma_in.has_value() && gamma_in->defined()) {
+        TORCH_CHECK(gamma_in->is_cuda() && gamma_in->numel() == 1 &&
+                        (gamma_in->scalar_type() == w.scalar_type() || gamma_in->scalar_type() == at::kFloat),
+                    "gamma must be one element on the GPU, of the type of w or float32");
+        gm = gamma_in->contiguous();
+        r.gamma = gm.data_ptr();
+        r.gamma_f32 = gm.scalar_type() == at::kFloat;
+    }
+    r.a0 = split ? (sp.numel() ? sp.data_ptr() : nullptr) : a.data_ptr();
+    r.a1 = split && a.numel() ? a.data_ptr() : nullptr;
+    r.a_patch_split = split;
+    r.w = w.data_ptr();
+    r.bias = opt_ptr(bias, n, w);
+    r.res = res.data_ptr();
+    r.out0 = out.data_ptr();
+    r.res_f32 = res.scalar_type() == at::kFloat;
+    r.out_f32 = out_float32;
+    check_status(svtad_adapter_rows(&r, dtype_code(w), stream_of(res)), "adapter_rows_res");
+    return out;
+}
+
 PYBIND11_MODULE(opentad_sparse_ops, m) {
     m.doc() = "MI355X (gfx950) SparseConv2D: drop-in for the reference opentad_sparse_ops";
     m.def("fwd", &op_fwd, "Forward", py::arg("x"), py::arg("neighbor_indices"), py::arg("weight"),
@@ -1035,6 +1243,18 @@ PYBIND11_MODULE(opentad_sparse_ops, m) {
     m.def("adapter_up", &op_adapter_up, "Adapter up_proj on cat(special, patch) * gamma + residual",
           py::arg("a_special"), py::arg("a_patch"), py::arg("weight"), py::arg("bias"), py::arg("gamma"),
           py::arg("residual"), py::arg("out_float32") = false);
+    m.def("adapter_rows_ok", &op_adapter_rows_ok, "Whether the adapter GEMMs over whole token tiles take these widths",
+          py::arg("embed"), py::arg("hidden"));
+    m.def("adapter_prep", &op_adapter_prep, "Adapter parameters cast and laid out for adapter_rows_*, one launch",
+          py::arg("w_d"), py::arg("b_d"), py::arg("w_c"), py::arg("b_c"), py::arg("w_u"), py::arg("b_u"),
+          py::arg("gamma"), py::arg("bf16"), py::arg("train"), py::arg("pack_conv"));
+    m.def("adapter_rows_down", &op_adapter_rows_down, "adapter_down over whole token tiles (weight of adapter_prep)",
+          py::arg("x"), py::arg("w"), py::arg("bias"), py::arg("n"), py::arg("n_special"), py::arg("copy"));
+    m.def("adapter_rows_split", &op_adapter_rows_split, "go W^T split into special and patch rows",
+          py::arg("go"), py::arg("w"), py::arg("n"), py::arg("n_special"), py::arg("copy"));
+    m.def("adapter_rows_res", &op_adapter_rows_res, "adapter_up over whole token tiles, or A W^T + residual",
+          py::arg("a_special"), py::arg("a"), py::arg("w"), py::arg("bias"), py::arg("gamma"), py::arg("residual"),
+          py::arg("out_float32") = false);
     m.def("heatmap_add_", &op_heatmap_add_, "In place: patch[i] += special[src_rows[i]] * gate (adapter heatmap injection)",
           py::arg("patch"), py::arg("special"), py::arg("src_rows"), py::arg("gate"));
     m.def("linear_wgrad", &op_linear_wgrad, "Linear-layer weight gradient g[rows]^T x (split rows, ordered sum)",

@@ -555,6 +555,61 @@ int svtad_gamma_grad_mixed(const void* w, const void* g, int64_t count, const vo
                            void* gs_scaled, void* workspace, size_t workspace_bytes, int dtype, int g_dtype,
                            int gamma_dtype, void* stream);
 
+/*
+ * The adapter's GEMMs over whole token tiles, for the widths of
+ * svtad_adapter_rows_ok, with the weight in fragment order.
+ *
+ * svtad_adapter_prep runs up to SVTAD_MAX_PREP_JOBS parameter preparations in
+ * one launch. A job reads `src` (f32 with src_f32, else dtype), casts to dtype
+ * and, with gamma, multiplies (rounding to dtype after each), and writes
+ *   SVTAD_PREP_CAST      dst[i] = src[i], off * n * k values (a multiple of 8)
+ *   SVTAD_PREP_ROWS      the fragment order of the [n, k] operand src [n, k]
+ *   SVTAD_PREP_COLS      the same of its transpose, src [k, n]
+ *   SVTAD_PREP_CONV_FWD  svtad_pack_weight's packed_fwd of src [9, k, n]
+ *   SVTAD_PREP_CONV_BWD  svtad_pack_weight's packed_bwd of src [9, n, k]
+ * n and k are multiples of 32 in the layouts. `pair` is 1 for the weight of
+ * SVTAD_ROWS_GELU / _SPLIT and 0 for that of SVTAD_ROWS_RES (column order).
+ */
+enum svtad_prep_kind {
+    SVTAD_PREP_CAST = 0,
+    SVTAD_PREP_ROWS = 1,
+    SVTAD_PREP_COLS = 2,
+    SVTAD_PREP_CONV_FWD = 3,
+    SVTAD_PREP_CONV_BWD = 4
+};
+enum { SVTAD_MAX_PREP_JOBS = 12 };
+typedef struct svtad_prep_job {
+    const void* src;
+    void* dst;
+    const void* gamma; /* one value (f32 with gamma_f32, else dtype), or NULL */
+    int kind, off, n, k;
+    int src_f32, gamma_f32, pair;
+} svtad_prep_job;
+int svtad_adapter_prep(const svtad_prep_job* jobs, int count, int dtype, void* stream);
+
+/*
+ * out = epilogue(A W^T), A [batch * n_tokens, k] (f32 with a_f32, cast to dtype
+ * on the way; a_copy, if not NULL, receives the cast rows), W [n, k] from
+ * SVTAD_PREP_ROWS / _COLS:
+ *   SVTAD_ROWS_GELU   out0 = z = A W^T + bias; GELU(z) with a sample's first
+ *                     n_special rows in out1, the others in out2
+ *   SVTAD_ROWS_SPLIT  A W^T in out1 / out2
+ *   SVTAD_ROWS_RES    out0 = (A W^T + bias) * gamma + res as svtad_adapter_up,
+ *                     or A W^T + res (fp32 sum, one rounding) with gamma NULL;
+ *                     with a_patch_split A is a0 (special) / a1 (patch rows)
+ * Returns SVTAD_ERR_UNSUPPORTED for other widths or type combinations.
+ */
+enum svtad_rows_kind { SVTAD_ROWS_GELU = 0, SVTAD_ROWS_SPLIT = 1, SVTAD_ROWS_RES = 2 };
+typedef struct svtad_rows_args {
+    const void *a0, *a1, *w, *bias, *gamma, *res;
+    void *a_copy, *out0, *out1, *out2;
+    int64_t batch, n_tokens, n_special;
+    int kind, k, n;
+    int a_f32, a_patch_split, gamma_f32, res_f32, out_f32;
+} svtad_rows_args;
+int svtad_adapter_rows_ok(int kind, int k, int n);
+int svtad_adapter_rows(const svtad_rows_args* args, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
