@@ -383,6 +383,49 @@ class SparseConvAdapterFunction(Function):
                 None, None, None, None, g_gate, None, None, None)
 
 
+class KeyTokenAttentionFunction(Function):
+    """``use_attn`` 2 up to the projection: LayerNorm, ``down_attn``, ``qkv``,
+    the per-head norms and the attention of the visual tokens to the first
+    ``nk`` tokens, ``x [B, N, hidden] -> [B, N, hidden / 2]`` (zeros in the key
+    rows) in ``cd``. Queries are projected for all rows and keys and values for
+    the key tokens only (the reference projects all three for every token and
+    leaves the rest unused). The norms, scores, softmax and weighted sum are
+    evaluated in float32 on the Linear outputs; the Linear layers' weight and
+    bias gradients run on the split-row kernels."""
+
+    @staticmethod
+    def forward(ctx, x, nw, nb, dw, db, qw, qb, qnw, qnb, knw, knb, nk, eps, cd):
+        ctx.dtypes = tuple(t.dtype for t in (x, nw, nb, dw, db, qw, qb, qnw, qnb, knw, knb))
+        x, dw, db, qw, qb = (_cast(t, cd) for t in (x, dw, db, qw, qb))
+        a = dw.shape[0]
+        xn, stats = _ops.layer_norm_rows(x, nw, nb, eps[0])
+        xa = nn.functional.linear(xn, dw, db)
+        q = nn.functional.linear(xa, qw[:a], qb[:a])
+        kv = nn.functional.linear(xa[:, :nk].contiguous(), qw[a:], qb[a:])
+        out = _ops.key_attention(q, kv, qnw, qnb, knw, knb, eps[1])
+        ctx.save_for_backward(x, nw, stats, xn, dw, xa, qw, q, kv, qnw, qnb, knw, knb)
+        ctx.meta = (nk, eps)
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        x, nw, stats, xn, dw, xa, qw, q, kv, qnw, qnb, knw, knb = ctx.saved_tensors
+        nk, eps = ctx.meta
+        B, N, a = q.shape
+        dq, dkv, dn = _ops.key_attention_bwd(_cast(g, q.dtype), q, kv, qnw, qnb, knw, knb, eps[1])
+        dq2, dkv2 = dq.view(-1, a), dkv.view(-1, 2 * a)
+        dxa = torch.matmul(dq, qw[:a])
+        dxa[:, :nk] = torch.matmul(dkv2, qw[a:]).view(B, nk, a)  # a key row has no query
+        gqw = torch.cat([_wgrad(dq2, _NO_ROWS(dq2), xa.view(-1, a)),
+                         torch.matmul(dkv2.t(), xa[:, :nk].reshape(-1, a))])
+        gqb = torch.cat([_colsum(dq2), dkv2.sum(0)])
+        dxa2 = dxa.view(-1, a)
+        gdw = _wgrad(dxa2, _NO_ROWS(dxa2), xn.view(-1, xn.shape[-1]))
+        dx, dwb = _ops.layer_norm_rows_bwd(torch.matmul(dxa, dw), x, stats, nw)
+        grads = (dx, dwb[0], dwb[1], gdw, _colsum(dxa2), gqw, gqb, dn[0], dn[1], dn[2], dn[3])
+        return (*(_cast(t, dt) for t, dt in zip(grads, ctx.dtypes)), None, None, None)
+
+
 def _trunc_normal_init(layer, std):
     """mmengine's trunc_normal_init(layer, std=std, bias=0) as the reference calls
     it: weight ~ N(0, std) truncated to [-2, 2], bias 0."""
@@ -544,6 +587,20 @@ class SparseConvAdapter(nn.Module):
         return AdapterUpFunction.apply(empty, x_comb.reshape(B * N, -1), self.up_proj.weight, self.up_proj.bias,
                                        self.gamma, x, self.gamma.dtype == torch.float32 and cd != torch.float32, cd)
 
+    def _key_attention_ok(self, n_tokens):
+        """Whether ``KeyTokenAttentionFunction`` takes this module: its widths
+        and key count, norms with weight and bias and one eps, biased Linear
+        layers, one parameter type for the norms of a kernel."""
+        norms = (self.attn_norm, self.q_norm, self.k_norm)
+        if any(m.weight is None or m.bias is None or m.weight.dtype != m.bias.dtype for m in norms):
+            return False
+        if self.q_norm.eps != self.k_norm.eps or self.q_norm.weight.dtype != self.k_norm.weight.dtype:
+            return False
+        if self.down_attn.bias is None or self.qkv.bias is None or self.hidden_dims not in (128, 256):
+            return False
+        return _ops.key_attention_ok(self.num_heads, self.hidden_dims // 2 // self.num_heads, n_tokens,
+                                     self.n_key_tokens)
+
     def _attention_branch(self, x_comb, S, indices, h, w, total_num_patches, fused, cd=None):
         """The ``use_attn`` branch on ``x_combined`` (vit_sparse_adapter_poguise.py:
         511-650). With ``fused`` the ``shortcut + attn_proj(.) * attn_gamma`` of
@@ -581,6 +638,13 @@ class SparseConvAdapter(nn.Module):
             fr_out = coarse[:, S:]
             pa_out = torch.gather(fr_out.float(), 1, idx).to(fr_out.dtype) if fused else torch.gather(fr_out, 1, idx)
             return shortcut + torch.cat([sp_out, pa_out], dim=1)
+        if fused and self.use_attn == 2 and self._key_attention_ok(N):
+            xa = KeyTokenAttentionFunction.apply(
+                x_comb, self.attn_norm.weight, self.attn_norm.bias, self.down_attn.weight, self.down_attn.bias,
+                self.qkv.weight, self.qkv.bias, self.q_norm.weight, self.q_norm.bias, self.k_norm.weight,
+                self.k_norm.bias, self.n_key_tokens, (self.attn_norm.eps, self.q_norm.eps), cd)
+            return AdapterUpFunction.apply(xa.new_empty(B, 0, xa.shape[-1]), xa.view(B * N, -1), self.attn_proj.weight,
+                                           self.attn_proj.bias, self.attn_gamma, shortcut, False, cd)
         xa = self.down_attn(self.attn_norm(x_comb))
         A = xa.shape[-1]
         hd = A // self.num_heads

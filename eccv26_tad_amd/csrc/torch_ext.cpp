@@ -1167,7 +1167,114 @@ at::Tensor op_adapter_rows_res(const c10::optional<at::Tensor>& sp_in, const at:
     return out;
 }
 
+// ---------------------------------------------------------------------------
+// attention to the key tokens
+// ---------------------------------------------------------------------------
+
+static void attn_params(const at::Tensor& like, std::initializer_list<const at::Tensor*> ps, int64_t n) {
+    const at::ScalarType t = (*ps.begin())->scalar_type();
+    TORCH_CHECK(t == like.scalar_type() || t == at::kFloat, "norm parameters take the row type or float32");
+    for (const at::Tensor* p : ps)
+        TORCH_CHECK(p->is_cuda() && p->numel() == n && p->is_contiguous() && p->scalar_type() == t,
+                    "norm parameters must be contiguous, of ", n, " elements and one type");
+}
+
+// layer_norm_rows(x [..., c], w, b, eps) -> (y, stats [rows, 2] float32)
+std::tuple<at::Tensor, at::Tensor> op_layer_norm_rows(const at::Tensor& x_in, const at::Tensor& w, const at::Tensor& b,
+                                                      double eps) {
+    check_gpu(x_in, "x");
+    at::Tensor x = x_in.contiguous();
+    const int64_t c = x.size(-1), rows = n_rows(x);
+    attn_params(x, {&w, &b}, c);
+    c10::DeviceGuard g(x.device());
+    at::Tensor y = at::empty_like(x), stats = at::empty({rows, 2}, x.options().dtype(at::kFloat));
+    check_status(svtad_layer_norm(x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), stats.data_ptr<float>(), rows,
+                                  (int)c, (float)eps, dtype_code(x), w.scalar_type() == at::kFloat, stream_of(x)),
+                 "layer_norm_rows");
+    return {y, stats};
+}
+
+// layer_norm_rows_bwd(dy, x, stats, w) -> (dx, dwb [2, c] float32)
+std::tuple<at::Tensor, at::Tensor> op_layer_norm_rows_bwd(const at::Tensor& dy_in, const at::Tensor& x_in,
+                                                          const at::Tensor& stats, const at::Tensor& w) {
+    check_gpu(x_in, "x");
+    at::Tensor x = x_in.contiguous(), dy = dy_in.contiguous();
+    const int64_t c = x.size(-1), rows = n_rows(x);
+    TORCH_CHECK(dy.is_cuda() && dy.numel() == x.numel() && dy.scalar_type() == x.scalar_type(), "dy must match x");
+    TORCH_CHECK(stats.numel() == 2 * rows && stats.scalar_type() == at::kFloat && stats.is_contiguous(), "bad stats");
+    attn_params(x, {&w}, c);
+    c10::DeviceGuard g(x.device());
+    const auto f = x.options().dtype(at::kFloat);
+    at::Tensor dx = at::empty_like(x), dwb = at::empty({2, c}, f);
+    const size_t ws = svtad_layer_norm_bwd_workspace_bytes(rows, (int)c);
+    at::Tensor work = at::empty({(int64_t)ws}, f.dtype(at::kByte));
+    check_status(svtad_layer_norm_bwd(dy.data_ptr(), x.data_ptr(), stats.data_ptr<float>(), w.data_ptr(), dx.data_ptr(),
+                                      dwb.data_ptr<float>(), work.data_ptr(), ws, rows, (int)c, dtype_code(x),
+                                      w.scalar_type() == at::kFloat, stream_of(x)),
+                 "layer_norm_rows_bwd");
+    return {dx, dwb};
+}
+
+static void attn_check(const at::Tensor& q, const at::Tensor& kv, const at::Tensor& qw, const at::Tensor& qb,
+                       const at::Tensor& kw, const at::Tensor& kb) {
+    check_gpu(q, "q");
+    check_gpu(kv, "kv");
+    TORCH_CHECK(q.dim() == 3 && kv.dim() == 3 && kv.size(0) == q.size(0) && kv.size(2) == 2 * q.size(2) &&
+                    kv.scalar_type() == q.scalar_type() && q.is_contiguous() && kv.is_contiguous(),
+                "q must be [B, N, a], kv [B, nk, 2 a], contiguous and of one type");
+    attn_params(q, {&qw, &qb, &kw, &kb}, q.size(2) / 4);
+}
+
+bool op_key_attention_ok(int64_t heads, int64_t head_dim, int64_t n, int64_t nk) {
+    return heads < 1024 && head_dim < 1024 && nk < 1024 && svtad_key_attention_ok((int)heads, (int)head_dim, n, (int)nk);
+}
+
+// key_attention(q [B, N, a], kv [B, nk, 2a], qn_w, qn_b, kn_w, kn_b, eps) -> [B, N, a]
+at::Tensor op_key_attention(const at::Tensor& q, const at::Tensor& kv, const at::Tensor& qw, const at::Tensor& qb,
+                            const at::Tensor& kw, const at::Tensor& kb, double eps) {
+    attn_check(q, kv, qw, qb, kw, kb);
+    c10::DeviceGuard g(q.device());
+    at::Tensor out = at::empty_like(q);
+    check_status(svtad_key_attention(q.data_ptr(), kv.data_ptr(), qw.data_ptr(), qb.data_ptr(), kw.data_ptr(), kb.data_ptr(),
+                                     out.data_ptr(), q.size(0), q.size(1), (int)kv.size(1), (int)q.size(2) / 4, (float)eps,
+                                     dtype_code(q), qw.scalar_type() == at::kFloat, stream_of(q)),
+                 "key_attention");
+    return out;
+}
+
+// key_attention_bwd(dout, q, kv, qn_w, qn_b, kn_w, kn_b, eps) -> (dq, dkv, dnorm [4, a / 4] float32)
+std::tuple<at::Tensor, at::Tensor, at::Tensor> op_key_attention_bwd(const at::Tensor& dout_in, const at::Tensor& q,
+                                                                    const at::Tensor& kv, const at::Tensor& qw,
+                                                                    const at::Tensor& qb, const at::Tensor& kw,
+                                                                    const at::Tensor& kb, double eps) {
+    attn_check(q, kv, qw, qb, kw, kb);
+    check_gpu(dout_in, "dout");
+    TORCH_CHECK(dout_in.sizes() == q.sizes() && dout_in.scalar_type() == q.scalar_type(), "dout must match q");
+    at::Tensor dout = dout_in.contiguous();
+    c10::DeviceGuard g(q.device());
+    const int64_t B = q.size(0), N = q.size(1), nk = kv.size(1), hd = q.size(2) / 4;
+    at::Tensor dq = at::empty_like(q), dkv = at::empty_like(kv), dn = at::empty({4, hd}, q.options().dtype(at::kFloat));
+    const size_t ws = svtad_key_attention_bwd_workspace_bytes(B, N, (int)nk, (int)hd);
+    at::Tensor work = at::empty({(int64_t)ws}, q.options().dtype(at::kByte));
+    check_status(svtad_key_attention_bwd(dout.data_ptr(), q.data_ptr(), kv.data_ptr(), qw.data_ptr(), qb.data_ptr(),
+                                         kw.data_ptr(), kb.data_ptr(), dq.data_ptr(), dkv.data_ptr(), dn.data_ptr<float>(),
+                                         work.data_ptr(), ws, B, N, (int)nk, (int)hd, (float)eps, dtype_code(q),
+                                         qw.scalar_type() == at::kFloat, stream_of(q)),
+                 "key_attention_bwd");
+    return {dq, dkv, dn};
+}
+
 PYBIND11_MODULE(opentad_sparse_ops, m) {
+    m.def("layer_norm_rows", &op_layer_norm_rows, "LayerNorm of rows of 128 or 256 channels (y, stats)", py::arg("x"),
+          py::arg("w"), py::arg("b"), py::arg("eps"));
+    m.def("layer_norm_rows_bwd", &op_layer_norm_rows_bwd, "LayerNorm backward (dx, [dw, db])", py::arg("dy"), py::arg("x"),
+          py::arg("stats"), py::arg("w"));
+    m.def("key_attention_ok", &op_key_attention_ok, "Whether key_attention takes these sizes", py::arg("heads"),
+          py::arg("head_dim"), py::arg("n"), py::arg("nk"));
+    m.def("key_attention", &op_key_attention, "Normalised attention of the visual tokens to the key tokens", py::arg("q"),
+          py::arg("kv"), py::arg("qn_w"), py::arg("qn_b"), py::arg("kn_w"), py::arg("kn_b"), py::arg("eps"));
+    m.def("key_attention_bwd", &op_key_attention_bwd, "Its gradients (dq, dkv, norm parameters)", py::arg("dout"),
+          py::arg("q"), py::arg("kv"), py::arg("qn_w"), py::arg("qn_b"), py::arg("kn_w"), py::arg("kn_b"), py::arg("eps"));
     m.doc() = "MI355X (gfx950) SparseConv2D: drop-in for the reference opentad_sparse_ops";
     m.def("fwd", &op_fwd, "Forward", py::arg("x"), py::arg("neighbor_indices"), py::arg("weight"),
           py::arg("C_out"), py::arg("tokens_per_batch"));

@@ -610,6 +610,37 @@ typedef struct svtad_rows_args {
 int svtad_adapter_rows_ok(int kind, int k, int n);
 int svtad_adapter_rows(const svtad_rows_args* args, int dtype, void* stream);
 
+/*
+ * The adapter's attention of visual tokens to a sample's first nk (key) tokens
+ * (vit_sparse_adapter_poguise.py:598-620), f16 / bf16, four heads of 16 or 32
+ * channels (a = 4 head_dim), 1 to 16 keys; parameters in dtype or, with
+ * param_f32, f32.
+ *
+ * svtad_layer_norm: y = LayerNorm(x) over rows of 128 or 256 channels, and each
+ * row's mean and 1 / std in stats [rows, 2]; svtad_layer_norm_bwd: dx, and the
+ * gradients of w and b in dwb [2, c] (f32).
+ * svtad_key_attention: out [batch, n, a] = softmax(LN(q) LN(k)^T / sqrt(hd)) v per
+ * head for the tokens after the first nk (whose rows are 0), q [batch, n, a],
+ * kv [batch, nk, 2 a] (keys, then values); svtad_key_attention_bwd: dq (0 in the
+ * key rows), dkv, and the gradients of qn_w, qn_b, kn_w, kn_b in dnorm [4, hd]
+ * (f32). The sums over rows are ordered.
+ */
+int svtad_layer_norm(const void* x, const void* w, const void* b, void* y, float* stats, int64_t rows, int c,
+                     float eps, int dtype, int param_f32, void* stream);
+size_t svtad_layer_norm_bwd_workspace_bytes(int64_t rows, int c);
+int svtad_layer_norm_bwd(const void* dy, const void* x, const float* stats, const void* w, void* dx, float* dwb,
+                         void* workspace, size_t workspace_bytes, int64_t rows, int c, int dtype, int param_f32,
+                         void* stream);
+int svtad_key_attention_ok(int heads, int head_dim, int64_t n, int nk);
+int svtad_key_attention(const void* q, const void* kv, const void* qn_w, const void* qn_b, const void* kn_w,
+                        const void* kn_b, void* out, int64_t batch, int64_t n, int nk, int head_dim, float eps,
+                        int dtype, int param_f32, void* stream);
+size_t svtad_key_attention_bwd_workspace_bytes(int64_t batch, int64_t n, int nk, int head_dim);
+int svtad_key_attention_bwd(const void* dout, const void* q, const void* kv, const void* qn_w, const void* qn_b,
+                            const void* kn_w, const void* kn_b, void* dq, void* dkv, float* dnorm, void* workspace,
+                            size_t workspace_bytes, int64_t batch, int64_t n, int nk, int head_dim, float eps, int dtype,
+                            int param_f32, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
