@@ -148,6 +148,23 @@ def _up_wgrad(go, B, N, S, a_sp, a_pa):
 
 
 _PATCH_ROWS = {}
+_TOKEN_ROWS = {}
+
+
+def _token_rows(B, N, S, device):
+    """Row of ``go.reshape(B * N, -1)`` for the special tokens of every sample,
+    then for the patch tokens in the order of the SparseConv2D rows, cached
+    per shape and device (bounded)."""
+    key = (B, N, S, device)
+    rows = _TOKEN_ROWS.get(key)
+    if rows is None:
+        r = torch.arange(B * S, device=device, dtype=torch.int32)
+        special = (r // max(S, 1)) * N + r % max(S, 1)
+        rows = torch.cat([special, _patch_rows(B, N, S, device)])
+        if len(_TOKEN_ROWS) >= 64:
+            _TOKEN_ROWS.clear()
+        _TOKEN_ROWS[key] = rows
+    return rows
 
 
 def _patch_rows(B, N, S, device):
@@ -256,7 +273,7 @@ class SparseConvAdapterFunction(Function):
 
     @staticmethod
     def forward(ctx, x, w_d, b_d, w_c, b_c, w_u, b_u, gamma, nbr, n_special, tpb, hm_rows=None, hm_gate=None,
-                packed=None, cd=None, keep_packed=None):
+                packed=None, cd=None):
         S = int(n_special)
         ctx.symmetric = is_symmetric_table(nbr)
         cd = x.dtype if cd is None else cd
@@ -273,46 +290,25 @@ class SparseConvAdapterFunction(Function):
         # z * gamma + x: float32 when gamma is a float32 parameter (the
         # reference's dtype promotion under autocast), else in cd
         out32 = gamma.dtype == torch.float32 and cd != gamma.dtype
-        rows = w_c.shape[2] == c_in and _ops.adapter_rows_ok(x.shape[-1], c_in)
-        w_dt = w_ut = None
-        if rows:
-            pack = packed is None or (need_bwd and packed[1] is None)
-            wd, b_d, wu, b_u_c, b_c_c, w_c, w_u_c, w_dt, w_ut, pf, pb = _ops.adapter_prep(
-                w_d, b_d, w_c, b_c, w_u, b_u, gamma, cd == torch.bfloat16, need_bwd, pack)
-            if not pack:
-                pf, pb = packed
-            elif keep_packed is not None:
-                keep_packed(pf, pb if need_bwd else None)
-            w_u, b_c = w_u_c, (None if b_c is None else b_c_c)
-            pre, sp, pa, xc = _ops.adapter_rows_down(x, wd, b_d, c_in, S, need_bwd)
-            if x.dtype == cd:
-                xc = x
-        else:
-            xc = _cast(x, cd)
-            w_d, b_d, w_c, b_c, w_u, b_u = (_cast(t, cd) for t in (w_d, b_d, w_c, b_c, w_u, b_u))
-            pre, sp, pa = _ops.adapter_down(xc, w_d, b_d, S)
-            if packed is None or (need_bwd and packed[1] is None):
-                packed = _ops.pack_weight(w_c, True, need_bwd)
-            pf, pb = packed
+        xc = _cast(x, cd)
+        w_d, b_d, w_c, b_c, w_u, b_u = (_cast(t, cd) for t in (w_d, b_d, w_c, b_c, w_u, b_u))
+        pre, sp, pa = _ops.adapter_down(xc, w_d, b_d, S)
         if hm_rows is not None:
             # heatmap injection on the SparseConv2D input (in place)
             _ops.heatmap_add_(pa, sp, hm_rows, hm_gate)
+        if packed is None or (need_bwd and packed[1] is None):
+            packed = _ops.pack_weight(w_c, True, need_bwd)
+        pf, pb = packed
         processed = _ops.fwd_packed(pa, nbr, w_c, pf, b_c, tpb, mode)
-        if rows:
-            out = _ops.adapter_rows_res(sp, processed, wu, b_u_c, gamma, x, out32)
-            b_u = None if b_u is None else b_u_c
-        else:
-            out = _ops.adapter_up(sp, processed, w_u, b_u, gamma, x, out32)
+        out = _ops.adapter_up(sp, processed, w_u, b_u, gamma, x, out32)
         if need_bwd:
-            ctx.save_for_backward(xc, None if rows else w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma,
-                                  hm_rows, hm_gate, w_dt, w_ut)
+            ctx.save_for_backward(xc, w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma, hm_rows, hm_gate)
         ctx.flags = (S, int(tpb), has_bd)
         return out
 
     @staticmethod
     def backward(ctx, go):
-        (x, w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma, hm_rows, hm_gate, w_dt,
-         w_ut) = ctx.saved_tensors
+        x, w_d, pre, sp, pa, nbr, w_c, b_c, pb, processed, w_u, b_u, gamma, hm_rows, hm_gate = ctx.saved_tensors
         S, tpb, has_bd = ctx.flags
         x_dt, wd_dt, bd_dt, wc_dt, bc_dt, wu_dt, bu_dt, _, _ = ctx.dtypes
         need = ctx.needs_input_grad
@@ -321,13 +317,7 @@ class SparseConvAdapterFunction(Function):
         cd = pre.dtype
         go = go.contiguous()
         go_res = go  # the residual's gradient (float32 under autocast)
-        if w_ut is not None:
-            # (go * gamma) W_u with go cast on the way (its cast is kept for
-            # the weight gradients) and the two kinds of rows stored apart
-            g_sp, g_pa, gc = _ops.adapter_rows_split(go, w_ut, k, S, True)
-            go = gc if go.dtype != cd else go
-        else:
-            go = _cast(go, cd)
+        go = _cast(go, cd)
         go2 = go.reshape(-1, n)
         # up projection: G = go^T cat(sp, processed) without the cat, in fp32
         G = _up_wgrad(go, B, N, S, sp, processed)
@@ -337,10 +327,9 @@ class SparseConvAdapterFunction(Function):
         g_gamma = g_gamma.view(gamma.shape) if need[7] else None
         gw_u = gw_u if need[5] else None
         gb_u = gb_u if b_u is not None and need[6] else None
-        if w_ut is None:
-            dc = torch.matmul(go, w_u_g)  # [B, N, k]: (go * gamma) W_u
-            g_sp = dc[:, :S]
-            g_pa = dc[:, S:].reshape(-1, k)
+        dc = torch.matmul(go, w_u_g)  # [B, N, k]: (go * gamma) W_u
+        g_sp = dc[:, :S]
+        g_pa = dc[:, S:].reshape(-1, k)
         # SparseConv2D
         need_bc = b_c is not None and need[4]
         gi_pa, gw_c, gb_c = _ops.bwd_packed(g_pa, pa, nbr, w_c, pb, w_c.shape[1], tpb, need_bc,
@@ -366,11 +355,7 @@ class SparseConvAdapterFunction(Function):
         x2 = x.reshape(-1, x.shape[-1])
         gx = None
         if need[0]:
-            if w_dt is not None:
-                # du W_d plus the residual's gradient, one rounding
-                gx = _ops.adapter_rows_res(None, du, w_dt, du.new_empty(0), None, go_res if x_dt != cd else go,
-                                           x_dt != cd)
-            elif x_dt == cd:
+            if x_dt == cd:
                 gx = torch.addmm(go2, du2, w_d).view(x.shape)
             else:
                 # float32 x under autocast: the down projection's gradient
@@ -380,7 +365,62 @@ class SparseConvAdapterFunction(Function):
         gb_d = _colsum(du2).to(bd_dt) if has_bd and need[2] else None
         return (gx, gw_d, gb_d, gw_c.to(wc_dt) if need[3] else None,
                 gb_c.to(bc_dt) if need_bc else None, _cast(gw_u, wu_dt), _cast(gb_u, bu_dt), g_gamma,
-                None, None, None, None, g_gate, None, None, None)
+                None, None, None, None, g_gate, None, None)
+
+
+_ATTN_PARAMS = 13  # tensors of SparseConvAdapter._attention_parameters
+
+
+class AdapterRowsFunction(Function):
+    """The adapter for the widths of ``adapter_rows_ok`` as one autograd node
+    and one native call each way, without attention or with the key-token
+    attention (``use_attn`` 2): the computation of
+    ``SparseConvAdapterFunction`` (and ``KeyTokenAttentionFunction``) with the
+    four GEMMs over whole token tiles. The casts of x and of the output
+    gradient happen as their rows are read, the parameters are cast and laid
+    out in one launch (which also packs the SparseConv2D weight when
+    ``packed`` is None and hands the layouts to ``keep_packed``), the gradient
+    of the up projection's operand leaves its GEMM as special and patch rows,
+    and the input gradient's residual is added in the same kernel.
+
+    ``attn`` are the attention's 13 parameters, or nothing; ``meta`` is
+    ``(n_special, tokens_per_batch, cd, nk, eps of the row norm, eps of the
+    head norms)``."""
+
+    @staticmethod
+    def forward(ctx, x, w_d, b_d, w_c, b_c, w_u, b_u, gamma, nbr, hm_rows, hm_gate, packed, keep_packed, meta, *attn):
+        S, tpb, cd, nk, eps0, eps1 = meta
+        c_in = w_c.shape[1]
+        mode = BIAS_NONE if b_c is None else (BIAS_FP32 if c_in >= IMPLICIT_GEMM_MIN_CIN else BIAS_AFTER)
+        train = any(ctx.needs_input_grad)
+        pack = packed is None or (train and packed[1] is None)
+        out, pf, pb, *saved = _ops.adapter_forward(
+            x, w_d, b_d, w_c, b_c, w_u, b_u, gamma, nbr, S, tpb, mode, hm_rows, hm_gate, None if pack else packed[0],
+            None if pack else packed[1], cd == torch.bfloat16, train, list(attn), nk, eps0, eps1)
+        if pack and keep_packed is not None:
+            keep_packed(pf, pb if train else None)
+        if train:
+            ctx.save_for_backward(gamma, nbr, hm_rows, hm_gate, *saved, *attn)
+            ctx.meta = (meta, is_symmetric_table(nbr), b_d is not None, b_c is not None, b_u is not None, x.dtype,
+                        [t is not None and t.dtype == torch.float32 for t in (w_d, b_d, w_c, b_c, w_u, b_u)])
+        return out
+
+    @staticmethod
+    def backward(ctx, go):
+        (S, tpb, cd, nk, _, eps1), symmetric, has_bd, has_bc, has_bu, x_dt, f32 = ctx.meta
+        gamma, nbr, hm_rows, hm_gate, *saved = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        attn = []
+        if len(need) > 14:
+            saved, attn = saved[:-_ATTN_PARAMS], saved[-_ATTN_PARAMS:]
+        B, N, _ = go.shape
+        rows = gamma.new_empty(0, dtype=torch.int32) if attn else _token_rows(B, N, S, go.device)
+        gx, gw_d, gb_d, gw_c, gb_c, gw_u, gb_u, g_gamma, g_gate, *ga = _ops.adapter_backward(
+            go, saved, gamma, nbr, hm_rows, hm_gate, rows, attn, S, tpb, nk, eps1, symmetric, has_bd, has_bc, need[0],
+            need[1], f32, x_dt == torch.float32)
+        g = lambda want, t: t if want else None  # noqa: E731
+        return (g(need[0], gx), g(need[1], gw_d), g(has_bd, gb_d), gw_c, g(has_bc, gb_c), gw_u, g(has_bu, gb_u), g_gamma,
+                None, None, g(hm_rows is not None, g_gate), None, None, None, *ga)
 
 
 class KeyTokenAttentionFunction(Function):
@@ -556,7 +596,8 @@ class SparseConvAdapter(nn.Module):
                 nbr = nbr.to(torch.int32)
             nbr = _keep_symmetric(neighbor_indices, nbr)
         conv = self.sparse_conv
-        if not self.use_attn:
+        key_attn = self.use_attn == 2 and self._key_attention_ok(N)
+        if not self.use_attn or key_attn:
             hm_rows = hm_gate = None
             if self._uses_heatmap():
                 H_hm, W_hm = self.heatmap_grid_size
@@ -567,18 +608,26 @@ class SparseConvAdapter(nn.Module):
                 hm_rows = (base + cells).reshape(-1).to(torch.int32)
                 hm_gate = self.heatmap_gate
             cache = conv.packed_weight_cache
-            packed = keep_packed = None
-            if cache is not None:
-                if _ops.adapter_rows_ok(self.embed_dims, self.hidden_dims):
+            packed = None
+            if _ops.adapter_rows_ok(self.embed_dims, self.hidden_dims):
+                keep_packed = None
+                if cache is not None:
                     # packed with the other parameters' preparation when not current
                     packed = cache.peek(conv.weight, cd, torch.is_grad_enabled())
                     keep_packed = functools.partial(cache.put, conv.weight, cd)
-                else:
-                    packed = cache.get(conv.weight, _cast(conv.weight, cd), torch.is_grad_enabled())
+                attn, nk, eps = (), 0, (0.0, 0.0)
+                if key_attn:
+                    attn, nk = self._attention_parameters(), self.n_key_tokens
+                    eps = (self.attn_norm.eps, self.q_norm.eps)
+                return AdapterRowsFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight, conv.bias,
+                                                 self.up_proj.weight, self.up_proj.bias, self.gamma, nbr, hm_rows,
+                                                 hm_gate, packed, keep_packed, (S, tokens_per_batch, cd, nk, *eps), *attn)
+        if not self.use_attn:
+            if cache is not None:
+                packed = cache.get(conv.weight, _cast(conv.weight, cd), torch.is_grad_enabled())
             return SparseConvAdapterFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight,
                                                    conv.bias, self.up_proj.weight, self.up_proj.bias, self.gamma,
-                                                   nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd,
-                                                   keep_packed)
+                                                   nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd)
         sp, pa = AdapterDownFunction.apply(x, self.down_proj.weight, self.down_proj.bias, S, cd)
         processed = conv(pa, nbr, tokens_per_batch=tokens_per_batch)
         x_comb = torch.cat([sp, processed.view(B, N - S, -1)], dim=1)
@@ -586,6 +635,12 @@ class SparseConvAdapter(nn.Module):
         empty = x_comb.new_empty(B, 0, x_comb.shape[-1])
         return AdapterUpFunction.apply(empty, x_comb.reshape(B * N, -1), self.up_proj.weight, self.up_proj.bias,
                                        self.gamma, x, self.gamma.dtype == torch.float32 and cd != torch.float32, cd)
+
+    def _attention_parameters(self):
+        """The key-token attention's parameters in the order of the native calls."""
+        return (self.attn_norm.weight, self.attn_norm.bias, self.down_attn.weight, self.down_attn.bias, self.qkv.weight,
+                self.qkv.bias, self.q_norm.weight, self.q_norm.bias, self.k_norm.weight, self.k_norm.bias,
+                self.attn_proj.weight, self.attn_proj.bias, self.attn_gamma)
 
     def _key_attention_ok(self, n_tokens):
         """Whether ``KeyTokenAttentionFunction`` takes this module: its widths
@@ -596,7 +651,7 @@ class SparseConvAdapter(nn.Module):
             return False
         if self.q_norm.eps != self.k_norm.eps or self.q_norm.weight.dtype != self.k_norm.weight.dtype:
             return False
-        if self.down_attn.bias is None or self.qkv.bias is None or self.hidden_dims not in (128, 256):
+        if self.down_attn.bias is None or self.qkv.bias is None or self.attn_proj.bias is None or self.hidden_dims not in (128, 256):
             return False
         return _ops.key_attention_ok(self.num_heads, self.hidden_dims // 2 // self.num_heads, n_tokens,
                                      self.n_key_tokens)

@@ -57,10 +57,22 @@ struct RowVec {
     T e[VPL];
 };
 
+// Row m of [batch, n_tokens, C] kept as special rows [batch, n_special, C] and
+// patch rows: its address in one of them (n_special 0: in `patch`).
+template <typename T>
+__device__ __forceinline__ T* split_row(T* special, T* patch, int64_t m, uint32_t n_tokens, uint32_t n_special, int c) {
+    if (n_special == 0) return patch + m * c;
+    const uint32_t b = (uint32_t)m / n_tokens, r = (uint32_t)m - b * n_tokens;
+    return r < n_special ? special + ((int64_t)b * n_special + r) * c
+                         : patch + ((int64_t)b * (n_tokens - n_special) + (r - n_special)) * c;
+}
+
 template <typename T, int VPL>
-__global__ __launch_bounds__(256) void k_ln_fwd(const T* __restrict__ x, const void* __restrict__ w,
-                                                const void* __restrict__ b, T* __restrict__ y,
-                                                float* __restrict__ stats, int64_t rows, float eps, bool p32) {
+__global__ __launch_bounds__(256) void k_ln_fwd(const T* __restrict__ special, const T* __restrict__ x,
+                                                T* __restrict__ copy, uint32_t n_tokens, uint32_t n_special,
+                                                const void* __restrict__ w, const void* __restrict__ b,
+                                                T* __restrict__ y, float* __restrict__ stats, int64_t rows, float eps,
+                                                bool p32) {
     constexpr int C = 64 * VPL;
     typedef RowVec<T, VPL> V;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -72,7 +84,8 @@ __global__ __launch_bounds__(256) void k_ln_fwd(const T* __restrict__ x, const v
     }
     const int64_t r1 = min<int64_t>(rows, (int64_t)(blockIdx.x + 1) * kLnRows);
     for (int64_t r = (int64_t)blockIdx.x * kLnRows + wave; r < r1; r += 4) {
-        const V v = *(const V*)(x + r * C + lane * VPL);
+        const V v = *(const V*)(split_row(special, x, r, n_tokens, n_special, C) + lane * VPL);
+        if (copy) *(V*)(copy + r * C + lane * VPL) = v;
         float f[VPL], s = 0.f;
 #pragma unroll
         for (int j = 0; j < VPL; ++j) {
@@ -95,11 +108,14 @@ __global__ __launch_bounds__(256) void k_ln_fwd(const T* __restrict__ x, const v
     }
 }
 
-// dx, and part[workgroup][0 / 1][C]: the workgroup's sums of dy xhat and dy
+// dx (+ add, the gradient of x by another way; stored by token kind), and
+// part[workgroup][0 / 1][C]: the workgroup's sums of dy xhat and dy
 template <typename T, int VPL>
 __global__ __launch_bounds__(256) void k_ln_bwd(const T* __restrict__ dy, const T* __restrict__ x,
-                                                const float* __restrict__ stats, const void* __restrict__ w,
-                                                T* __restrict__ dx, float* __restrict__ part, int64_t rows, bool p32) {
+                                                const T* __restrict__ add, const float* __restrict__ stats,
+                                                const void* __restrict__ w, T* __restrict__ dx_special,
+                                                T* __restrict__ dx, uint32_t n_tokens, uint32_t n_special,
+                                                float* __restrict__ part, int64_t rows, bool p32) {
     constexpr int C = 64 * VPL;
     typedef RowVec<T, VPL> V;
     __shared__ float red[4][2][C];
@@ -127,10 +143,14 @@ __global__ __launch_bounds__(256) void k_ln_bwd(const T* __restrict__ dy, const 
         }
         s1 = lane_sum<64>(s1) * (1.f / C);
         s2 = lane_sum<64>(s2) * (1.f / C);
-        V o;
+        V o, ad;
+        if (add) ad = *(const V*)(add + r * C + lane * VPL);
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) o.e[j] = (T)(rstd * (g[j] - s1 - xh[j] * s2));
-        *(V*)(dx + r * C + lane * VPL) = o;
+        for (int j = 0; j < VPL; ++j) {
+            const float t = rstd * (g[j] - s1 - xh[j] * s2);
+            o.e[j] = (T)(add ? t + (float)ad.e[j] : t);
+        }
+        *(V*)(split_row(dx_special, dx, r, n_tokens, n_special, C) + lane * VPL) = o;
     }
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
@@ -350,16 +370,25 @@ static bool half_type(int d) { return d == SVTAD_F16 || d == SVTAD_BF16; }
 
 using namespace svtad;
 
-extern "C" int svtad_layer_norm(const void* x, const void* w, const void* b, void* y, float* stats, int64_t rows, int c,
-                                float eps, int dtype, int param_f32, void* stream) {
+// the split of svtad_layer_norm / _bwd: whole samples, 32-bit row numbers
+static bool split_ok(int64_t rows, int64_t n_tokens, int64_t n_special) {
+    return n_special == 0 || (n_special > 0 && n_special <= n_tokens && n_tokens < (int64_t)INT32_MAX &&
+                              rows < (int64_t)INT32_MAX && rows % n_tokens == 0);
+}
+
+extern "C" int svtad_layer_norm(const void* special, const void* x, void* copy, int64_t n_tokens, int64_t n_special,
+                                const void* w, const void* b, void* y, float* stats, int64_t rows, int c, float eps,
+                                int dtype, int param_f32, void* stream) {
     if (!half_type(dtype) || (c != 128 && c != 256))
         return set_error(SVTAD_ERR_UNSUPPORTED, "layer_norm: f16 / bf16 rows of 128 or 256 channels");
-    if (rows < 0 || (rows > 0 && (!x || !w || !b || !y || !stats)) || !al16a(x) || !al16a(y))
+    if (rows < 0 || !split_ok(rows, n_tokens, n_special) ||
+        (rows > 0 && ((!x && (n_special == 0 || n_tokens > n_special)) || (n_special > 0 && !special) || !w || !b || !y || !stats)) ||
+        !al16a(x) || !al16a(special) || !al16a(copy) || !al16a(y))
         return set_error(SVTAD_ERR_INVALID, "layer_norm: bad arguments");
     if (rows == 0) return SVTAD_OK;
     const dim3 g((unsigned)cdiv(rows, kLnRows));
 #define SVTAD_LN(T, V) \
-    hipLaunchKernelGGL((k_ln_fwd<T, V>), g, dim3(256), 0, (hipStream_t)stream, (const T*)x, w, b, (T*)y, stats, rows, eps, param_f32 != 0)
+    hipLaunchKernelGGL((k_ln_fwd<T, V>), g, dim3(256), 0, (hipStream_t)stream, (const T*)special, (const T*)x, (T*)copy, (uint32_t)n_tokens, (uint32_t)n_special, w, b, (T*)y, stats, rows, eps, param_f32 != 0)
     if (dtype == SVTAD_F16) {
         if (c == 128) SVTAD_LN(f16, 2);
         else SVTAD_LN(f16, 4);
@@ -375,19 +404,22 @@ extern "C" size_t svtad_layer_norm_bwd_workspace_bytes(int64_t rows, int c) {
     return rows <= 0 || c <= 0 ? 0 : (size_t)cdiv(rows, kLnRows) * 2 * c * 4;
 }
 
-extern "C" int svtad_layer_norm_bwd(const void* dy, const void* x, const float* stats, const void* w, void* dx, float* dwb,
+extern "C" int svtad_layer_norm_bwd(const void* dy, const void* x, const void* add, const float* stats, const void* w,
+                                    void* dx_special, void* dx, int64_t n_tokens, int64_t n_special, float* dwb,
                                     void* workspace, size_t workspace_bytes, int64_t rows, int c, int dtype,
                                     int param_f32, void* stream) {
     if (!half_type(dtype) || (c != 128 && c != 256))
         return set_error(SVTAD_ERR_UNSUPPORTED, "layer_norm_bwd: f16 / bf16 rows of 128 or 256 channels");
-    if (rows < 1 || !dy || !x || !stats || !w || !dx || !dwb || !workspace || !al16a(dy) || !al16a(x) || !al16a(dx))
+    if (rows < 1 || !split_ok(rows, n_tokens, n_special) || !dy || !x || !stats || !w || (!dx && (n_special == 0 || n_tokens > n_special)) ||
+        (n_special > 0 && !dx_special) || !dwb || !workspace || !al16a(dy) || !al16a(x) || !al16a(add) || !al16a(dx_special) ||
+        !al16a(dx))
         return set_error(SVTAD_ERR_INVALID, "layer_norm_bwd: bad arguments");
     if (workspace_bytes < svtad_layer_norm_bwd_workspace_bytes(rows, c))
         return set_error(SVTAD_ERR_WORKSPACE, "layer_norm_bwd: workspace too small");
     const int64_t wgs = cdiv(rows, kLnRows);
 #define SVTAD_LN(T, V)                                                                                             \
     hipLaunchKernelGGL((k_ln_bwd<T, V>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, (const T*)dy, (const T*)x, \
-                       stats, w, (T*)dx, (float*)workspace, rows, param_f32 != 0)
+                       (const T*)add, stats, w, (T*)dx_special, (T*)dx, (uint32_t)n_tokens, (uint32_t)n_special, (float*)workspace, rows, param_f32 != 0)
     if (dtype == SVTAD_F16) {
         if (c == 128) SVTAD_LN(f16, 2);
         else SVTAD_LN(f16, 4);

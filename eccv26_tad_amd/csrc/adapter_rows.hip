@@ -49,6 +49,15 @@ __global__ __launch_bounds__(256) void k_adapter_prep(PrepJobs jobs) {
     const int64_t total = (int64_t)j.off * j.n * j.k;
     if (j.kind == SVTAD_PREP_CONV_BWD && slot == 0) *(uint32_t*)((T*)j.dst + total) = 0u;  // orphan flag after the layout
     if (slot * 8 >= total) return;
+    if (j.kind == SVTAD_PREP_WIDEN) {
+        const u32x4 v = *(const u32x4*)((const T*)j.src + slot * 8);
+        f32x4 o[2];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e >> 2][e & 3] = (float)__builtin_bit_cast(T, (u16)((e & 1) ? v[e >> 1] >> 16 : v[e >> 1] & 0xffffu));
+        *(f32x4*)((float*)j.dst + slot * 8) = o[0];
+        *(f32x4*)((float*)j.dst + slot * 8 + 4) = o[1];
+        return;
+    }
     const float gm = !j.gamma ? 1.f : j.gamma_f32 ? *(const float*)j.gamma : (float)*(const T*)j.gamma;
     auto at = [&](int64_t i) -> T {
         const T v = j.src_f32 ? (T)f32_rounded(((const float*)j.src)[i]) : ((const T*)j.src)[i];
@@ -415,16 +424,20 @@ static bool rows_gemm(const RowsArgs& p, int epi, int k, bool af32, bool asplit,
         rows_out<T, KK, SP, G, R, O>(p, s);                                                   \
         return true;                                                                          \
     }
-#define SVTAD_OK(KK)                        \
-    SVTAD_O(KK, true, false, false, false)  \
-    SVTAD_O(KK, true, true, true, true)     \
-    SVTAD_O(KK, true, true, false, true)    \
-    SVTAD_O(KK, true, true, true, false)    \
-    SVTAD_O(KK, true, true, false, false)   \
-    SVTAD_O(KK, false, false, false, false) \
-    SVTAD_O(KK, false, false, true, true)
-    SVTAD_OK(128)
-    SVTAD_OK(256)
+#define SVTAD_OK(KK, SP)              \
+    SVTAD_O(KK, SP, false, false, false) \
+    SVTAD_O(KK, SP, true, true, true)    \
+    SVTAD_O(KK, SP, true, false, true)   \
+    SVTAD_O(KK, SP, true, true, false)   \
+    SVTAD_O(KK, SP, true, false, false)
+    SVTAD_OK(128, true)
+    SVTAD_OK(256, true)
+    SVTAD_OK(128, false)
+    SVTAD_OK(256, false)
+    SVTAD_O(128, false, false, true, true)  // no gamma: the input gradient under autocast
+    SVTAD_O(256, false, false, true, true)
+    SVTAD_O(64, false, false, false, false)
+    SVTAD_O(64, false, true, false, false)
 #undef SVTAD_OK
 #undef SVTAD_O
     return false;
@@ -446,10 +459,12 @@ extern "C" int svtad_adapter_prep(const svtad_prep_job* jobs, int count, int dty
     int64_t blocks = 0;
     for (int q = 0; q < count; ++q) {
         const svtad_prep_job& j = jobs[q];
-        if (!j.src || !j.dst || !al16r(j.dst) || j.kind < SVTAD_PREP_CAST || j.kind > SVTAD_PREP_CONV_BWD || j.off < 1 ||
+        if (!j.src || !j.dst || !al16r(j.dst) || j.kind < SVTAD_PREP_CAST || j.kind > SVTAD_PREP_WIDEN || j.off < 1 ||
             j.n < 1 || j.k < 1)
             return set_error(SVTAD_ERR_INVALID, "adapter_prep: bad job");
-        if (j.kind == SVTAD_PREP_CAST ? (int64_t)j.off * j.n * j.k % 8 != 0 : (j.k % 32 != 0 || j.n % 32 != 0))
+        if (j.kind == SVTAD_PREP_WIDEN && (!al16r(j.src) || j.src_f32 || j.gamma))
+            return set_error(SVTAD_ERR_INVALID, "adapter_prep: bad job");
+        if (j.kind == SVTAD_PREP_CAST || j.kind == SVTAD_PREP_WIDEN ? (int64_t)j.off * j.n * j.k % 8 != 0 : (j.k % 32 != 0 || j.n % 32 != 0))
             return set_error(SVTAD_ERR_UNSUPPORTED, "adapter_prep: shape without a layout");
         if ((int64_t)j.off * j.n * j.k >= (int64_t)INT32_MAX)
             return set_error(SVTAD_ERR_UNSUPPORTED, "adapter_prep: 2^31 values or more");
@@ -467,7 +482,7 @@ extern "C" int svtad_adapter_prep(const svtad_prep_job* jobs, int count, int dty
 }
 
 extern "C" int svtad_adapter_rows_ok(int kind, int k, int n) {
-    if (kind == SVTAD_ROWS_RES) return (k == 128 || k == 256) && n > 0 && n % 128 == 0;
+    if (kind == SVTAD_ROWS_RES) return (k == 64 || k == 128 || k == 256) && n > 0 && n % 128 == 0;
     return (kind == SVTAD_ROWS_GELU || kind == SVTAD_ROWS_SPLIT) && (k == 384 || k == 768 || k == 1024) &&
            (n == 128 || n == 256);
 }

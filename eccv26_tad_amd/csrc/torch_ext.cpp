@@ -970,6 +970,62 @@ bool op_adapter_rows_ok(int64_t embed, int64_t hidden) {
            svtad_adapter_rows_ok(SVTAD_ROWS_RES, (int)hidden, (int)embed);
 }
 
+// Jobs of one svtad_adapter_prep launch and the tensors they read.
+struct PrepList {
+    at::TensorOptions opt;  // the compute type
+    at::ScalarType t;
+    std::vector<svtad_prep_job> jobs;
+    std::vector<at::Tensor> keep;
+
+    explicit PrepList(const at::Tensor& like, bool bf16)
+        : opt(like.options().dtype(bf16 ? at::kBFloat16 : at::kHalf)), t(bf16 ? at::kBFloat16 : at::kHalf) {}
+
+    at::Tensor param(const at::Tensor& p) {
+        TORCH_CHECK(p.is_cuda() && p.device() == opt.device(), "adapter: parameters must share the GPU");
+        TORCH_CHECK(p.scalar_type() == t || p.scalar_type() == at::kFloat,
+                    "adapter: parameters take the compute type or float32, got ", p.scalar_type());
+        return p.contiguous();
+    }
+    void push(int kind, const at::Tensor& src, const at::Tensor& dst, int off, int64_t n, int64_t k, bool pair,
+              const at::Tensor* gamma) {
+        jobs.push_back(svtad_prep_job{src.data_ptr(), dst.data_ptr(), gamma ? gamma->data_ptr() : nullptr, kind, off, (int)n,
+                                      (int)k, kind != SVTAD_PREP_WIDEN && src.scalar_type() == at::kFloat,
+                                      gamma && gamma->scalar_type() == at::kFloat, pair});
+        keep.push_back(src);
+    }
+    at::Tensor add(int kind, const at::Tensor& src, int off, int64_t n, int64_t k, bool pair, const at::Tensor* gamma = nullptr,
+                   int64_t extra = 0) {
+        at::Tensor dst = at::empty({(int64_t)off * n * k + extra}, opt);
+        push(kind, src, dst, off, n, k, pair, gamma);
+        return dst;
+    }
+    at::Tensor cast(const at::Tensor& p_in) {  // in the compute type, 16-byte aligned
+        at::Tensor p = param(p_in);
+        if (p.scalar_type() == t) return ((uintptr_t)p.data_ptr() & 15) ? p.clone() : p;
+        if (p.numel() % 8) return p.to(t);
+        return add(SVTAD_PREP_CAST, p, 1, 1, p.numel(), false).view(p.sizes());
+    }
+    at::Tensor bias(const c10::optional<at::Tensor>& b, int64_t n) {
+        if (!bias_present(b)) return at::empty({0}, opt);
+        TORCH_CHECK(b->numel() == n, "adapter: a bias must have ", n, " elements");
+        return cast(*b);
+    }
+    // g (the compute type) in the parameter's type: converted by launch() to float32
+    at::Tensor grad(const at::Tensor& g, at::ScalarType want) {
+        if (!g.defined() || g.numel() == 0 || g.scalar_type() == want) return g;
+        if (want != at::kFloat || g.numel() % 8 || ((uintptr_t)g.data_ptr() & 15) || !g.is_contiguous()) return g.to(want);
+        at::Tensor dst = at::empty(g.sizes(), opt.dtype(at::kFloat));
+        push(SVTAD_PREP_WIDEN, g, dst, 1, 1, g.numel(), false, nullptr);
+        return dst;
+    }
+    void launch() {
+        if (!jobs.empty())
+            check_status(svtad_adapter_prep(jobs.data(), (int)jobs.size(), t == at::kHalf ? SVTAD_F16 : SVTAD_BF16,
+                                            stream_of(keep[0])),
+                         "adapter_prep");
+    }
+};
+
 // adapter_prep(w_d, b_d, w_c, b_c, w_u, b_u, gamma, bf16, train, pack_conv)
 //   -> [wd, b_d, wu, b_u, b_c, w_c, w_u, wdT, wuT, packed_fwd, packed_bwd]
 // One launch: the parameters (f32 or the compute type) cast, wd / wu in the
@@ -977,67 +1033,49 @@ bool op_adapter_rows_ok(int64_t embed, int64_t hidden) {
 // of the input gradient / the up projection's backward (scaled by gamma), w_u
 // as is; with pack_conv the SparseConv2D layouts of w_c (packed_bwd with
 // train). An item that is not wanted, or a missing bias, is empty.
-std::vector<at::Tensor> op_adapter_prep(const at::Tensor& w_d_in, const c10::optional<at::Tensor>& b_d,
-                                        const at::Tensor& w_c_in, const c10::optional<at::Tensor>& b_c,
-                                        const at::Tensor& w_u_in, const c10::optional<at::Tensor>& b_u,
-                                        const at::Tensor& gamma_in, bool bf16, bool train, bool pack_conv) {
-    const at::ScalarType t = bf16 ? at::kBFloat16 : at::kHalf;
-    const int dt = bf16 ? SVTAD_BF16 : SVTAD_F16;
-    check_gpu(w_d_in, "w_d");
-    auto param = [&](const at::Tensor& p) {
-        TORCH_CHECK(p.is_cuda() && p.device() == w_d_in.device(), "adapter_prep: parameters must share the GPU");
-        TORCH_CHECK(p.scalar_type() == t || p.scalar_type() == at::kFloat,
-                    "adapter_prep: parameters take the compute type or float32, got ", p.scalar_type());
-        return p.contiguous();
-    };
-    at::Tensor w_d = param(w_d_in), w_c = param(w_c_in), w_u = param(w_u_in), gm = param(gamma_in);
+static std::vector<at::Tensor> adapter_prep_jobs(PrepList& L, const at::Tensor& w_d_in, const c10::optional<at::Tensor>& b_d,
+                                                 const at::Tensor& w_c_in, const c10::optional<at::Tensor>& b_c,
+                                                 const at::Tensor& w_u_in, const c10::optional<at::Tensor>& b_u,
+                                                 const at::Tensor& gamma_in, bool train, bool pack_conv) {
+    const int dt = L.t == at::kHalf ? SVTAD_F16 : SVTAD_BF16;
+    at::Tensor w_d = L.param(w_d_in), w_c = L.param(w_c_in), w_u = L.param(w_u_in), gm = L.param(gamma_in);
     TORCH_CHECK(w_d.dim() == 2 && w_u.dim() == 2 && w_c.dim() == 3 && w_c.size(0) == 9 && gm.numel() == 1 &&
                     w_u.size(0) == w_d.size(1) && w_u.size(1) == w_d.size(0) && w_c.size(1) == w_d.size(0) &&
                     w_c.size(2) == w_d.size(0),
-                "adapter_prep: w_d [h, E], w_c [9, h, h], w_u [E, h] and a gamma of one element");
+                "adapter: w_d [h, E], w_c [9, h, h], w_u [E, h] and a gamma of one element");
     const int64_t h = w_d.size(0), E = w_d.size(1);
-    c10::DeviceGuard g(w_d.device());
-    const auto opt = w_d.options().dtype(t);
-    std::vector<svtad_prep_job> jobs;
-    std::vector<at::Tensor> keep;
-    auto add = [&](int kind, const at::Tensor& src, int off, int64_t n, int64_t k, bool pair, bool scaled, int64_t extra) {
-        at::Tensor dst = at::empty({(int64_t)off * n * k + extra}, opt);
-        jobs.push_back(svtad_prep_job{src.data_ptr(), dst.data_ptr(), scaled ? gm.data_ptr() : nullptr, kind, off, (int)n,
-                                      (int)k, src.scalar_type() == at::kFloat, gm.scalar_type() == at::kFloat, pair});
-        keep.push_back(src);
-        return dst;
-    };
-    auto cast = [&](const at::Tensor& p) {
-        if (p.scalar_type() == t) return ((uintptr_t)p.data_ptr() & 15) ? p.clone() : p;
-        if (p.numel() % 8) return p.to(t);
-        return add(SVTAD_PREP_CAST, p, 1, 1, p.numel(), false, false, 0).view(p.sizes());
-    };
-    auto bias = [&](const c10::optional<at::Tensor>& b, int64_t n) {
-        if (!bias_present(b)) return at::empty({0}, opt);
-        TORCH_CHECK(b->numel() == n, "adapter_prep: a bias must have ", n, " elements");
-        return cast(param(*b));
-    };
-    const at::Tensor none = at::empty({0}, opt), noneb = at::empty({0}, opt.dtype(at::kByte));
-    std::vector<at::Tensor> out(11, none);
-    out[0] = add(SVTAD_PREP_ROWS, w_d, 1, h, E, true, false, 0);
-    out[1] = bias(b_d, h);
-    out[2] = add(SVTAD_PREP_ROWS, w_u, 1, E, h, false, false, 0);
-    out[3] = bias(b_u, E);
-    out[4] = bias(b_c, h);
-    out[5] = cast(w_c);
+    std::vector<at::Tensor> out(11, at::empty({0}, L.opt));
+    out[0] = L.add(SVTAD_PREP_ROWS, w_d, 1, h, E, true);
+    out[1] = L.bias(b_d, h);
+    out[2] = L.add(SVTAD_PREP_ROWS, w_u, 1, E, h, false);
+    out[3] = L.bias(b_u, E);
+    out[4] = L.bias(b_c, h);
+    out[5] = L.cast(w_c);
     if (train) {
-        out[6] = cast(w_u);
-        out[7] = add(SVTAD_PREP_COLS, w_d, 1, E, h, false, false, 0);
-        out[8] = add(SVTAD_PREP_COLS, w_u, 1, h, E, true, true, 0);
+        out[6] = L.cast(w_u);
+        out[7] = L.add(SVTAD_PREP_COLS, w_d, 1, E, h, false);
+        L.keep.push_back(gm);
+        out[8] = L.add(SVTAD_PREP_COLS, w_u, 1, h, E, true, &gm);
     }
-    out[9] = out[10] = noneb;
+    out[9] = out[10] = at::empty({0}, L.opt.dtype(at::kByte));
     if (pack_conv) {
         const size_t bf = svtad_fwd_workspace_bytes((int)h, (int)h, dt), bb = svtad_bwd_in_workspace_bytes((int)h, (int)h, dt);
-        if (bf == (size_t)9 * h * h * 2) out[9] = add(SVTAD_PREP_CONV_FWD, w_c, 9, h, h, false, false, 0).view(at::kByte);
+        if (bf == (size_t)9 * h * h * 2) out[9] = L.add(SVTAD_PREP_CONV_FWD, w_c, 9, h, h, false).view(at::kByte);
         if (train && bb > bf && bf)
-            out[10] = add(SVTAD_PREP_CONV_BWD, w_c, 9, h, h, false, false, (int64_t)(bb - bf) / 2).view(at::kByte);
+            out[10] = L.add(SVTAD_PREP_CONV_BWD, w_c, 9, h, h, false, nullptr, (int64_t)(bb - bf) / 2).view(at::kByte);
     }
-    check_status(svtad_adapter_prep(jobs.data(), (int)jobs.size(), dt, stream_of(w_d)), "adapter_prep");
+    return out;
+}
+
+std::vector<at::Tensor> op_adapter_prep(const at::Tensor& w_d, const c10::optional<at::Tensor>& b_d, const at::Tensor& w_c,
+                                        const c10::optional<at::Tensor>& b_c, const at::Tensor& w_u,
+                                        const c10::optional<at::Tensor>& b_u, const at::Tensor& gamma, bool bf16, bool train,
+                                        bool pack_conv) {
+    check_gpu(w_d, "w_d");
+    c10::DeviceGuard g(w_d.device());
+    PrepList L(w_d, bf16);
+    auto out = adapter_prep_jobs(L, w_d, b_d, w_c, b_c, w_u, b_u, gamma, train, pack_conv);
+    L.launch();
     return out;
 }
 
@@ -1188,7 +1226,7 @@ std::tuple<at::Tensor, at::Tensor> op_layer_norm_rows(const at::Tensor& x_in, co
     attn_params(x, {&w, &b}, c);
     c10::DeviceGuard g(x.device());
     at::Tensor y = at::empty_like(x), stats = at::empty({rows, 2}, x.options().dtype(at::kFloat));
-    check_status(svtad_layer_norm(x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), stats.data_ptr<float>(), rows,
+    check_status(svtad_layer_norm(nullptr, x.data_ptr(), nullptr, rows, 0, w.data_ptr(), b.data_ptr(), y.data_ptr(), stats.data_ptr<float>(), rows,
                                   (int)c, (float)eps, dtype_code(x), w.scalar_type() == at::kFloat, stream_of(x)),
                  "layer_norm_rows");
     return {y, stats};
@@ -1208,8 +1246,8 @@ std::tuple<at::Tensor, at::Tensor> op_layer_norm_rows_bwd(const at::Tensor& dy_i
     at::Tensor dx = at::empty_like(x), dwb = at::empty({2, c}, f);
     const size_t ws = svtad_layer_norm_bwd_workspace_bytes(rows, (int)c);
     at::Tensor work = at::empty({(int64_t)ws}, f.dtype(at::kByte));
-    check_status(svtad_layer_norm_bwd(dy.data_ptr(), x.data_ptr(), stats.data_ptr<float>(), w.data_ptr(), dx.data_ptr(),
-                                      dwb.data_ptr<float>(), work.data_ptr(), ws, rows, (int)c, dtype_code(x),
+    check_status(svtad_layer_norm_bwd(dy.data_ptr(), x.data_ptr(), nullptr, stats.data_ptr<float>(), w.data_ptr(), nullptr,
+                                      dx.data_ptr(), rows, 0, dwb.data_ptr<float>(), work.data_ptr(), ws, rows, (int)c, dtype_code(x),
                                       w.scalar_type() == at::kFloat, stream_of(x)),
                  "layer_norm_rows_bwd");
     return {dx, dwb};
@@ -1264,7 +1302,228 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> op_key_attention_bwd(const at::Te
     return {dq, dkv, dn};
 }
 
+// ---------------------------------------------------------------------------
+// the adapter's forward and backward as one call each (widths of adapter_rows_ok)
+// ---------------------------------------------------------------------------
+
+enum { A_NW, A_NB, A_DW, A_DB, A_QW, A_QB, A_QNW, A_QNB, A_KNW, A_KNB, A_PW, A_PB, A_GAMMA, A_COUNT };
+enum { S_X, S_PRE, S_CBUF, S_PA, S_WC, S_WU, S_BU, S_WDT, S_WUT, S_PB, S_COUNT };
+enum { S_COMB = S_COUNT, S_STATS, S_XN, S_DW, S_XA, S_QW, S_Q, S_KV, S_ATT, S_PW, S_PBIAS, S_X2, S_ACOUNT };
+
+// adapter_forward(x [B, N, E], w_d, b_d, w_c, b_c, w_u, b_u, gamma, neighbor_indices, n_special, tokens_per_batch, bias_mode,
+//                 hm_rows, hm_gate, packed_fwd, packed_bwd, bf16, train, attn, nk, eps_norm, eps_head)
+//   -> [out, packed_fwd, packed_bwd, saved tensors of adapter_backward if train]
+// packed_fwd None: the SparseConv2D weight is packed here. attn holds the
+// parameters of the key-token attention (13 tensors), or nothing.
+std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor& w_d, const c10::optional<at::Tensor>& b_d,
+                                           const at::Tensor& w_c, const c10::optional<at::Tensor>& b_c,
+                                           const at::Tensor& w_u, const c10::optional<at::Tensor>& b_u,
+                                           const at::Tensor& gamma, const at::Tensor& nbr, int64_t S, int64_t tpb,
+                                           int64_t bias_mode, const c10::optional<at::Tensor>& hm_rows,
+                                           const c10::optional<at::Tensor>& hm_gate, const c10::optional<at::Tensor>& pf_in,
+                                           const c10::optional<at::Tensor>& pb_in, bool bf16, bool train,
+                                           const std::vector<at::Tensor>& attn, int64_t nk, double eps_norm, double eps_head) {
+    check_gpu(x, "x");
+    TORCH_CHECK(x.dim() == 3 && (attn.empty() || attn.size() == A_COUNT), "adapter_forward: x [B, N, E], 0 or 13 attn tensors");
+    c10::DeviceGuard g(x.device());
+    const int64_t B = x.size(0), N = x.size(1), h = w_d.size(0), M = B * N;
+    TORCH_CHECK(S >= 0 && S <= N, "n_special out of range");
+    PrepList L(x, bf16);
+    const bool pack = !pf_in.has_value();
+    auto P = adapter_prep_jobs(L, w_d, b_d, w_c, b_c, w_u, b_u, gamma, train, pack);
+    at::Tensor pf = pack ? P[9] : *pf_in, pb = pack ? P[10] : pb_in.has_value() ? *pb_in : P[10];
+    at::Tensor dw, db, qw, qb, pw, pwf, pbias;
+    const int64_t a = attn.empty() ? 0 : attn[A_DW].size(0);
+    if (a) {
+        dw = L.cast(attn[A_DW]);
+        db = L.cast(attn[A_DB]);
+        qw = L.cast(attn[A_QW]);
+        qb = L.cast(attn[A_QB]);
+        pwf = L.add(SVTAD_PREP_ROWS, L.param(attn[A_PW]), 1, h, a, false);
+        if (train) pw = L.cast(attn[A_PW]);
+        pbias = L.cast(attn[A_PB]);
+    }
+    L.launch();
+    // special rows first, then the patch rows' SparseConv2D output: the up
+    // projection's operand, and its weight gradient's in one row list
+    at::Tensor cbuf = at::empty({M, h}, L.opt);
+    at::Tensor sp = cbuf.narrow(0, 0, B * S).view({B, S, h}), conv = cbuf.narrow(0, B * S, M - B * S);
+    at::Tensor xin = rows_input(x), pre = at::empty({B, N, h}, L.opt), pa = at::empty({M - B * S, h}, L.opt);
+    rows_check(xin, P[0], x.size(2), h, "x");
+    const bool f32 = xin.scalar_type() == at::kFloat;
+    at::Tensor xc = train && f32 ? at::empty(x.sizes(), L.opt) : xin;
+    void* const st = stream_of(x);
+    const int dt = L.t == at::kHalf ? SVTAD_F16 : SVTAD_BF16;
+    svtad_rows_args r = rows_args(SVTAD_ROWS_GELU, B, N, S, x.size(2), h);
+    r.a0 = xin.data_ptr();
+    r.w = P[0].data_ptr();
+    r.bias = P[1].numel() ? P[1].data_ptr() : nullptr;
+    r.a_copy = train && f32 ? xc.data_ptr() : nullptr;
+    r.out0 = pre.data_ptr();
+    r.out1 = S ? sp.data_ptr() : nullptr;
+    r.out2 = pa.numel() ? pa.data_ptr() : nullptr;
+    r.a_f32 = f32;
+    check_status(svtad_adapter_rows(&r, dt, st), "adapter_forward");
+    if (hm_rows.has_value()) op_heatmap_add_(pa, sp, *hm_rows, *hm_gate);
+    at::Tensor tab = table_i32(nbr, pa.size(0));
+    int mode = P[4].numel() ? (int)bias_mode : SVTAD_BIAS_NONE;
+    if (mode == SVTAD_BIAS_FP32) mode = SVTAD_BIAS_PRE;  // the bias in the compute type, widened exactly
+    if (pf.numel())
+        check_status(svtad_fwd_packed(pa.data_ptr(), tab.data_ptr<int32_t>(), pf.data_ptr(),
+                                      mode ? P[4].data_ptr() : nullptr, mode, conv.data_ptr(), pa.size(0), (int)h, (int)h,
+                                      tpb, dt, st),
+                     "adapter_forward");
+    else
+        conv.copy_(conv_fwd(pa, tab, P[5], P[4], tpb, (int)bias_mode, -1));
+    at::Tensor comb, stats, xn, xa, q, kv, att, x2;
+    if (a) {
+        TORCH_CHECK(svtad_key_attention_ok(4, (int)a / 4, N, (int)nk), "adapter_forward: attention size");
+        attn_params(cbuf, {&attn[A_NW], &attn[A_NB]}, h);
+        comb = S ? at::empty({B, N, h}, L.opt) : conv.view({B, N, h});
+        xn = at::empty({M, h}, L.opt);
+        stats = at::empty({M, 2}, L.opt.dtype(at::kFloat));
+        check_status(svtad_layer_norm(S ? sp.data_ptr() : nullptr, conv.data_ptr(), S ? comb.data_ptr() : nullptr, N, S,
+                                      attn[A_NW].data_ptr(), attn[A_NB].data_ptr(), xn.data_ptr(), stats.data_ptr<float>(), M,
+                                      (int)h, (float)eps_norm, dt, attn[A_NW].scalar_type() == at::kFloat, st),
+                     "adapter_forward");
+        xa = at::addmm(db, xn, dw.t());
+        q = at::addmm(qb.narrow(0, 0, a), xa, qw.narrow(0, 0, a).t()).view({B, N, a});
+        at::Tensor xk = xa.view({B, N, a}).narrow(1, 0, nk).reshape({B * nk, a});
+        kv = at::addmm(qb.narrow(0, a, 2 * a), xk, qw.narrow(0, a, 2 * a).t()).view({B, nk, 2 * a});
+        att = op_key_attention(q, kv, attn[A_QNW], attn[A_QNB], attn[A_KNW], attn[A_KNB], eps_head);
+        x2 = op_adapter_rows_res(c10::nullopt, att, pwf, pbias, attn[A_GAMMA], comb, false);
+    }
+    const bool out32 = gamma.scalar_type() == at::kFloat;
+    at::Tensor out = a ? op_adapter_rows_res(c10::nullopt, x2, P[2], P[3], gamma, xin, out32)
+                       : op_adapter_rows_res(sp, conv, P[2], P[3], gamma, xin, out32);
+    std::vector<at::Tensor> ret{out, pf, pb};
+    if (!train) return ret;
+    for (const at::Tensor& t : {xc, pre, cbuf, pa, P[5], P[6], P[3], P[7], P[8], pb}) ret.push_back(t);
+    if (a)
+        for (const at::Tensor& t : {comb, stats, xn, dw, xa, qw, q, kv, att, pw, pbias, x2}) ret.push_back(t);
+    return ret;
+}
+
+// adapter_backward(go, saved, gamma, neighbor_indices, hm_rows, hm_gate, rows, attn, n_special, tokens_per_batch, nk, eps_head,
+//                  symmetric, has_bd, has_bc, need_x, need_wd, param types [w_d, b_d, w_c, b_c, w_u, b_u], x_float32)
+//   -> [gx, gw_d, gb_d, gw_c, gb_c, gw_u, gb_u, g_gamma, g_gate, attention parameters]
+// rows: the row of go of each row of the saved special / patch buffer.
+// Gradients that are not wanted or do not exist are empty.
+std::vector<at::Tensor> op_adapter_backward(const at::Tensor& go_in, const std::vector<at::Tensor>& saved,
+                                            const at::Tensor& gamma, const at::Tensor& nbr,
+                                            const c10::optional<at::Tensor>& hm_rows,
+                                            const c10::optional<at::Tensor>& hm_gate, const at::Tensor& rows,
+                                            const std::vector<at::Tensor>& attn, int64_t S, int64_t tpb, int64_t nk,
+                                            double eps_head, bool symmetric, bool has_bd, bool has_bc, bool need_x,
+                                            bool need_wd, const std::vector<bool>& f32, bool x_f32) {
+    const bool with_attn = !attn.empty();
+    TORCH_CHECK(saved.size() == (size_t)(with_attn ? S_ACOUNT : S_COUNT) && f32.size() == 6, "adapter_backward: bad saved tensors");
+    const at::Tensor &xc = saved[S_X], &pre = saved[S_PRE], &pa = saved[S_PA], &w_u = saved[S_WU], &b_u = saved[S_BU];
+    c10::DeviceGuard guard(pre.device());
+    const int64_t B = pre.size(0), N = pre.size(1), h = pre.size(2), M = B * N, E = xc.size(2);
+    const at::ScalarType t = pre.scalar_type();
+    const int dt = dtype_code(pre);
+    void* const st = stream_of(pre);
+    const auto opt = pre.options();
+    const at::Tensor none = at::empty({0}, opt), no_rows = at::empty({0}, opt.dtype(at::kInt));
+    PrepList L(pre, t == at::kBFloat16);
+    auto want = [&](int i) { return f32[i] ? at::kFloat : t; };
+    // gradients of (c W^T + b) gamma from G = go^T c (fp32) and the column sums of go
+    auto up_grads = [&](const at::Tensor& w, const at::Tensor& G, const at::Tensor& b, const at::Tensor& gs,
+                        const at::Tensor& gm_in, at::Tensor* w_sc, at::Tensor* gw, at::Tensor* gb) {
+        at::Tensor gm = gm_in.contiguous(), out = at::empty({1}, gm.options());
+        const bool bias = b.numel() > 0;
+        if (w_sc) *w_sc = at::empty_like(w);
+        *gw = at::empty_like(w);
+        *gb = bias ? at::empty_like(gs) : none;
+        const size_t wsb = svtad_gamma_grad_workspace_bytes();
+        at::Tensor work = at::empty({(int64_t)wsb}, opt.dtype(at::kByte));
+        check_status(svtad_gamma_grad_mixed(w.data_ptr(), G.data_ptr(), w.numel(), bias ? b.data_ptr() : nullptr,
+                                            bias ? gs.data_ptr() : nullptr, bias ? b.numel() : 0, out.data_ptr(),
+                                            gm.data_ptr(), w_sc ? w_sc->data_ptr() : nullptr, gw->data_ptr(),
+                                            bias ? gb->data_ptr() : nullptr, work.data_ptr(), wsb, dt, SVTAD_F32,
+                                            dtype_code(gm), st),
+                     "adapter_backward");
+        return out.view(gm_in.sizes());
+    };
+    at::Tensor go = go_in.contiguous();
+    at::Tensor g_sp, g_pa, goc;
+    std::tie(g_sp, g_pa, goc) = op_adapter_rows_split(go, saved[S_WUT], h, with_attn ? 0 : S, true);
+    if (go.scalar_type() == t) goc = go;
+    at::Tensor go2 = goc.view({M, E});
+    at::Tensor G = with_attn ? op_linear_wgrad(go2, no_rows, saved[S_X2].view({M, h}), true)
+                             : op_linear_wgrad(go2, rows, saved[S_CBUF], true);
+    at::Tensor gsum = b_u.numel() ? op_column_sums(go2) : none, gw_u, gb_u;
+    at::Tensor g_gamma = up_grads(w_u, G, b_u, gsum, gamma, nullptr, &gw_u, &gb_u);
+    std::vector<at::Tensor> ag;
+    if (with_attn) {
+        const at::Tensor &xn = saved[S_XN], &dw = saved[S_DW], &xa = saved[S_XA], &qw = saved[S_QW], &q = saved[S_Q],
+                         &kv = saved[S_KV], &att = saved[S_ATT], &pw = saved[S_PW], &pbias = saved[S_PBIAS];
+        const int64_t a = q.size(2);
+        at::Tensor dx2 = g_pa;  // [M, h], token order
+        at::Tensor pw_sc, gpw, gpb;
+        at::Tensor Gp = op_linear_wgrad(dx2, no_rows, att.view({M, a}), true);
+        at::Tensor g_ag = up_grads(pw, Gp, pbias, op_column_sums(dx2), attn[A_GAMMA], &pw_sc, &gpw, &gpb);
+        at::Tensor datt = at::mm(dx2, pw_sc), dq, dkv, dn;
+        std::tie(dq, dkv, dn) = op_key_attention_bwd(datt.view({B, N, a}), q, kv, attn[A_QNW], attn[A_QNB], attn[A_KNW],
+                                                     attn[A_KNB], eps_head);
+        at::Tensor dq2 = dq.view({M, a}), dkv2 = dkv.view({B * nk, 2 * a});
+        at::Tensor dxa = at::mm(dq2, qw.narrow(0, 0, a));
+        // a key row has no query: its gradient comes from its key and value
+        dxa.view({B, N, a}).narrow(1, 0, nk).copy_(at::mm(dkv2, qw.narrow(0, a, 2 * a)).view({B, nk, a}));
+        auto wt = [&](int i) { return attn[i].scalar_type(); };
+        at::Tensor xk = xa.view({B, N, a}).narrow(1, 0, nk).reshape({B * nk, a});
+        at::Tensor gqw = at::cat({op_linear_wgrad(dq2, no_rows, xa, false), at::mm(dkv2.t(), xk)});
+        at::Tensor gqb = at::cat({op_column_sums(dq2), dkv2.sum(0)});
+        at::Tensor gdw = op_linear_wgrad(dxa, no_rows, xn, wt(A_DW) == at::kFloat), gdb = op_column_sums(dxa);
+        at::Tensor dxn = at::mm(dxa, dw), dwb = at::empty({2, h}, opt.dtype(at::kFloat));
+        g_sp = at::empty({B, S, h}, opt);
+        g_pa = at::empty({M - B * S, h}, opt);
+        const size_t ws = svtad_layer_norm_bwd_workspace_bytes(M, (int)h);
+        at::Tensor work = at::empty({(int64_t)ws}, opt.dtype(at::kByte));
+        check_status(svtad_layer_norm_bwd(dxn.data_ptr(), saved[S_COMB].data_ptr(), dx2.data_ptr(),
+                                          saved[S_STATS].data_ptr<float>(), attn[A_NW].data_ptr(),
+                                          S ? g_sp.data_ptr() : nullptr, g_pa.data_ptr(), N, S, dwb.data_ptr<float>(),
+                                          work.data_ptr(), ws, M, (int)h, dt, attn[A_NW].scalar_type() == at::kFloat, st),
+                     "adapter_backward");
+        ag.resize(A_COUNT);
+        ag[A_NW] = dwb[0].to(wt(A_NW));
+        ag[A_NB] = dwb[1].to(wt(A_NB));
+        ag[A_DW] = gdw;
+        ag[A_DB] = L.grad(gdb, wt(A_DB));
+        ag[A_QW] = L.grad(gqw, wt(A_QW));
+        ag[A_QB] = L.grad(gqb, wt(A_QB));
+        for (int i = 0; i < 4; ++i) ag[A_QNW + i] = dn[i].to(wt(A_QNW + i));
+        ag[A_PW] = L.grad(gpw, wt(A_PW));
+        ag[A_PB] = L.grad(gpb, wt(A_PB));
+        ag[A_GAMMA] = g_ag;
+    }
+    at::Tensor gi, gw_c, gb_c;
+    std::tie(gi, gw_c, gb_c) = op_bwd_packed(g_pa, pa, nbr, saved[S_WC], saved[S_PB], h, tpb, has_bc, symmetric);
+    at::Tensor g_gate = none;
+    if (hm_rows.has_value()) {
+        // backward of patches + special[hm_rows] * gate: the gather's
+        // scatter-add into the special-token gradient, summed in float32 and
+        // rounded once, and the gate's sum
+        at::Tensor sp_rows = saved[S_CBUF].narrow(0, 0, B * S), gf = gi.to(at::kFloat);
+        g_gate = (gf * sp_rows.index_select(0, *hm_rows).to(at::kFloat)).sum().view(hm_gate->sizes()).to(hm_gate->scalar_type());
+        g_sp = g_sp.reshape({B * S, h}).to(at::kFloat).index_add(0, *hm_rows, gf * hm_gate->to(at::kFloat)).to(t).view({B, S, h});
+    }
+    at::Tensor du = op_gelu_backward_split(g_sp, gi, pre, S), du2 = du.view({M, h});
+    at::Tensor gx = need_x ? op_adapter_rows_res(c10::nullopt, du, saved[S_WDT], none, c10::nullopt, x_f32 ? go : goc, x_f32)
+                           : none;
+    at::Tensor gw_d = need_wd ? op_linear_wgrad(du2, no_rows, xc.view({M, E}), f32[0]) : none;
+    at::Tensor gb_d = has_bd ? L.grad(op_column_sums(du2), want(1)) : none;
+    std::vector<at::Tensor> ret{gx, gw_d, gb_d, L.grad(gw_c, want(2)), has_bc ? L.grad(gb_c, want(3)) : none,
+                                L.grad(gw_u, want(4)), b_u.numel() ? L.grad(gb_u, want(5)) : none, g_gamma, g_gate};
+    L.launch();
+    ret.insert(ret.end(), ag.begin(), ag.end());
+    return ret;
+}
+
 PYBIND11_MODULE(opentad_sparse_ops, m) {
+    m.def("adapter_forward", &op_adapter_forward, "The sparse-conv adapter's forward over whole token tiles");
+    m.def("adapter_backward", &op_adapter_backward, "Its backward");
     m.def("layer_norm_rows", &op_layer_norm_rows, "LayerNorm of rows of 128 or 256 channels (y, stats)", py::arg("x"),
           py::arg("w"), py::arg("b"), py::arg("eps"));
     m.def("layer_norm_rows_bwd", &op_layer_norm_rows_bwd, "LayerNorm backward (dx, [dw, db])", py::arg("dy"), py::arg("x"),

@@ -563,6 +563,7 @@ int svtad_gamma_grad_mixed(const void* w, const void* g, int64_t count, const vo
  * one launch. A job reads `src` (f32 with src_f32, else dtype), casts to dtype
  * and, with gamma, multiplies (rounding to dtype after each), and writes
  *   SVTAD_PREP_CAST      dst[i] = src[i], off * n * k values (a multiple of 8)
+ *   SVTAD_PREP_WIDEN     the same from dtype to an f32 dst
  *   SVTAD_PREP_ROWS      the fragment order of the [n, k] operand src [n, k]
  *   SVTAD_PREP_COLS      the same of its transpose, src [k, n]
  *   SVTAD_PREP_CONV_FWD  svtad_pack_weight's packed_fwd of src [9, k, n]
@@ -575,9 +576,10 @@ enum svtad_prep_kind {
     SVTAD_PREP_ROWS = 1,
     SVTAD_PREP_COLS = 2,
     SVTAD_PREP_CONV_FWD = 3,
-    SVTAD_PREP_CONV_BWD = 4
+    SVTAD_PREP_CONV_BWD = 4,
+    SVTAD_PREP_WIDEN = 5
 };
-enum { SVTAD_MAX_PREP_JOBS = 12 };
+enum { SVTAD_MAX_PREP_JOBS = 20 };
 typedef struct svtad_prep_job {
     const void* src;
     void* dst;
@@ -618,18 +620,22 @@ int svtad_adapter_rows(const svtad_rows_args* args, int dtype, void* stream);
  *
  * svtad_layer_norm: y = LayerNorm(x) over rows of 128 or 256 channels, and each
  * row's mean and 1 / std in stats [rows, 2]; svtad_layer_norm_bwd: dx, and the
- * gradients of w and b in dwb [2, c] (f32).
+ * gradients of w and b in dwb [2, c] (f32). With n_special > 0, x (dx) holds the
+ * rows of a sample's tokens after the first n_special and special (dx_special)
+ * those; copy, if not NULL, receives x in token order; add, if not NULL, is
+ * added to dx before its rounding.
  * svtad_key_attention: out [batch, n, a] = softmax(LN(q) LN(k)^T / sqrt(hd)) v per
  * head for the tokens after the first nk (whose rows are 0), q [batch, n, a],
  * kv [batch, nk, 2 a] (keys, then values); svtad_key_attention_bwd: dq (0 in the
  * key rows), dkv, and the gradients of qn_w, qn_b, kn_w, kn_b in dnorm [4, hd]
  * (f32). The sums over rows are ordered.
  */
-int svtad_layer_norm(const void* x, const void* w, const void* b, void* y, float* stats, int64_t rows, int c,
-                     float eps, int dtype, int param_f32, void* stream);
+int svtad_layer_norm(const void* special, const void* x, void* copy, int64_t n_tokens, int64_t n_special,
+                     const void* w, const void* b, void* y, float* stats, int64_t rows, int c, float eps, int dtype,
+                     int param_f32, void* stream);
 size_t svtad_layer_norm_bwd_workspace_bytes(int64_t rows, int c);
-int svtad_layer_norm_bwd(const void* dy, const void* x, const float* stats, const void* w, void* dx, float* dwb,
-                         void* workspace, size_t workspace_bytes, int64_t rows, int c, int dtype, int param_f32,
+int svtad_layer_norm_bwd(const void* dy, const void* x, const void* add, const float* stats, const void* w,
+                         void* dx_special, void* dx, int64_t n_tokens, int64_t n_special, float* dwb, void* workspace, size_t workspace_bytes, int64_t rows, int c, int dtype, int param_f32,
                          void* stream);
 int svtad_key_attention_ok(int heads, int head_dim, int64_t n, int nk);
 int svtad_key_attention(const void* q, const void* kv, const void* qn_w, const void* qn_b, const void* kn_w,

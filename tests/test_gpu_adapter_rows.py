@@ -82,3 +82,52 @@ def test_rows_match_float64(dev, embed, hidden, B, N, S, cd, param):
     acc = (h + 4) * eps * (a.abs() @ cast[0].abs() + x.double().abs())
     got = ops.adapter_rows_res(None, du, wdT, du.new_empty(0), None, x, PT == torch.float32)
     _near("gx", got, y, (0 if PT == torch.float32 else u) * y.abs() + acc + 1e-7)
+
+
+@pytest.mark.parametrize("embed,attn,S,heat", [(384, 0, 2, False), (768, 2, 3, False), (384, 2, 1, False), (1024, 2, 5, False),
+                                               (768, 0, 31, True), (768, 0, 0, False)])
+@pytest.mark.parametrize("amp", [True, False])
+def test_module_gradients_match_float32(dev, embed, attn, S, heat, amp):
+    """The native forward and backward of the module against the float32
+    restatement of the reference adapter, every gradient."""
+    from tests.adapter_ref import adapter_fp32, gain_scales
+    import eccv26_tad_amd as sv
+
+    B, T, H, W = 2, 3, 5, 6
+    g = torch.Generator(device=dev).manual_seed(embed + S + attn)
+    kw = dict(heatmap_grid_size=(H, W)) if heat else {}
+    mod = sv.SparseConvAdapter(embed, 0.25, use_attn=attn, n_key_tokens=max(S, 1), **kw).to(dev)
+    with torch.no_grad():
+        for name, p in mod.named_parameters():
+            if name.endswith("weight") and p.dim() > 1:
+                p.copy_(torch.randn(p.shape, generator=g, device=dev) * p.shape[-1] ** -0.5)
+            else:
+                p.add_(0.2 * torch.randn(p.shape, generator=g, device=dev) + 0.1)
+    cd = torch.bfloat16 if amp else torch.float16
+    dt = torch.float32 if amp else cd
+    mod = mod.to(dt)
+    mask = torch.zeros(B, T * H * W, dtype=torch.uint8, device=dev)
+    idx = torch.rand(B, T * H * W, generator=g, device=dev).topk(40, 1).indices.sort(1).values
+    mask.scatter_(1, idx, 1)
+    table = sv.build_neighbor_table(mask.view(B, T, H, W), batched=True, n=80)
+    x = torch.randn(B, S + 40, embed, generator=g, device=dev).to(dt).requires_grad_(True)
+    go = (torch.randn(B, S + 40, embed, generator=g, device=dev) + 0.5).to(dt)
+    args = (H, W, idx, T * H * W)
+    with torch.autocast("cuda", dtype=cd, enabled=amp):
+        y = mod(x, *args, table)
+    names = [n for n, _ in mod.named_parameters() if n != "k_norm.bias" and (heat or n != "heatmap_gate")]
+    grads = torch.autograd.grad(y, [x] + [mod.get_parameter(n) for n in names], go)
+    xr = x.detach().float().requires_grad_(True)
+    gains = {}
+    yr, P = adapter_fp32(mod, xr, *args, gains=gains)
+    yr.backward(go.float())
+    scales = gain_scales(gains)
+    tol = 2.5e-2 if amp else 4e-3  # a few roundings of each chain in bf16 / f16
+    assert float((y.float() - yr).norm() / yr.norm()) <= tol
+    for name, got in zip(["x"] + names, grads):
+        want = xr.grad if name == "x" else P[name].grad
+        assert got.dtype == dt and got.shape == want.shape, name
+        err = float((got.float() - want).norm())
+        # a scalar gain's gradient against its sum of absolute terms
+        bar = tol * scales[name] * 0.2 if name in scales else tol * float(want.norm())
+        assert err <= bar, (name, err, bar)
