@@ -364,6 +364,64 @@ __global__ __launch_bounds__(4 * HD) void k_key_attn_keys(KeyAttnArgs p, const f
 }
 
 static bool al16a(const void* p) { return ((uintptr_t)p & 15) == 0; }
+// ---------------------------------------------------------------------------
+// projection of the few key rows (a library product costs the host 40 us for
+// these 6 x 256 x 128 values; both launches here 3-5 us)
+// ---------------------------------------------------------------------------
+constexpr int kKeyRowsMax = 64;
+
+// one workgroup of 2 A threads per key row, one output column per thread
+template <typename T, int A>
+__global__ __launch_bounds__(2 * A) void k_key_proj(const T* __restrict__ xa, const T* __restrict__ w,
+                                                    const T* __restrict__ b, T* __restrict__ kv, int64_t n, int nk) {
+    __shared__ float x[A];
+    const int row = blockIdx.x, c = threadIdx.x;
+    if (c < A) x[c] = (float)xa[((int64_t)(row / nk) * n + row % nk) * A + c];
+    __syncthreads();
+    float s = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < A; k += 8) {
+        const RowVec<T, 8> v = *(const RowVec<T, 8>*)(w + (int64_t)c * A + k);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += x[k + e] * (float)v.e[e];
+    }
+    kv[(int64_t)row * 2 * A + c] = (T)(s + (float)b[c]);
+}
+
+// workgroups of A threads: [0, 2 A) one row of dw (and its db), then one key
+// row of dxa each
+template <typename T, int A>
+__global__ __launch_bounds__(A) void k_key_proj_bwd(const T* __restrict__ dkv, const T* __restrict__ xa,
+                                                    const T* __restrict__ w, T* __restrict__ dxa, void* __restrict__ dw,
+                                                    void* __restrict__ db, int64_t n, int nk, int rows, bool w32, bool b32) {
+    __shared__ float g[2 * A > kKeyRowsMax ? 2 * A : kKeyRowsMax];
+    const int c = threadIdx.x;
+    if ((int)blockIdx.x < 2 * A) {
+        const int o = blockIdx.x;
+        for (int r = c; r < rows; r += A) g[r] = (float)dkv[(int64_t)r * 2 * A + o];
+        __syncthreads();
+        float s = 0.f, t = 0.f;
+        for (int r = 0; r < rows; ++r) {
+            s += g[r] * (float)xa[((int64_t)(r / nk) * n + r % nk) * A + c];
+            t += g[r];
+        }
+        if (w32) ((float*)dw)[o * A + c] = s;
+        else ((T*)dw)[o * A + c] = (T)s;
+        if (c == 0) {
+            if (b32) ((float*)db)[o] = t;
+            else ((T*)db)[o] = (T)t;
+        }
+        return;
+    }
+    const int row = blockIdx.x - 2 * A;
+    for (int e = c; e < 2 * A; e += A) g[e] = (float)dkv[(int64_t)row * 2 * A + e];
+    __syncthreads();
+    float s = 0.f;
+#pragma unroll 8
+    for (int e = 0; e < 2 * A; ++e) s += g[e] * (float)w[(int64_t)e * A + c];
+    dxa[((int64_t)(row / nk) * n + row % nk) * A + c] = (T)s;
+}
+
 static bool half_type(int d) { return d == SVTAD_F16 || d == SVTAD_BF16; }
 
 }  // namespace svtad
@@ -510,3 +568,44 @@ extern "C" int svtad_key_attention_bwd(const void* dout, const void* q, const vo
 #undef SVTAD_KK
     return launch_status();
 }
+
+static int key_proj_check(const char* what, int64_t batch, int64_t n, int nk, int a, int dtype) {
+    if (!half_type(dtype) || (a != 64 && a != 128)) return set_error(SVTAD_ERR_UNSUPPORTED, what);
+    if (batch < 1 || nk < 1 || n < nk || batch * nk > kKeyRowsMax) return set_error(SVTAD_ERR_UNSUPPORTED, what);
+    return SVTAD_OK;
+}
+
+#define SVTAD_KP(K, ...)                                                            \
+    if (dtype == SVTAD_F16) {                                                       \
+        if (a == 64) { K(f16, 64); } else { K(f16, 128); }                          \
+    } else {                                                                        \
+        if (a == 64) { K(bf16, 64); } else { K(bf16, 128); }                        \
+    }
+
+extern "C" int svtad_key_proj(const void* xa, const void* w, const void* b, void* kv, int64_t batch, int64_t n, int nk, int a,
+                              int dtype, void* stream) {
+    const int st = key_proj_check("key_proj: f16 / bf16, a 64 or 128, at most 64 key rows", batch, n, nk, a, dtype);
+    if (st) return st;
+    if (!xa || !w || !b || !kv || !al16a(w)) return set_error(SVTAD_ERR_INVALID, "key_proj: bad pointer");
+#define SVTAD_KP1(T, A)                                                                                            \
+    hipLaunchKernelGGL((k_key_proj<T, A>), dim3((unsigned)(batch * nk)), dim3(2 * A), 0, (hipStream_t)stream, (const T*)xa, \
+                       (const T*)w, (const T*)b, (T*)kv, n, nk)
+    SVTAD_KP(SVTAD_KP1)
+#undef SVTAD_KP1
+    return launch_status();
+}
+
+extern "C" int svtad_key_proj_bwd(const void* dkv, const void* xa, const void* w, void* dxa, void* dw, void* db, int64_t batch,
+                                  int64_t n, int nk, int a, int dtype, int dw_f32, int db_f32, void* stream) {
+    const int st = key_proj_check("key_proj_bwd: f16 / bf16, a 64 or 128, at most 64 key rows", batch, n, nk, a, dtype);
+    if (st) return st;
+    if (!dkv || !xa || !w || !dxa || !dw || !db) return set_error(SVTAD_ERR_INVALID, "key_proj_bwd: null pointer");
+#define SVTAD_KP1(T, A)                                                                                                \
+    hipLaunchKernelGGL((k_key_proj_bwd<T, A>), dim3((unsigned)(2 * A + batch * nk)), dim3(A), 0, (hipStream_t)stream,  \
+                       (const T*)dkv, (const T*)xa, (const T*)w, (T*)dxa, dw, db, n, nk, (int)(batch * nk), dw_f32 != 0, \
+                       db_f32 != 0)
+    SVTAD_KP(SVTAD_KP1)
+#undef SVTAD_KP1
+    return launch_status();
+}
+#undef SVTAD_KP

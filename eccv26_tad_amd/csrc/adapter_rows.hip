@@ -116,7 +116,7 @@ struct RowsArgs {
     int64_t n_tiles;
 };
 
-enum { ROWS_GELU = 0, ROWS_SPLIT = 1, ROWS_RES = 2 };
+enum { ROWS_GELU = 0, ROWS_SPLIT = 1, ROWS_RES = 2, ROWS_PLAIN = 3 };
 
 __device__ __forceinline__ float gelu_erf_rows(float u) { return 0.5f * u * (1.0f + erff(u * 0.70710678118654752f)); }
 
@@ -131,6 +131,7 @@ __device__ __forceinline__ float gelu_erf_rows(float u) { return 0.5f * u * (1.0
 // EPI: ROWS_GELU   out0 = z = T(acc + bias); GELU(z) split into out1 (special)
 //                  and out2 (patch rows)
 //      ROWS_SPLIT  T(acc) split into out1 and out2
+//      ROWS_PLAIN  out0 = T(acc + bias)
 //      ROWS_RES    with gamma: out0 = T?(z) gamma + res, else out0 = acc + res
 // AF32: A rows are fp32. ASPLIT: A rows come from a0 / a1 by token kind.
 // GF32 / RF32 / OF32: gamma, residual, output in fp32 (else T); a fp32 gamma
@@ -342,13 +343,13 @@ __global__ __launch_bounds__(256, K > 768 && FM == 2 ? 2 : 3) void k_adapter_row
     }
     // 16-bit outputs from the MFMA layout, 16 bytes per pair of fragments
     const uint32_t oel = (uint32_t)(r16 * p.n_out + col0 + g * 8);  // first output element of the lane in the tile
-    const rsrc_t rso = EPI == ROWS_GELU ? tile_rsrc(p.out0, p.n_out, 2) : make_rsrc(p.a0, 0u);
+    const rsrc_t rso = EPI != ROWS_SPLIT ? tile_rsrc(p.out0, p.n_out, 2) : make_rsrc(p.a0, 0u);
 #pragma unroll
     for (int a = 0; a < FM; ++a) {
         const int64_t m = row0 + a * 16 + r16;
         const bool ok = m < p.m_rows;
-        bool sp;
-        const int64_t rs = split(ok ? m : 0, sp);
+        bool sp = false;
+        const int64_t rs = EPI == ROWS_PLAIN ? 0 : split(ok ? m : 0, sp);
 #pragma unroll
         for (int v = 0; v < FN / 2; ++v) {
             u32x4 o, ge;
@@ -361,9 +362,9 @@ __global__ __launch_bounds__(256, K > 768 && FM == 2 ? 2 : 3) void k_adapter_row
                     ge[h] = (unsigned)__builtin_bit_cast(u16, (T)gelu_erf_rows((float)lo)) |
                             ((unsigned)__builtin_bit_cast(u16, (T)gelu_erf_rows((float)hi)) << 16);
             }
-            if constexpr (EPI == ROWS_GELU)
+            if constexpr (EPI != ROWS_SPLIT)
                 __builtin_amdgcn_raw_buffer_store_b128(o, rso, (oel + (uint32_t)(a * 16 * p.n_out + v * 32)) * 2u, 0, 0);
-            if (ok) *(u32x4*)((T*)(sp ? p.out1 : p.out2) + rs * p.n_out + col0 + v * 32 + g * 8) = EPI == ROWS_GELU ? ge : o;
+            if (EPI != ROWS_PLAIN && ok) *(u32x4*)((T*)(sp ? p.out1 : p.out2) + rs * p.n_out + col0 + v * 32 + g * 8) = EPI == ROWS_GELU ? ge : o;
         }
     }
 }
@@ -419,6 +420,12 @@ template <typename T>
 static bool rows_gemm(const RowsArgs& p, int epi, int k, bool af32, bool asplit, bool g32, bool r32, bool o32, hipStream_t s) {
     if (epi == ROWS_GELU) return rows_in_k<T, ROWS_GELU>(p, k, af32, s);
     if (epi == ROWS_SPLIT) return rows_in_k<T, ROWS_SPLIT>(p, k, af32, s);
+    if (epi == ROWS_PLAIN) {  // 17250 rows, 256 -> 128, 128 -> 128, 128 -> 256: 6.3, 5.4, 6.6 us
+        if (af32) return false;
+        if (k == 128) launch_rows<T, ROWS_PLAIN, 128, 2, 2, 4, false, false, false, false, false>(p, s);
+        else launch_rows<T, ROWS_PLAIN, 256, 2, 2, 8, false, false, false, false, false>(p, s);
+        return true;
+    }
 #define SVTAD_O(KK, SP, G, R, O)                                                              \
     if (k == KK && asplit == SP && g32 == G && r32 == R && o32 == O) {                        \
         rows_out<T, KK, SP, G, R, O>(p, s);                                                   \
@@ -482,6 +489,7 @@ extern "C" int svtad_adapter_prep(const svtad_prep_job* jobs, int count, int dty
 }
 
 extern "C" int svtad_adapter_rows_ok(int kind, int k, int n) {
+    if (kind == SVTAD_ROWS_PLAIN) return (k == 128 || k == 256) && n > 0 && n % 128 == 0;
     if (kind == SVTAD_ROWS_RES) return (k == 64 || k == 128 || k == 256) && n > 0 && n % 128 == 0;
     return (kind == SVTAD_ROWS_GELU || kind == SVTAD_ROWS_SPLIT) && (k == 384 || k == 768 || k == 1024) &&
            (n == 128 || n == 256);
@@ -500,8 +508,8 @@ extern "C" int svtad_adapter_rows(const svtad_rows_args* a, int dtype, void* str
     const bool any_sp = a->n_special > 0, any_pa = a->n_tokens > a->n_special;
     const bool split_src = res && a->a_patch_split;
     if (!a->w || (split_src ? (any_sp && !a->a0) || (any_pa && !a->a1) : !a->a0) ||
-        (res ? !a->res || !a->out0 : (any_sp && !a->out1) || (any_pa && !a->out2)) ||
-        (a->kind == SVTAD_ROWS_GELU && !a->out0))
+        (res ? !a->res || !a->out0 : a->kind != SVTAD_ROWS_PLAIN && ((any_sp && !a->out1) || (any_pa && !a->out2))) ||
+        ((a->kind == SVTAD_ROWS_GELU || a->kind == SVTAD_ROWS_PLAIN) && !a->out0))
         return set_error(SVTAD_ERR_INVALID, "adapter_rows: null pointer");
     for (const void* q : {a->a0, a->a1, a->w, a->bias, a->res, (const void*)a->a_copy, (const void*)a->out0,
                           (const void*)a->out1, (const void*)a->out2})
@@ -521,7 +529,7 @@ extern "C" int svtad_adapter_rows(const svtad_rows_args* a, int dtype, void* str
     p.n_out = a->n;
     p.n_tokens = (uint32_t)a->n_tokens;
     p.n_special = (uint32_t)a->n_special;
-    const int epi = res ? ROWS_RES : a->kind == SVTAD_ROWS_GELU ? ROWS_GELU : ROWS_SPLIT;
+    const int epi = a->kind;  // the public kinds are ROWS_*
     const bool done = dtype == SVTAD_F16
                           ? rows_gemm<f16>(p, epi, a->k, a->a_f32, split_src, a->gamma_f32, a->res_f32, a->out_f32, (hipStream_t)stream)
                           : rows_gemm<bf16>(p, epi, a->k, a->a_f32, split_src, a->gamma_f32, a->res_f32, a->out_f32, (hipStream_t)stream);

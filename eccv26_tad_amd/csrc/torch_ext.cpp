@@ -1308,7 +1308,21 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> op_key_attention_bwd(const at::Te
 
 enum { A_NW, A_NB, A_DW, A_DB, A_QW, A_QB, A_QNW, A_QNB, A_KNW, A_KNB, A_PW, A_PB, A_GAMMA, A_COUNT };
 enum { S_X, S_PRE, S_CBUF, S_PA, S_WC, S_WU, S_BU, S_WDT, S_WUT, S_PB, S_COUNT };
-enum { S_COMB = S_COUNT, S_STATS, S_XN, S_DW, S_XA, S_QW, S_Q, S_KV, S_ATT, S_PW, S_PBIAS, S_X2, S_ACOUNT };
+enum { S_COMB = S_COUNT, S_STATS, S_XN, S_DW, S_XA, S_QW, S_Q, S_KV, S_ATT, S_PW, S_PBIAS, S_X2, S_DWT, S_QWT, S_PWT, S_ACOUNT };
+
+// x [M, k] W^T + bias, [M, n] in x's type (W in fragment order, pair columns)
+static at::Tensor rows_plain(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, int64_t n) {
+    const int64_t M = x.size(0), k = x.size(1);
+    at::Tensor out = at::empty({M, n}, x.options());
+    at::Tensor b = bias.numel() && ((uintptr_t)bias.data_ptr() & 15) ? bias.clone() : bias;
+    svtad_rows_args r = rows_args(SVTAD_ROWS_PLAIN, 1, M, 0, k, n);
+    r.a0 = x.data_ptr();
+    r.w = w.data_ptr();
+    r.bias = b.numel() ? b.data_ptr() : nullptr;
+    r.out0 = out.data_ptr();
+    check_status(svtad_adapter_rows(&r, dtype_code(x), stream_of(x)), "adapter_rows");
+    return out;
+}
 
 // adapter_forward(x [B, N, E], w_d, b_d, w_c, b_c, w_u, b_u, gamma, neighbor_indices, n_special, tokens_per_batch, bias_mode,
 //                 hm_rows, hm_gate, packed_fwd, packed_bwd, bf16, train, attn, nk, eps_norm, eps_head)
@@ -1332,7 +1346,7 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
     const bool pack = !pf_in.has_value();
     auto P = adapter_prep_jobs(L, w_d, b_d, w_c, b_c, w_u, b_u, gamma, train, pack);
     at::Tensor pf = pack ? P[9] : *pf_in, pb = pack ? P[10] : pb_in.has_value() ? *pb_in : P[10];
-    at::Tensor dw, db, qw, qb, pw, pwf, pbias;
+    at::Tensor dw, db, qw, qb, pw, pwf, pbias, dwf, qwf, dwt, qwt, pwt;
     const int64_t a = attn.empty() ? 0 : attn[A_DW].size(0);
     if (a) {
         dw = L.cast(attn[A_DW]);
@@ -1341,6 +1355,18 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
         qb = L.cast(attn[A_QB]);
         pwf = L.add(SVTAD_PREP_ROWS, L.param(attn[A_PW]), 1, h, a, false);
         if (train) pw = L.cast(attn[A_PW]);
+        if (svtad_adapter_rows_ok(SVTAD_ROWS_PLAIN, (int)h, (int)a)) {  // and so a -> a, a -> h
+            at::Tensor d = L.param(attn[A_DW]), qq = L.param(attn[A_QW]).narrow(0, 0, a);
+            dwf = L.add(SVTAD_PREP_ROWS, d, 1, a, h, true);
+            qwf = L.add(SVTAD_PREP_ROWS, qq, 1, a, a, true);
+            if (train) {
+                at::Tensor gm = L.param(attn[A_GAMMA]), pp = L.param(attn[A_PW]);
+                L.keep.push_back(gm);
+                dwt = L.add(SVTAD_PREP_COLS, d, 1, h, a, true);
+                qwt = L.add(SVTAD_PREP_COLS, qq, 1, a, a, true);
+                pwt = L.add(SVTAD_PREP_COLS, pp, 1, a, h, true, &gm);
+            }
+        }
         pbias = L.cast(attn[A_PB]);
     }
     L.launch();
@@ -1386,10 +1412,18 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
                                       attn[A_NW].data_ptr(), attn[A_NB].data_ptr(), xn.data_ptr(), stats.data_ptr<float>(), M,
                                       (int)h, (float)eps_norm, dt, attn[A_NW].scalar_type() == at::kFloat, st),
                      "adapter_forward");
-        xa = at::addmm(db, xn, dw.t());
-        q = at::addmm(qb.narrow(0, 0, a), xa, qw.narrow(0, 0, a).t()).view({B, N, a});
-        at::Tensor xk = xa.view({B, N, a}).narrow(1, 0, nk).reshape({B * nk, a});
-        kv = at::addmm(qb.narrow(0, a, 2 * a), xk, qw.narrow(0, a, 2 * a).t()).view({B, nk, 2 * a});
+        xa = dwf.defined() ? rows_plain(xn, dwf, db, a) : at::addmm(db, xn, dw.t());
+        q = (qwf.defined() ? rows_plain(xa, qwf, qb.narrow(0, 0, a), a) : at::addmm(qb.narrow(0, 0, a), xa, qw.narrow(0, 0, a).t()))
+                .view({B, N, a});
+        if (B * nk <= 64) {
+            kv = at::empty({B, nk, 2 * a}, L.opt);
+            check_status(svtad_key_proj(xa.data_ptr(), qw.narrow(0, a, 2 * a).data_ptr(), qb.narrow(0, a, 2 * a).data_ptr(),
+                                        kv.data_ptr(), B, N, (int)nk, (int)a, dt, st),
+                         "adapter_forward");
+        } else {
+            at::Tensor xk = xa.view({B, N, a}).narrow(1, 0, nk).reshape({B * nk, a});
+            kv = at::addmm(qb.narrow(0, a, 2 * a), xk, qw.narrow(0, a, 2 * a).t()).view({B, nk, 2 * a});
+        }
         att = op_key_attention(q, kv, attn[A_QNW], attn[A_QNB], attn[A_KNW], attn[A_KNB], eps_head);
         x2 = op_adapter_rows_res(c10::nullopt, att, pwf, pbias, attn[A_GAMMA], comb, false);
     }
@@ -1400,7 +1434,8 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
     if (!train) return ret;
     for (const at::Tensor& t : {xc, pre, cbuf, pa, P[5], P[6], P[3], P[7], P[8], pb}) ret.push_back(t);
     if (a)
-        for (const at::Tensor& t : {comb, stats, xn, dw, xa, qw, q, kv, att, pw, pbias, x2}) ret.push_back(t);
+        for (const at::Tensor& t : {comb, stats, xn, dw, xa, qw, q, kv, att, pw, pbias, x2, dwt, qwt, pwt})
+            ret.push_back(t.defined() ? t : at::empty({0}, L.opt));
     return ret;
 }
 
@@ -1463,20 +1498,33 @@ std::vector<at::Tensor> op_adapter_backward(const at::Tensor& go_in, const std::
         at::Tensor dx2 = g_pa;  // [M, h], token order
         at::Tensor pw_sc, gpw, gpb;
         at::Tensor Gp = op_linear_wgrad(dx2, no_rows, att.view({M, a}), true);
-        at::Tensor g_ag = up_grads(pw, Gp, pbias, op_column_sums(dx2), attn[A_GAMMA], &pw_sc, &gpw, &gpb);
-        at::Tensor datt = at::mm(dx2, pw_sc), dq, dkv, dn;
+        const bool plain = saved[S_DWT].numel() > 0;
+        at::Tensor g_ag = up_grads(pw, Gp, pbias, op_column_sums(dx2), attn[A_GAMMA], plain ? nullptr : &pw_sc, &gpw, &gpb);
+        at::Tensor datt = plain ? rows_plain(dx2, saved[S_PWT], none, a) : at::mm(dx2, pw_sc), dq, dkv, dn;
         std::tie(dq, dkv, dn) = op_key_attention_bwd(datt.view({B, N, a}), q, kv, attn[A_QNW], attn[A_QNB], attn[A_KNW],
                                                      attn[A_KNB], eps_head);
         at::Tensor dq2 = dq.view({M, a}), dkv2 = dkv.view({B * nk, 2 * a});
-        at::Tensor dxa = at::mm(dq2, qw.narrow(0, 0, a));
-        // a key row has no query: its gradient comes from its key and value
-        dxa.view({B, N, a}).narrow(1, 0, nk).copy_(at::mm(dkv2, qw.narrow(0, a, 2 * a)).view({B, nk, a}));
+        at::Tensor dxa = plain ? rows_plain(dq2, saved[S_QWT], none, a) : at::mm(dq2, qw.narrow(0, 0, a));
         auto wt = [&](int i) { return attn[i].scalar_type(); };
-        at::Tensor xk = xa.view({B, N, a}).narrow(1, 0, nk).reshape({B * nk, a});
-        at::Tensor gqw = at::cat({op_linear_wgrad(dq2, no_rows, xa, false), at::mm(dkv2.t(), xk)});
-        at::Tensor gqb = at::cat({op_column_sums(dq2), dkv2.sum(0)});
+        at::Tensor gqw, gqb;
+        // a key row has no query: its gradient comes from its key and value
+        if (B * nk <= 64) {
+            gqw = at::empty({3 * a, a}, opt.dtype(wt(A_QW)));
+            gqb = at::empty({3 * a}, opt);
+            gqw.narrow(0, 0, a).copy_(op_linear_wgrad(dq2, no_rows, xa, wt(A_QW) == at::kFloat));
+            gqb.narrow(0, 0, a).copy_(op_column_sums(dq2));
+            check_status(svtad_key_proj_bwd(dkv.data_ptr(), xa.data_ptr(), qw.narrow(0, a, 2 * a).data_ptr(), dxa.data_ptr(),
+                                            gqw.narrow(0, a, 2 * a).data_ptr(), gqb.narrow(0, a, 2 * a).data_ptr(), B, N,
+                                            (int)nk, (int)a, dt, wt(A_QW) == at::kFloat, 0, st),
+                         "adapter_backward");
+        } else {
+            at::Tensor xk = xa.view({B, N, a}).narrow(1, 0, nk).reshape({B * nk, a});
+            dxa.view({B, N, a}).narrow(1, 0, nk).copy_(at::mm(dkv2, qw.narrow(0, a, 2 * a)).view({B, nk, a}));
+            gqw = at::cat({op_linear_wgrad(dq2, no_rows, xa, false), at::mm(dkv2.t(), xk)});
+            gqb = at::cat({op_column_sums(dq2), dkv2.sum(0)});
+        }
         at::Tensor gdw = op_linear_wgrad(dxa, no_rows, xn, wt(A_DW) == at::kFloat), gdb = op_column_sums(dxa);
-        at::Tensor dxn = at::mm(dxa, dw), dwb = at::empty({2, h}, opt.dtype(at::kFloat));
+        at::Tensor dxn = plain ? rows_plain(dxa, saved[S_DWT], none, h) : at::mm(dxa, dw), dwb = at::empty({2, h}, opt.dtype(at::kFloat));
         g_sp = at::empty({B, S, h}, opt);
         g_pa = at::empty({M - B * S, h}, opt);
         const size_t ws = svtad_layer_norm_bwd_workspace_bytes(M, (int)h);

@@ -568,8 +568,8 @@ int svtad_gamma_grad_mixed(const void* w, const void* g, int64_t count, const vo
  *   SVTAD_PREP_COLS      the same of its transpose, src [k, n]
  *   SVTAD_PREP_CONV_FWD  svtad_pack_weight's packed_fwd of src [9, k, n]
  *   SVTAD_PREP_CONV_BWD  svtad_pack_weight's packed_bwd of src [9, n, k]
- * n and k are multiples of 32 in the layouts. `pair` is 1 for the weight of
- * SVTAD_ROWS_GELU / _SPLIT and 0 for that of SVTAD_ROWS_RES (column order).
+ * n and k are multiples of 32 in the layouts. `pair` is 0 for the weight of
+ * SVTAD_ROWS_RES and 1 for those of the other kinds (column order).
  */
 enum svtad_prep_kind {
     SVTAD_PREP_CAST = 0,
@@ -579,7 +579,7 @@ enum svtad_prep_kind {
     SVTAD_PREP_CONV_BWD = 4,
     SVTAD_PREP_WIDEN = 5
 };
-enum { SVTAD_MAX_PREP_JOBS = 20 };
+enum { SVTAD_MAX_PREP_JOBS = 28 };
 typedef struct svtad_prep_job {
     const void* src;
     void* dst;
@@ -596,12 +596,13 @@ int svtad_adapter_prep(const svtad_prep_job* jobs, int count, int dtype, void* s
  *   SVTAD_ROWS_GELU   out0 = z = A W^T + bias; GELU(z) with a sample's first
  *                     n_special rows in out1, the others in out2
  *   SVTAD_ROWS_SPLIT  A W^T in out1 / out2
+ *   SVTAD_ROWS_PLAIN  out0 = A W^T + bias in dtype (A in dtype)
  *   SVTAD_ROWS_RES    out0 = (A W^T + bias) * gamma + res as svtad_adapter_up,
  *                     or A W^T + res (fp32 sum, one rounding) with gamma NULL;
  *                     with a_patch_split A is a0 (special) / a1 (patch rows)
  * Returns SVTAD_ERR_UNSUPPORTED for other widths or type combinations.
  */
-enum svtad_rows_kind { SVTAD_ROWS_GELU = 0, SVTAD_ROWS_SPLIT = 1, SVTAD_ROWS_RES = 2 };
+enum svtad_rows_kind { SVTAD_ROWS_GELU = 0, SVTAD_ROWS_SPLIT = 1, SVTAD_ROWS_RES = 2, SVTAD_ROWS_PLAIN = 3 };
 typedef struct svtad_rows_args {
     const void *a0, *a1, *w, *bias, *gamma, *res;
     void *a_copy, *out0, *out1, *out2;
@@ -637,6 +638,14 @@ size_t svtad_layer_norm_bwd_workspace_bytes(int64_t rows, int c);
 int svtad_layer_norm_bwd(const void* dy, const void* x, const void* add, const float* stats, const void* w,
                          void* dx_special, void* dx, int64_t n_tokens, int64_t n_special, float* dwb, void* workspace, size_t workspace_bytes, int64_t rows, int c, int dtype, int param_f32,
                          void* stream);
+/* The keys' and values' projection kv [batch, nk, 2 a] of the key rows of xa
+ * [batch, n, a], w [2 a, a] and b [2 a] in dtype; and its gradients: the key
+ * rows of dxa (overwritten), dw [2 a, a] and db [2 a] (f32 with out_f32, else
+ * dtype). a = 64 or 128, at most 64 key rows. */
+int svtad_key_proj(const void* xa, const void* w, const void* b, void* kv, int64_t batch, int64_t n, int nk, int a,
+                   int dtype, void* stream);
+int svtad_key_proj_bwd(const void* dkv, const void* xa, const void* w, void* dxa, void* dw, void* db, int64_t batch,
+                       int64_t n, int nk, int a, int dtype, int dw_f32, int db_f32, void* stream);
 int svtad_key_attention_ok(int heads, int head_dim, int64_t n, int nk);
 int svtad_key_attention(const void* q, const void* kv, const void* qn_w, const void* qn_b, const void* kn_w,
                         const void* kn_b, void* out, int64_t batch, int64_t n, int nk, int head_dim, float eps,

@@ -85,6 +85,7 @@ def test_rows_match_float64(dev, embed, hidden, B, N, S, cd, param):
 
 
 @pytest.mark.parametrize("embed,attn,S,heat", [(384, 0, 2, False), (768, 2, 3, False), (384, 2, 1, False), (1024, 2, 5, False),
+                                               (768, 2, 32, False), (384, 2, 32, False), (768, 2, 33, False),
                                                (768, 0, 31, True), (768, 0, 0, False)])
 @pytest.mark.parametrize("amp", [True, False])
 def test_module_gradients_match_float32(dev, embed, attn, S, heat, amp):
