@@ -253,22 +253,23 @@ constexpr int gg_lds_rows(int CR, int FM, int FN, int WS) {
 // from masks of frames up to 19 tokens wide stay within them at any keep rate.
 constexpr int kSpecMargin = 20;
 
-template <int CR, int FM, int FN, int WS>
+template <int CR, int FM, int FN, int WS, int NH = 1>
 struct GgWideLds {
     __align__(16) u16 Ab[gg_lds_rows(CR, FM, FN, WS)][CR];
     int srow[9][FM * 16];  // gathered source row, -1 if missing
     int kvalid[9];
     int klist[10];
     int nk_s, lo_s, hi_s;
-    __align__(16) float bias[CR >= 512 ? 4 * FN * 16 : 4];  // the forward's bias (512 channels)
+    __align__(16) float bias[CR * NH >= 512 ? 4 * FN * 16 : 4];  // the forward's bias (512 channels)
 };
 
 // One tile of the wide gathered GEMM, run by threads [0, 256 * WS) of a
 // workgroup (k_gg_wide, or the backward-input role of k_bwd_fused) in the
-// LDS block L.
-template <typename T, int MODE, int CR, int FM, int FN, int D, int WS>
+// LDS block L. A row has NH * CR values: with NH = 2 the LDS rows hold one half
+// of the reduction at a time, and the accumulators take both halves in turn.
+template <typename T, int MODE, int CR, int FM, int FN, int D, int WS, int NH = 1>
 __device__ __forceinline__ void gg_wide_tile(
-    GgWideLds<CR, FM, FN, WS>& L, int64_t tile, const T* __restrict__ src, const int32_t* __restrict__ nbr,
+    GgWideLds<CR, FM, FN, WS, NH>& L, int64_t tile, const T* __restrict__ src, const int32_t* __restrict__ nbr,
     const T* __restrict__ wb, const void* __restrict__ bias, int bias_mode, T* __restrict__ out, int64_t n,
     int n_out, int64_t tpb, int n_col_tiles, uint32_t* __restrict__ orphan_flag, bool sym) {
     constexpr int BM = FM * 16;
@@ -299,7 +300,8 @@ __device__ __forceinline__ void gg_wide_tile(
     const int lane = tid & 63, wave = ltid >> 6;
     const int64_t row0 = (tile / n_col_tiles) * BM;
     const int col0 = (int)(tile % n_col_tiles) * BN;
-    const rsrc_t rs_src = make_rsrc(src, (uint32_t)(n * CR * 2));
+    constexpr uint32_t ROWB = CR * NH * 2;  // bytes of a source row
+    const rsrc_t rs_src = make_rsrc(src, (uint32_t)(n * ROWB));
 
     constexpr int NT = 256 * WS;
     // The tile's table rows are contiguous (entry e = m*9 + kk). All table
@@ -354,7 +356,7 @@ __device__ __forceinline__ void gg_wide_tile(
         const int r = e / CPR;
         const int64_t gr = spec_lo + r;
         sp[q] = bload16(rs_src, e < SPEC_CHUNKS && gr >= 0 && gr < n
-                                    ? (uint32_t)gr * (uint32_t)(CR * 2) + (uint32_t)(e - r * CPR) * 16u
+                                    ? (uint32_t)gr * ROWB + (uint32_t)(e - r * CPR) * 16u
                                     : kOOB);
     }
     // At 512 channels the forward's bias goes through LDS: one column per
@@ -365,7 +367,7 @@ __device__ __forceinline__ void gg_wide_tile(
     // At 192 channels the LDS form measured 2 us slower per training step
     // (c2 at 55 % keep) with no cause found, so the other widths keep the
     // registers.
-    constexpr bool BIAS_LDS = CR >= 512;
+    constexpr bool BIAS_LDS = CR * NH >= 512;
     const bool has_bias = MODE == MODE_FWD && bias_mode != SVTAD_BIAS_NONE;  // uniform
     const bool bias32 = bias_mode == SVTAD_BIAS_FP32;
     uint32_t bias_raw = 0u;
@@ -456,7 +458,7 @@ __device__ __forceinline__ void gg_wide_tile(
 
     const int nf = (n_out + 15) / 16;
     const uint32_t step_bytes = (uint32_t)nf * 1024u;  // one reduction step, all column blocks
-    const rsrc_t rs_w = make_rsrc(wb, 9u * NC * step_bytes);
+    const rsrc_t rs_w = make_rsrc(wb, 9u * NC * NH * step_bytes);
 
     // Weight fragments (k_pack_frag layout): the 64 lanes of fragment (k,
     // step, column block) are 1 KB contiguous, so a fragment load is fully
@@ -471,9 +473,14 @@ __device__ __forceinline__ void gg_wide_tile(
         const int blk = (col0 + wave * FN * 16) / 16 + f;
         boff[f] = blk < nf ? (uint32_t)(blk * 64 + lane) * 16u : kOOB;
     }
-    auto slab_of = [&](int it) -> uint32_t {
+    // slice it of half h; one past a half's end is the next half's first
+    auto slab_of = [&](int it, int h) -> uint32_t {
+        if (NH > 1 && it >= nk_set && h + 1 < NH) {
+            it = 0;
+            ++h;
+        }
         const int k = it < nk_set ? klist[min(it * WS + set, 9)] : 0;
-        return __builtin_amdgcn_readfirstlane((uint32_t)k * (uint32_t)NC * step_bytes);
+        return __builtin_amdgcn_readfirstlane((uint32_t)(k * NH + h) * (uint32_t)NC * step_bytes);
     };
     u32x4 ring[D][FN];
     auto load_b = [&](uint32_t so, u32x4* rb) {
@@ -556,7 +563,7 @@ __device__ __forceinline__ void gg_wide_tile(
         o1 = r * RP + (sw ^ 32);
     };
 
-    uint32_t slab = slab_of(0);
+    uint32_t slab = slab_of(0, 0);
 #pragma unroll
     for (int d = 0; d < D; ++d) load_b(slab + (uint32_t)d * step_bytes, ring[d]);
 
@@ -565,23 +572,46 @@ __device__ __forceinline__ void gg_wide_tile(
             // rows wlo .. wlo + wrows - 1 into LDS rows 0 .., zeros in row wrows
             for (int e = tid; e < (wrows + 1) * CPR; e += 256 * WS) {
                 const int r = e / CPR, q = e - r * CPR;
-                const u32x4 v = bload16(rs_src, r < wrows ? (uint32_t)(wlo + r) * (uint32_t)(CR * 2) + (uint32_t)q * 16u : kOOB);
+                const u32x4 v = bload16(rs_src, r < wrows ? (uint32_t)(wlo + r) * ROWB + (uint32_t)q * 16u : kOOB);
                 *(u32x4*)&lds[r * RP + ((q ^ (r & 7)) * 8)] = v;
             }
         }
         __syncthreads();
-        // no barrier from here on: the sets walk their slices independently
-        for (int it = 0; it < nk_set; ++it) {
-            const int k = klist[it * WS + set];
-            const uint32_t slab_next = slab_of(it + 1);
-            int off0[FM], off1[FM];
+        for (int h = 0; h < NH; ++h) {
+            if (h > 0) {
+                // the window's rows (the zero row stays) in the next half
+                const int r0 = spec_ok ? lo_t - (int)wlo : 0;
+                const uint32_t base = (uint32_t)lo_t * ROWB + (uint32_t)(h * CR * 2);
+                constexpr int BATCH = 8;
+                u32x4 v[BATCH];
+                for (int e0 = 0; e0 < wrows * CPR; e0 += NT * BATCH) {
 #pragma unroll
-            for (int a = 0; a < FM; ++a) {
-                const int r = srow[k][a * 16 + arow];
-                row_offs(r >= 0 ? (int)(r - wlo) : zrow, off0[a], off1[a]);
+                    for (int q = 0; q < BATCH; ++q) {
+                        const int e = e0 + tid + q * NT, r = e / CPR;
+                        v[q] = bload16(rs_src, r < wrows ? base + (uint32_t)r * ROWB + (uint32_t)(e - r * CPR) * 16u : kOOB);
+                    }
+                    if (e0 == 0) __syncthreads();  // every wave has read the last half
+#pragma unroll
+                    for (int q = 0; q < BATCH; ++q) {
+                        const int e = e0 + tid + q * NT, r = e / CPR, lr = r0 + r;
+                        if (r < wrows) *(u32x4*)&lds[lr * RP + (((e - r * CPR) ^ (lr & 7)) * 8)] = v[q];
+                    }
+                }
+                __syncthreads();
             }
-            compute(off0, off1, slab, slab_next);
-            slab = slab_next;
+            // no barrier within a half: the sets walk their slices independently
+            for (int it = 0; it < nk_set; ++it) {
+                const int k = klist[it * WS + set];
+                const uint32_t slab_next = slab_of(it + 1, h);
+                int off0[FM], off1[FM];
+#pragma unroll
+                for (int a = 0; a < FM; ++a) {
+                    const int r = srow[k][a * 16 + arow];
+                    row_offs(r >= 0 ? (int)(r - wlo) : zrow, off0[a], off1[a]);
+                }
+                compute(off0, off1, slab, slab_next);
+                slab = slab_next;
+            }
         }
     } else {
         // any table: per iteration each set stages its offset's BM gathered
@@ -589,20 +619,22 @@ __device__ __forceinline__ void gg_wide_tile(
         int off0[FM], off1[FM];
 #pragma unroll
         for (int a = 0; a < FM; ++a) row_offs(set * BM + a * 16 + arow, off0[a], off1[a]);
-        for (int it = 0; it < iters; ++it) {
-            const bool live = it < nk_set;
-            const int k = klist[live ? it * WS + set : 0];
-            for (int e = ltid; e < A_CHUNKS; e += 256) {
-                const int m = e / CPR, q = e - m * CPR;
-                const int r = live ? srow[k][m] : -1;
-                const u32x4 v = bload16(rs_src, r >= 0 ? (uint32_t)r * (uint32_t)(CR * 2) + (uint32_t)q * 16u : kOOB);
-                *(u32x4*)&lds[(set * BM + m) * RP + ((q ^ (m & 7)) * 8)] = v;
+        for (int h = 0; h < NH; ++h) {
+            for (int it = 0; it < iters; ++it) {
+                const bool live = it < nk_set;
+                const int k = klist[live ? it * WS + set : 0];
+                for (int e = ltid; e < A_CHUNKS; e += 256) {
+                    const int m = e / CPR, q = e - m * CPR;
+                    const int r = live ? srow[k][m] : -1;
+                    const u32x4 v = bload16(rs_src, r >= 0 ? (uint32_t)r * ROWB + (uint32_t)(h * CR * 2 + q * 16) : kOOB);
+                    *(u32x4*)&lds[(set * BM + m) * RP + ((q ^ (m & 7)) * 8)] = v;
+                }
+                __syncthreads();
+                const uint32_t slab_next = slab_of(it + 1, h);
+                if (live) compute(off0, off1, slab, slab_next);
+                slab = slab_next;
+                __syncthreads();
             }
-            __syncthreads();
-            const uint32_t slab_next = slab_of(it + 1);
-            if (live) compute(off0, off1, slab, slab_next);
-            slab = slab_next;
-            __syncthreads();
         }
     }
     // the bias into LDS for the epilogue (its load arrived long ago)
@@ -696,13 +728,13 @@ __device__ __forceinline__ void gg_wide_tile(
     }
 }
 
-template <typename T, int MODE, int CR, int FM, int FN, int D, int WS>
+template <typename T, int MODE, int CR, int FM, int FN, int D, int WS, int NH>
 __global__ __launch_bounds__(256 * WS) void k_gg_wide(
     const T* __restrict__ src, const int32_t* __restrict__ nbr, const T* __restrict__ wb,
     const void* __restrict__ bias, int bias_mode, T* __restrict__ out, int64_t n, int n_out,
     int64_t tpb, int n_col_tiles, int64_t n_tiles, uint32_t* __restrict__ orphan_flag, bool sym) {
-    __shared__ GgWideLds<CR, FM, FN, WS> lds;
-    gg_wide_tile<T, MODE, CR, FM, FN, D, WS>(lds, xcd_tile(blockIdx.x, n_tiles), src, nbr, wb, bias, bias_mode,
+    __shared__ GgWideLds<CR, FM, FN, WS, NH> lds;
+    gg_wide_tile<T, MODE, CR, FM, FN, D, WS, NH>(lds, xcd_tile(blockIdx.x, n_tiles), src, nbr, wb, bias, bias_mode,
                                              out, n, n_out, tpb, n_col_tiles, orphan_flag, sym);
 }
 
@@ -1623,7 +1655,7 @@ int cu_count() {
     return cached[dev];
 }
 
-template <typename T, int MODE, int CR, int FM, int FN, int D>
+template <typename T, int MODE, int CR, int FM, int FN, int D, int NH = 1>
 static void launch_wide(const void* src, const int32_t* nbr, const void* wb, const void* bias,
                         int bias_mode, void* out, int64_t n, int n_out, int64_t tpb, uint32_t* flag,
                         bool sym, hipStream_t s) {
@@ -1632,12 +1664,12 @@ static void launch_wide(const void* src, const int32_t* nbr, const void* wb, con
     // their LDS fits and the accumulators, weight ring and row fragments
     // leave room for the rest; else one set
     constexpr int WS = (size_t)gg_lds_rows(CR, FM, FN, 2) * CR * 2 <= 150 * 1024 &&
-                               4 * (FM * FN + D * FN + FM + (MODE == MODE_FWD ? FN : 0)) <= 176
+                               4 * (FM * FN + D * FN + FM + (MODE == MODE_FWD && CR * NH < 512 ? FN : 0)) <= 176
                            ? 2
                            : 1;
     const int n_col = (int)cdiv(n_out, BN);
     const int64_t tiles = cdiv(n, 16 * FM) * n_col;
-    hipLaunchKernelGGL((k_gg_wide<T, MODE, CR, FM, FN, D, WS>), dim3((unsigned)tiles), dim3(256 * WS),
+    hipLaunchKernelGGL((k_gg_wide<T, MODE, CR, FM, FN, D, WS, NH>), dim3((unsigned)tiles), dim3(256 * WS),
                        0, s, (const T*)src, nbr, (const T*)wb, bias, bias_mode, (T*)out, n, n_out,
                        tpb, n_col, tiles, flag, sym);
 }
@@ -1706,6 +1738,36 @@ static void launch_wide_fm(const void* src, const int32_t* nbr, const void* wb, 
         }
     } else {
         static const int have[] = {2, 4};
+        if constexpr (CR == 512) {
+            // A tile of 16 FM rows streams the weight of its 256 columns (2.4
+            // MB, about 28 us at the rate a CU reads its XCD's L2), and whole
+            // 512-value rows leave LDS for FM = 4 at most. With half rows FM
+            // reaches 7. A round of workgroups takes about 14 + 5 FM us in
+            // either form (FM 4, 5, 6, 7: 33, 38, 44, 49 us), so the line lies
+            // at the least rounds x (14 + 5 FM): 13106 rows two rounds at FM 4
+            // 67.4 us, one at FM 7 50.6; 9832 rows 65.5 -> 39.6 (FM 5); 19664
+            // rows 96.5 -> 74.9 (FM 5); 22940 rows 103.3 -> 87.9 (FM 6); 4096
+            // rows 27.7 at FM 2, 33 at FM 5.
+            static const int all[] = {2, 4, 5, 6, 7};
+            int fm = 2;
+            int64_t best = INT64_MAX;
+            for (int f : all) {
+                const int64_t t = cdiv(cdiv(n, 16 * f) * n_col, cu_count()) * (14 + 5 * f);
+                if (t < best) best = t, fm = f;
+            }
+#define SVTAD_HALVES(F)                                                                                                       \
+    if (fm == F) {                                                                                                            \
+        launch_wide<T, MODE, 256, F, FN, 2, 2>(src, nbr, wb, bias, bias_mode, out, n, n_out, tpb, flag, sym, s);              \
+        return;                                                                                                               \
+    }
+            SVTAD_HALVES(5)
+            SVTAD_HALVES(6)
+            SVTAD_HALVES(7)
+#undef SVTAD_HALVES
+            if (fm == 2) launch_wide<T, MODE, CR, 2, FN, D>(src, nbr, wb, bias, bias_mode, out, n, n_out, tpb, flag, sym, s);
+            else launch_wide<T, MODE, CR, 4, FN, D>(src, nbr, wb, bias, bias_mode, out, n, n_out, tpb, flag, sym, s);
+            return;
+        }
         if (pick_fm(n, n_col, have, 2) == 2)
             launch_wide<T, MODE, CR, 2, FN, D>(src, nbr, wb, bias, bias_mode, out, n, n_out, tpb, flag, sym, s);
         else
