@@ -466,6 +466,14 @@ class KeyTokenAttentionFunction(Function):
         return (*(_cast(t, dt) for t, dt in zip(grads, ctx.dtypes)), None, None, None)
 
 
+def _is_plain(m, cls):
+    """Whether calling ``m`` computes ``cls.forward`` on its parameters and
+    nothing else: no subclass, no replaced ``forward``, no hook (weight_norm and
+    spectral_norm set the weight in one)."""
+    return type(m) is cls and "forward" not in m.__dict__ and not (
+        m._forward_pre_hooks or m._forward_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+
 def _trunc_normal_init(layer, std):
     """mmengine's trunc_normal_init(layer, std=std, bias=0) as the reference calls
     it: weight ~ N(0, std) truncated to [-2, 2], bias 0."""
@@ -596,7 +604,7 @@ class SparseConvAdapter(nn.Module):
                 nbr = nbr.to(torch.int32)
             nbr = _keep_symmetric(neighbor_indices, nbr)
         conv = self.sparse_conv
-        key_attn = self.use_attn == 2 and self._key_attention_ok(N)
+        key_attn = self.use_attn == 2 and self._key_attention_ok(B, N)
         if not self.use_attn or key_attn:
             hm_rows = hm_gate = None
             if self._uses_heatmap():
@@ -624,7 +632,7 @@ class SparseConvAdapter(nn.Module):
                                                  hm_gate, packed, keep_packed, (S, tokens_per_batch, cd, nk, *eps), *attn)
         if not self.use_attn:
             if cache is not None:
-                packed = cache.get(conv.weight, _cast(conv.weight, cd), torch.is_grad_enabled())
+                packed = cache.get(conv.weight, _cast(conv.weight, cd), grad)
             return SparseConvAdapterFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight,
                                                    conv.bias, self.up_proj.weight, self.up_proj.bias, self.gamma,
                                                    nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd)
@@ -642,11 +650,18 @@ class SparseConvAdapter(nn.Module):
                 self.qkv.bias, self.q_norm.weight, self.q_norm.bias, self.k_norm.weight, self.k_norm.bias,
                 self.attn_proj.weight, self.attn_proj.bias, self.attn_gamma)
 
-    def _key_attention_ok(self, n_tokens):
+    def _key_attention_ok(self, batch, n_tokens):
         """Whether ``KeyTokenAttentionFunction`` takes this module: its widths
         and key count, norms with weight and bias and one eps, biased Linear
-        layers, one parameter type for the norms of a kernel."""
+        layers, one parameter type for the norms of a kernel, and layers that a
+        call runs as they are; the kernels' grids take 1 to 65535 samples."""
+        if not 1 <= batch <= 65535:
+            return False
         norms = (self.attn_norm, self.q_norm, self.k_norm)
+        if not all(_is_plain(m, nn.LayerNorm) for m in norms):
+            return False
+        if not (_is_plain(self.down_attn, nn.Linear) and _is_plain(self.qkv, nn.Linear)):
+            return False
         if any(m.weight is None or m.bias is None or m.weight.dtype != m.bias.dtype for m in norms):
             return False
         if self.q_norm.eps != self.k_norm.eps or self.q_norm.weight.dtype != self.k_norm.weight.dtype:
@@ -693,7 +708,7 @@ class SparseConvAdapter(nn.Module):
             fr_out = coarse[:, S:]
             pa_out = torch.gather(fr_out.float(), 1, idx).to(fr_out.dtype) if fused else torch.gather(fr_out, 1, idx)
             return shortcut + torch.cat([sp_out, pa_out], dim=1)
-        if fused and self.use_attn == 2 and self._key_attention_ok(N):
+        if fused and self.use_attn == 2 and self._key_attention_ok(B, N):
             xa = KeyTokenAttentionFunction.apply(
                 x_comb, self.attn_norm.weight, self.attn_norm.bias, self.down_attn.weight, self.down_attn.bias,
                 self.qkv.weight, self.qkv.bias, self.q_norm.weight, self.q_norm.bias, self.k_norm.weight,
