@@ -632,7 +632,7 @@ class SparseConvAdapter(nn.Module):
                                                  hm_gate, packed, keep_packed, (S, tokens_per_batch, cd, nk, *eps), *attn)
         if not self.use_attn:
             if cache is not None:
-                packed = cache.get(conv.weight, _cast(conv.weight, cd), grad)
+                packed = cache.get(conv.weight, _cast(conv.weight, cd), torch.is_grad_enabled())
             return SparseConvAdapterFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight,
                                                    conv.bias, self.up_proj.weight, self.up_proj.bias, self.gamma,
                                                    nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd)
