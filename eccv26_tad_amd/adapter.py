@@ -430,7 +430,9 @@ class KeyTokenAttentionFunction(Function):
     rows) in ``cd``. Queries are projected for all rows and keys and values for
     the key tokens only (the reference projects all three for every token and
     leaves the rest unused). The norms, scores, softmax and weighted sum are
-    evaluated in float32 on the Linear outputs; the Linear layers' weight and
+    evaluated in float32 on the Linear outputs, rounded to ``cd`` where the
+    reference's chain rounds (normalised queries and keys; with float32
+    parameters the scores and probabilities too); the Linear layers' weight and
     bias gradients run on the split-row kernels."""
 
     @staticmethod

@@ -203,6 +203,10 @@ __global__ __launch_bounds__(256) void k_key_attn(KeyAttnArgs p) {
         rstd = rsqrtf(lane_sum<HD>(d * d) * (1.f / HD) + p.eps);
         xh = d * rstd;
     };
+    // The reference's roundings: queries and keys enter the score product in
+    // T; with float32 parameters (autocast) the scores, their scaling and the
+    // probabilities of the weighted sum are rounded to T as well.
+    auto round_amp = [&](float v) { return p.p32 ? (float)(T)v : v; };
     const float qw = load_param<T>(p.qn_w, j, p.p32), qb = load_param<T>(p.qn_b, j, p.p32);
     const float kw = load_param<T>(p.kn_w, j, p.p32), kb = load_param<T>(p.kn_b, j, p.p32);
     float kh[NKT], vv[NKT];
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(256) void k_key_attn(KeyAttnArgs p) {
         if (t < p.nk) {  // uniform
             float xh, rstd;
             norm((float)kv[t * 2 * A + c], xh, rstd);
-            kh[t] = (xh * kw + kb) * p.scale;
+            kh[t] = (float)(T)(xh * kw + kb);
             vv[t] = (float)kv[t * 2 * A + A + c];
         }
     }
@@ -227,11 +231,11 @@ __global__ __launch_bounds__(256) void k_key_attn(KeyAttnArgs p) {
         }
         float xh, rstd;
         norm((float)q[r * A + c], xh, rstd);
-        const float qh = xh * qw + qb;
-        float s[NKT], mx = -__builtin_huge_valf();
+        const float qh = (float)(T)(xh * qw + qb);
+        float s[NKT], pr[NKT], mx = -__builtin_huge_valf();
 #pragma unroll
         for (int t = 0; t < NKT; ++t) {
-            s[t] = t < p.nk ? lane_sum<HD>(qh * kh[t]) : -__builtin_huge_valf();
+            s[t] = t < p.nk ? round_amp(round_amp(lane_sum<HD>(qh * kh[t])) * p.scale) : -__builtin_huge_valf();
             mx = fmaxf(mx, s[t]);
         }
         float z = 0.f;
@@ -242,11 +246,14 @@ __global__ __launch_bounds__(256) void k_key_attn(KeyAttnArgs p) {
         }
         const float iz = 1.f / z;
 #pragma unroll
-        for (int t = 0; t < NKT; ++t) s[t] *= iz;
+        for (int t = 0; t < NKT; ++t) {
+            s[t] *= iz;
+            pr[t] = round_amp(s[t]);
+        }
         if constexpr (!BWD) {
             float o = 0.f;
 #pragma unroll
-            for (int t = 0; t < NKT; ++t) o += s[t] * vv[t];
+            for (int t = 0; t < NKT; ++t) o += pr[t] * vv[t];
             out[r * A + c] = (T)o;
         } else {
             const float d = (float)((const T*)p.dout + b * p.n * A)[r * A + c];
@@ -255,14 +262,14 @@ __global__ __launch_bounds__(256) void k_key_attn(KeyAttnArgs p) {
             for (int t = 0; t < NKT; ++t) {
                 dp[t] = t < p.nk ? lane_sum<HD>(d * vv[t]) : 0.f;
                 dot += s[t] * dp[t];
-                dv[t] += s[t] * d;
+                dv[t] += pr[t] * d;
             }
             float g = 0.f;  // gradient of the normalised query
 #pragma unroll
             for (int t = 0; t < NKT; ++t) {
-                const float ds = s[t] * (dp[t] - dot);
-                g += ds * kh[t];   // the scale is in kh
-                dk[t] += ds * qh;  // times the scale later
+                const float ds = s[t] * (dp[t] - dot) * p.scale;
+                g += ds * kh[t];
+                dk[t] += ds * qh;
             }
             dqw += g * xh;
             dqb += g;
@@ -274,7 +281,7 @@ __global__ __launch_bounds__(256) void k_key_attn(KeyAttnArgs p) {
     if constexpr (BWD) {
 #pragma unroll
         for (int t = 0; t < NKT; ++t) {
-            red[wave][t][lane] = dk[t] * p.scale;
+            red[wave][t][lane] = dk[t];
             red[wave][NKT + t][lane] = dv[t];
         }
         red[wave][2 * NKT][lane] = dqw;

@@ -59,7 +59,12 @@ def test_key_attention(dev, hd, B, N, nk, cd, param):
     Q, KV, *PD = (t.double().requires_grad_(True) for t in (q, kv, *P))
     qn = F.layer_norm(Q[:, nk:].view(B, -1, 4, hd), (hd,), PD[0], PD[1], 1e-5)
     kn = F.layer_norm(KV[:, :, :a].view(B, nk, 4, hd), (hd,), PD[2], PD[3], 1e-5)
-    p = torch.softmax((qn.unsqueeze(2) * kn.unsqueeze(1)).sum(-1) / hd ** 0.5, 2)
+    # the kernels' roundings to T, passed over by the gradient: queries and keys,
+    # and with float32 parameters the scores, their scaling and the probabilities
+    to_t = lambda v: v + (v.detach().to(T).double() - v.detach())  # noqa: E731
+    amp = to_t if PT != T else lambda v: v
+    qn, kn = to_t(qn), to_t(kn)
+    p = amp(torch.softmax(amp(amp((qn.unsqueeze(2) * kn.unsqueeze(1)).sum(-1)) / hd ** 0.5), 2))
     att = (p.unsqueeze(-1) * KV[:, None, :, a:].view(B, 1, nk, 4, hd)).sum(2).reshape(B, N - nk, a)
     OUT = torch.cat([torch.zeros(B, nk, a, dtype=torch.float64, device=dev), att], 1)
     gq, gkv, *gp = torch.autograd.grad(OUT, (Q, KV, *PD), dout.double())
@@ -69,7 +74,9 @@ def test_key_attention(dev, hd, B, N, nk, cd, param):
     if nk > 1:
         assert _rel(dq, gq) <= 2 * ULP[T] and _rel(dkv, gkv) <= 2 * ULP[T]
         for k in (0, 1, 2):
-            assert _rel(dn[k], gp[k]) <= 1e-4, k
+            # a float32 value beside the middle of two values of T rounds the other way: 1 ulp in a few of
+            # the values that a sum over all rows of a head's channel takes
+            assert _rel(dn[k], gp[k]) <= 1e-4 + ULP[T] / 8, k
     else:
         assert _rel(dkv[:, :, a:], gkv[:, :, a:]) <= 2 * ULP[T]
         assert float(dq.double().abs().max()) <= 1e-5 and float(dn[:3].abs().max()) <= 1e-3
