@@ -369,6 +369,9 @@ class SparseConvAdapterFunction(Function):
 
 
 _ATTN_PARAMS = 13  # tensors of SparseConvAdapter._attention_parameters
+_ATTN_WEIGHTS = (2, 4, 10)  # their Linear weights: the backward reads the type alone (a copy in cd is saved)
+_ATTN_BIASES = (3, 5, 11)
+_NO_VALUES = {t: torch.empty(0, dtype=t) for t in (torch.float16, torch.bfloat16, torch.float32)}
 
 
 class AdapterRowsFunction(Function):
@@ -400,7 +403,12 @@ class AdapterRowsFunction(Function):
         if pack and keep_packed is not None:
             keep_packed(pf, pb if train else None)
         if train:
-            ctx.save_for_backward(gamma, nbr, hm_rows, hm_gate, *saved, *attn)
+            # a parameter that is read in its own type must not change before
+            # the backward; one that was cast may
+            attn = [_NO_VALUES[t.dtype] if i in _ATTN_BIASES or (i in _ATTN_WEIGHTS and t.dtype != cd) else t
+                    for i, t in enumerate(attn)]
+            own = [t if t is not None and t.dtype == cd else None for t in (w_d, b_c)]
+            ctx.save_for_backward(*own, gamma, nbr, hm_rows, hm_gate, *saved, *attn)
             ctx.meta = (meta, is_symmetric_table(nbr), b_d is not None, b_c is not None, b_u is not None, x.dtype,
                         [t is not None and t.dtype == torch.float32 for t in (w_d, b_d, w_c, b_c, w_u, b_u)])
         return out
@@ -408,7 +416,7 @@ class AdapterRowsFunction(Function):
     @staticmethod
     def backward(ctx, go):
         (S, tpb, cd, nk, _, eps1), symmetric, has_bd, has_bc, has_bu, x_dt, f32 = ctx.meta
-        gamma, nbr, hm_rows, hm_gate, *saved = ctx.saved_tensors
+        _, _, gamma, nbr, hm_rows, hm_gate, *saved = ctx.saved_tensors
         need = ctx.needs_input_grad
         attn = []
         if len(need) > 14:

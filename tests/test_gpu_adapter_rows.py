@@ -132,3 +132,36 @@ def test_module_gradients_match_float32(dev, embed, attn, S, heat, amp):
         # a scalar gain's gradient against its sum of absolute terms
         bar = tol * scales[name] * 0.2 if name in scales else tol * float(want.norm())
         assert err <= bar, (name, err, bar)
+
+
+@pytest.mark.parametrize("amp", [True, False])
+@pytest.mark.parametrize("name", ["down_proj.weight", "sparse_conv.bias", "up_proj.weight", "down_attn.weight", "qkv.weight"])
+def test_parameter_changed_before_backward(dev, amp, name):
+    """A parameter changed in place between the two passes is refused when its
+    own values were saved and has no effect when it had been cast."""
+    import eccv26_tad_amd as sv
+
+    g = torch.Generator(device=dev).manual_seed(5)
+    dt = torch.float32 if amp else torch.float16
+    mod = sv.SparseConvAdapter(384, 0.25, use_attn=2, n_key_tokens=2).to(dev, dt)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.add_(0.1 * torch.randn(p.shape, generator=g, device=dev))
+    idx = torch.arange(40, device=dev).expand(1, -1)
+    table = sv.build_neighbor_table(torch.ones(1, 2, 4, 5, dtype=torch.uint8, device=dev), batched=True, n=40)
+    x = torch.randn(1, 42, 384, generator=g, device=dev).to(dt).requires_grad_(True)
+
+    def gradient(change):
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            y = mod(x, 4, 5, idx, 40, table)
+        if change:
+            with torch.no_grad():
+                mod.get_parameter(name).add_(0.25)
+        return torch.autograd.grad(y, x, torch.ones_like(y))[0]
+
+    if amp:
+        want = gradient(False)
+        assert torch.equal(gradient(True), want)
+    else:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            gradient(True)
