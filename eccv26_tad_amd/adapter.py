@@ -479,9 +479,10 @@ class KeyTokenAttentionFunction(Function):
 def _is_plain(m, cls):
     """Whether calling ``m`` computes ``cls.forward`` on its parameters and
     nothing else: no subclass, no replaced ``forward``, no hook (weight_norm and
-    spectral_norm set the weight in one)."""
+    spectral_norm set the weight in one), no hook on all modules."""
     return type(m) is cls and "forward" not in m.__dict__ and not (
-        m._forward_pre_hooks or m._forward_hooks or m._backward_hooks or m._backward_pre_hooks)
+        m._forward_pre_hooks or m._forward_hooks or m._backward_hooks or m._backward_pre_hooks
+        or nn.modules.module._has_any_global_hook())
 
 
 def _trunc_normal_init(layer, std):

@@ -48,3 +48,13 @@ def test_changed_layers_are_called(change):
     m = _module()
     CHANGES[change](m)
     assert not m._key_attention_ok(2, 4)
+
+
+def test_hook_on_all_modules():
+    m = _module()
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    try:
+        assert not m._key_attention_ok(2, 4)
+    finally:
+        handle.remove()
+    assert m._key_attention_ok(2, 4)
