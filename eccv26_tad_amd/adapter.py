@@ -615,7 +615,8 @@ class SparseConvAdapter(nn.Module):
                 nbr = nbr.to(torch.int32)
             nbr = _keep_symmetric(neighbor_indices, nbr)
         conv = self.sparse_conv
-        key_attn = self.use_attn == 2 and self._key_attention_ok(B, N)
+        # with attention sparse_conv is called, unless a call would only read its parameters
+        key_attn = self.use_attn == 2 and _is_plain(conv, SparseConv2d) and self._key_attention_ok(B, N)
         if not self.use_attn or key_attn:
             hm_rows = hm_gate = None
             if self._uses_heatmap():

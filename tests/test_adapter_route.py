@@ -4,6 +4,9 @@ from __future__ import annotations
 
 import pytest
 import torch
+import torch.nn.utils.prune
+
+import eccv26_tad_amd as sv
 
 
 def _module():
@@ -58,3 +61,55 @@ def test_hook_on_all_modules():
     finally:
         handle.remove()
     assert m._key_attention_ok(2, 4)
+
+
+class _Route(Exception):
+    pass
+
+
+def _route(m, monkeypatch):
+    """Which route a 16-bit call takes: "one node", or "layers" when the
+    modules' calls (sparse_conv among them) run."""
+    from eccv26_tad_amd import adapter
+
+    def take(name):
+        def apply(*args):
+            raise _Route(name)
+        return apply
+
+    monkeypatch.setattr(adapter.SparseConvAdapter, "_fused_dtype", lambda self, x: torch.bfloat16)
+    monkeypatch.setattr(adapter.AdapterRowsFunction, "apply", take("one node"))
+    monkeypatch.setattr(adapter.AdapterDownFunction, "apply", take("layers"))
+    with pytest.raises(_Route) as route:
+        m(torch.zeros(2, 8, 768), 1, 5, torch.arange(5).expand(2, -1), 5, torch.full((2, 5, 9), -1, dtype=torch.int32))
+    return str(route.value)
+
+
+class _ScaledConv(sv.SparseConv2d):
+    def forward(self, *args, **kwargs):
+        return 2 * super().forward(*args, **kwargs)
+
+
+class _Wrapped(torch.nn.Module):
+    def __init__(self, conv):
+        super().__init__()
+        self.conv = conv
+
+
+CONV_CHANGES = {
+    "wrapped": lambda m: setattr(m, "sparse_conv", _Wrapped(m.sparse_conv)),
+    "spectral_norm": lambda m: torch.nn.utils.spectral_norm(m.sparse_conv),
+    "weight_norm": lambda m: torch.nn.utils.parametrizations.weight_norm(m.sparse_conv),
+    "pruned": lambda m: torch.nn.utils.prune.l1_unstructured(m.sparse_conv, "weight", 0.5),
+    "forward_hook": lambda m: m.sparse_conv.register_forward_hook(lambda *a: None),
+    "backward_hook": lambda m: m.sparse_conv.register_full_backward_hook(lambda *a: None),
+    "forward": lambda m: setattr(m.sparse_conv, "forward", lambda *a, **k: None),
+    "subclass": lambda m: setattr(m, "sparse_conv", _ScaledConv(256, 256)),
+}
+
+
+@pytest.mark.parametrize("change", ["plain"] + sorted(CONV_CHANGES))
+def test_changed_sparse_conv_is_called(change, monkeypatch):
+    m = _module()
+    CONV_CHANGES.get(change, lambda m: None)(m)
+    assert _route(m, monkeypatch) == ("one node" if change == "plain" else "layers")
