@@ -269,11 +269,13 @@ class SparseConvAdapterFunction(Function):
     then autograd adds ``go`` in a separate pass over the 768-wide tokens.
     The kernels are those of ``AdapterDownFunction``, ``SparseConv2dFunction``
     and ``AdapterUpFunction``; ``packed`` is the SparseConv2D weight's
-    ``(packed_fwd, packed_bwd)`` as ``SparseConv2dFunction`` takes it."""
+    ``(packed_fwd, packed_bwd)`` as ``SparseConv2dFunction`` takes it;
+    ``grad_mode`` is the caller's (``needs_input_grad`` is set by parameters
+    that require a gradient under ``no_grad`` too)."""
 
     @staticmethod
     def forward(ctx, x, w_d, b_d, w_c, b_c, w_u, b_u, gamma, nbr, n_special, tpb, hm_rows=None, hm_gate=None,
-                packed=None, cd=None):
+                packed=None, cd=None, grad_mode=True):
         S = int(n_special)
         ctx.symmetric = is_symmetric_table(nbr)
         cd = x.dtype if cd is None else cd
@@ -281,7 +283,7 @@ class SparseConvAdapterFunction(Function):
         # the heatmap gate keep their dtype, as in the reference chain
         params = (w_d, b_d, w_c, b_c, w_u, b_u, gamma, hm_gate)
         ctx.dtypes = tuple(None if t is None else t.dtype for t in (x,) + params)
-        need_bwd = any(ctx.needs_input_grad)
+        need_bwd = grad_mode and any(ctx.needs_input_grad)
         c_in = w_c.shape[1]
         if c_in % 4 != 0:
             raise ValueError(f"C_in ({c_in}) must be divisible by 4 for optimized kernel.")
@@ -365,7 +367,7 @@ class SparseConvAdapterFunction(Function):
         gb_d = _colsum(du2).to(bd_dt) if has_bd and need[2] else None
         return (gx, gw_d, gb_d, gw_c.to(wc_dt) if need[3] else None,
                 gb_c.to(bc_dt) if need_bc else None, _cast(gw_u, wu_dt), _cast(gb_u, bu_dt), g_gamma,
-                None, None, None, None, g_gate, None, None)
+                None, None, None, None, g_gate, None, None, None)
 
 
 _ATTN_PARAMS = 13  # tensors of SparseConvAdapter._attention_parameters
@@ -388,14 +390,16 @@ class AdapterRowsFunction(Function):
 
     ``attn`` are the attention's 13 parameters, or nothing; ``meta`` is
     ``(n_special, tokens_per_batch, cd, nk, eps of the row norm, eps of the
-    head norms)``."""
+    head norms, grad mode)``. Without the grad mode the forward lays out, copies
+    and keeps nothing for a backward: embed 768 at 17250 rows under autocast
+    94.5 -> 85.7 us, embed 384 in bfloat16 at 8184 rows 48.3 -> 39.8 us."""
 
     @staticmethod
     def forward(ctx, x, w_d, b_d, w_c, b_c, w_u, b_u, gamma, nbr, hm_rows, hm_gate, packed, keep_packed, meta, *attn):
-        S, tpb, cd, nk, eps0, eps1 = meta
+        S, tpb, cd, nk, eps0, eps1, grad_mode = meta
         c_in = w_c.shape[1]
         mode = BIAS_NONE if b_c is None else (BIAS_FP32 if c_in >= IMPLICIT_GEMM_MIN_CIN else BIAS_AFTER)
-        train = any(ctx.needs_input_grad)
+        train = grad_mode and any(ctx.needs_input_grad)
         pack = packed is None or (train and packed[1] is None)
         out, pf, pb, *saved = _ops.adapter_forward(
             x, w_d, b_d, w_c, b_c, w_u, b_u, gamma, nbr, S, tpb, mode, hm_rows, hm_gate, None if pack else packed[0],
@@ -415,7 +419,7 @@ class AdapterRowsFunction(Function):
 
     @staticmethod
     def backward(ctx, go):
-        (S, tpb, cd, nk, _, eps1), symmetric, has_bd, has_bc, has_bu, x_dt, f32 = ctx.meta
+        (S, tpb, cd, nk, _, eps1, _), symmetric, has_bd, has_bc, has_bu, x_dt, f32 = ctx.meta
         _, _, gamma, nbr, hm_rows, hm_gate, *saved = ctx.saved_tensors
         need = ctx.needs_input_grad
         attn = []
@@ -629,11 +633,12 @@ class SparseConvAdapter(nn.Module):
                 hm_gate = self.heatmap_gate
             cache = conv.packed_weight_cache
             packed = None
+            grad_mode = torch.is_grad_enabled()
             if _ops.adapter_rows_ok(self.embed_dims, self.hidden_dims):
                 keep_packed = None
                 if cache is not None:
                     # packed with the other parameters' preparation when not current
-                    packed = cache.peek(conv.weight, cd, torch.is_grad_enabled())
+                    packed = cache.peek(conv.weight, cd, grad_mode)
                     keep_packed = functools.partial(cache.put, conv.weight, cd)
                 attn, nk, eps = (), 0, (0.0, 0.0)
                 if key_attn:
@@ -641,13 +646,14 @@ class SparseConvAdapter(nn.Module):
                     eps = (self.attn_norm.eps, self.q_norm.eps)
                 return AdapterRowsFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight, conv.bias,
                                                  self.up_proj.weight, self.up_proj.bias, self.gamma, nbr, hm_rows,
-                                                 hm_gate, packed, keep_packed, (S, tokens_per_batch, cd, nk, *eps), *attn)
+                                                 hm_gate, packed, keep_packed,
+                                                 (S, tokens_per_batch, cd, nk, *eps, grad_mode), *attn)
         if not self.use_attn:
             if cache is not None:
-                packed = cache.get(conv.weight, _cast(conv.weight, cd), torch.is_grad_enabled())
+                packed = cache.get(conv.weight, _cast(conv.weight, cd), grad_mode)
             return SparseConvAdapterFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight,
                                                    conv.bias, self.up_proj.weight, self.up_proj.bias, self.gamma,
-                                                   nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd)
+                                                   nbr, S, tokens_per_batch, hm_rows, hm_gate, packed, cd, grad_mode)
         sp, pa = AdapterDownFunction.apply(x, self.down_proj.weight, self.down_proj.bias, S, cd)
         processed = conv(pa, nbr, tokens_per_batch=tokens_per_batch)
         x_comb = torch.cat([sp, processed.view(B, N - S, -1)], dim=1)

@@ -113,3 +113,25 @@ def test_changed_sparse_conv_is_called(change, monkeypatch):
     m = _module()
     CONV_CHANGES.get(change, lambda m: None)(m)
     assert _route(m, monkeypatch) == ("one node" if change == "plain" else "layers")
+
+
+@pytest.mark.parametrize("mode", ["no_grad", "inference_mode", "frozen", "grad"])
+@pytest.mark.parametrize("attn", [0, 2])
+def test_inference_prepares_no_backward(mode, attn, monkeypatch):
+    """Parameters require gradients when a model is served under no_grad too."""
+    from eccv26_tad_amd import adapter
+
+    seen = []
+
+    def forward(x, *args):
+        seen.append(args[16])
+        return x.clone(), x.new_empty(0), x.new_empty(0), *[x.new_empty(0)] * (25 if attn else 10)
+
+    m = sv.SparseConvAdapter(768, 0.25, use_attn=attn, n_key_tokens=3)
+    m.sparse_conv.packed_weight_cache = None  # keyed by the stream of a GPU
+    m.requires_grad_(mode != "frozen")
+    monkeypatch.setattr(adapter.SparseConvAdapter, "_fused_dtype", lambda self, x: torch.bfloat16)
+    monkeypatch.setattr(adapter._ops, "adapter_forward", forward)
+    with {"no_grad": torch.no_grad, "inference_mode": torch.inference_mode}.get(mode, torch.enable_grad)():
+        y = m(torch.zeros(2, 8, 768), 1, 5, torch.arange(5).expand(2, -1), 5, torch.full((2, 5, 9), -1, dtype=torch.int32))
+    assert seen == [mode == "grad"] and y.requires_grad == (mode == "grad")

@@ -165,3 +165,33 @@ def test_parameter_changed_before_backward(dev, amp, name):
     else:
         with pytest.raises(RuntimeError, match="modified by an inplace operation"):
             gradient(True)
+
+
+@pytest.mark.parametrize("embed,attn", [(384, 0), (768, 2), (512, 0)])
+@pytest.mark.parametrize("amp", [True, False])
+def test_no_grad_matches_grad_mode(dev, embed, attn, amp):
+    """A forward without gradients gives the same bits, and packs and keeps the
+    forward's layout of the convolution only."""
+    import eccv26_tad_amd as sv
+
+    g = torch.Generator(device=dev).manual_seed(embed)
+    mod = sv.SparseConvAdapter(embed, 0.25, use_attn=attn, n_key_tokens=2).to(dev, torch.float32 if amp else torch.float16)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.add_(0.05 * torch.randn(p.shape, generator=g, device=dev))
+    idx = torch.arange(40, device=dev).expand(2, -1)
+    table = sv.build_neighbor_table(torch.ones(2, 2, 4, 5, dtype=torch.uint8, device=dev), batched=True, n=80)
+    x = torch.randn(2, 42, embed, generator=g, device=dev).to(mod.gamma.dtype)
+    cache = mod.sparse_conv.packed_weight_cache
+
+    def call(mode):
+        with mode(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            return mod(x, 4, 5, idx, 40, table).detach()
+
+    cold = call(torch.no_grad)
+    kept = cache._packed
+    assert kept[1] is None
+    assert torch.equal(call(torch.no_grad), cold) and cache._packed is kept
+    assert torch.equal(call(torch.enable_grad), cold) and cache._packed[1] is not None
+    kept = cache._packed
+    assert torch.equal(call(torch.no_grad), cold) and cache._packed is kept
