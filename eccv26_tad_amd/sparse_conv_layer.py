@@ -68,11 +68,13 @@ class PackedWeightCache:
         None (the caller packs) off the GPU or for an inference tensor."""
         if not weight.is_cuda or param.is_inference():
             return None
-        packed = self.peek(param, weight.dtype, need_bwd)
-        if packed is None:
-            pf, pb = _ops.pack_weight(weight.detach(), True, need_bwd)
-            packed = self.put(param, weight.dtype, pf, pb if need_bwd else None)
-        return packed
+        stream = torch.cuda.current_stream(weight.device).cuda_stream
+        key = (param.data_ptr(), param._version, weight.dtype, weight.device, stream)
+        if param is self._param and key == self._key and (self._packed[1] is not None or not need_bwd):
+            return self._packed
+        pf, pb = _ops.pack_weight(weight.detach(), True, need_bwd)
+        self._param, self._key, self._packed = param, key, (pf, pb if need_bwd else None)
+        return self._packed
 
     @staticmethod
     def _key_of(param, dtype):
@@ -82,7 +84,7 @@ class PackedWeightCache:
     def peek(self, param, dtype, need_bwd):
         """The kept layouts of ``param`` in ``dtype`` when they are current,
         else None (nothing is packed)."""
-        if not param.is_cuda or param.is_inference() or param is not self._param:
+        if param is not self._param or not param.is_cuda or param.is_inference():
             return None
         if self._key != self._key_of(param, dtype) or (need_bwd and self._packed[1] is None):
             return None
@@ -91,10 +93,8 @@ class PackedWeightCache:
     def put(self, param, dtype, packed_fwd, packed_bwd):
         """Keep layouts of ``param`` in ``dtype`` that the caller packed on the
         current stream (``packed_bwd`` None when it has none)."""
-        packed = (packed_fwd, packed_bwd)
         if not param.is_inference():
-            self._param, self._key, self._packed = param, self._key_of(param, dtype), packed
-        return packed
+            self._param, self._key, self._packed = param, self._key_of(param, dtype), (packed_fwd, packed_bwd)
 
 
 class SparseConv2dFunction(Function):
