@@ -143,44 +143,8 @@ def _up_wgrad(go, B, N, S, a_sp, a_pa):
     if S == 0:
         return _wgrad(go2, _NO_ROWS(go2), a_pa, True)
     k = a_pa.shape[-1]
-    G = _wgrad(go2, _patch_rows(B, N, S, go.device), a_pa, True)
+    G = _wgrad(go2, _ops.patch_rows(go2, B, N, S), a_pa, True)
     return G.add_(torch.matmul(go[:, :S].reshape(-1, n).t().float(), a_sp.reshape(-1, k).float()))
-
-
-_PATCH_ROWS = {}
-_TOKEN_ROWS = {}
-
-
-def _token_rows(B, N, S, device):
-    """Row of ``go.reshape(B * N, -1)`` for the special tokens of every sample,
-    then for the patch tokens in the order of the SparseConv2D rows, cached
-    per shape and device (bounded)."""
-    key = (B, N, S, device)
-    rows = _TOKEN_ROWS.get(key)
-    if rows is None:
-        r = torch.arange(B * S, device=device, dtype=torch.int32)
-        special = (r // max(S, 1)) * N + r % max(S, 1)
-        rows = torch.cat([special, _patch_rows(B, N, S, device)])
-        if len(_TOKEN_ROWS) >= 64:
-            _TOKEN_ROWS.clear()
-        _TOKEN_ROWS[key] = rows
-    return rows
-
-
-def _patch_rows(B, N, S, device):
-    """Row of ``go.reshape(B * N, -1)`` for each patch token in the order of
-    the SparseConv2D rows (``b * N + S + r``), cached per shape and device:
-    built on every backward it costs five small integer kernels."""
-    key = (B, N, S, device)
-    rows = _PATCH_ROWS.get(key)
-    if rows is None:
-        P = N - S
-        r = torch.arange(B * P, device=device, dtype=torch.int32)
-        rows = (r // P) * N + S + r % P
-        if len(_PATCH_ROWS) >= 64:
-            _PATCH_ROWS.clear()
-        _PATCH_ROWS[key] = rows
-    return rows
 
 
 class AdapterDownFunction(Function):
@@ -425,10 +389,8 @@ class AdapterRowsFunction(Function):
         attn = []
         if len(need) > 14:
             saved, attn = saved[:-_ATTN_PARAMS], saved[-_ATTN_PARAMS:]
-        B, N, _ = go.shape
-        rows = gamma.new_empty(0, dtype=torch.int32) if attn else _token_rows(B, N, S, go.device)
         gx, gw_d, gb_d, gw_c, gb_c, gw_u, gb_u, g_gamma, g_gate, *ga = _ops.adapter_backward(
-            go, saved, gamma, nbr, hm_rows, hm_gate, rows, attn, S, tpb, nk, eps1, symmetric, has_bd, has_bc, need[0],
+            go, saved, gamma, nbr, hm_rows, hm_gate, attn, S, tpb, nk, eps1, symmetric, has_bd, has_bc, need[0],
             need[1], f32, x_dt == torch.float32)
         g = lambda want, t: t if want else None  # noqa: E731
         return (g(need[0], gx), g(need[1], gw_d), g(has_bd, gb_d), gw_c, g(has_bc, gb_c), gw_u, g(has_bu, gb_u), g_gamma,

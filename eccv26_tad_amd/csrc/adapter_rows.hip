@@ -37,6 +37,11 @@ struct PrepJobs {
     int count;
 };
 
+// Outputs of a job.
+__host__ __device__ __forceinline__ int64_t prep_outputs(const svtad_prep_job& j) {
+    return j.kind == SVTAD_PREP_TOKEN_ROWS ? (int64_t)j.off * (j.pair ? j.n - j.k : j.n) : (int64_t)j.off * j.n * j.k;
+}
+
 // One thread per 8 output values. The values go through T first (autocast's
 // cast) and, with gamma, through T again after the product, as the separate
 // casts and multiply round them.
@@ -46,9 +51,20 @@ __global__ __launch_bounds__(256) void k_adapter_prep(PrepJobs jobs) {
     while (q + 1 < jobs.count && (int)blockIdx.x >= jobs.first[q + 1]) ++q;
     const svtad_prep_job j = jobs.j[q];
     const int64_t slot = (int64_t)((int)blockIdx.x - jobs.first[q]) * 256 + threadIdx.x;
-    const int64_t total = (int64_t)j.off * j.n * j.k;
+    const int64_t total = prep_outputs(j);
     if (j.kind == SVTAD_PREP_CONV_BWD && slot == 0) *(uint32_t*)((T*)j.dst + total) = 0u;  // orphan flag after the layout
     if (slot * 8 >= total) return;
+    if (j.kind == SVTAD_PREP_TOKEN_ROWS) {
+        // written by the training forward's one launch: a list kept between
+        // calls would have to follow streams and graph captures
+        const uint32_t S = (uint32_t)j.k, P = (uint32_t)(j.n - j.k), head = j.pair ? 0u : (uint32_t)j.off * S;
+        for (int64_t e = slot * 8; e < total && e < slot * 8 + 8; ++e) {
+            const uint32_t t = (uint32_t)e;
+            const uint32_t b = t < head ? t / S : (t - head) / P;
+            ((int32_t*)j.dst)[e] = (int32_t)(b * (uint32_t)j.n + (t < head ? t - b * S : S + (t - head) - b * P));
+        }
+        return;
+    }
     if (j.kind == SVTAD_PREP_WIDEN) {
         const u32x4 v = *(const u32x4*)((const T*)j.src + slot * 8);
         f32x4 o[2];
@@ -466,18 +482,19 @@ extern "C" int svtad_adapter_prep(const svtad_prep_job* jobs, int count, int dty
     int64_t blocks = 0;
     for (int q = 0; q < count; ++q) {
         const svtad_prep_job& j = jobs[q];
-        if (!j.src || !j.dst || !al16r(j.dst) || j.kind < SVTAD_PREP_CAST || j.kind > SVTAD_PREP_WIDEN || j.off < 1 ||
-            j.n < 1 || j.k < 1)
+        const bool list = j.kind == SVTAD_PREP_TOKEN_ROWS;
+        if ((!j.src && !list) || !j.dst || !al16r(j.dst) || j.kind < SVTAD_PREP_CAST || j.kind > SVTAD_PREP_TOKEN_ROWS ||
+            j.off < 1 || j.n < 1 || j.k < (list ? 0 : 1) || (list && (j.k > j.n || (int64_t)j.off * j.n >= (int64_t)INT32_MAX)))
             return set_error(SVTAD_ERR_INVALID, "adapter_prep: bad job");
         if (j.kind == SVTAD_PREP_WIDEN && (!al16r(j.src) || j.src_f32 || j.gamma))
             return set_error(SVTAD_ERR_INVALID, "adapter_prep: bad job");
-        if (j.kind == SVTAD_PREP_CAST || j.kind == SVTAD_PREP_WIDEN ? (int64_t)j.off * j.n * j.k % 8 != 0 : (j.k % 32 != 0 || j.n % 32 != 0))
+        if (!list && (j.kind == SVTAD_PREP_CAST || j.kind == SVTAD_PREP_WIDEN ? (int64_t)j.off * j.n * j.k % 8 != 0 : (j.k % 32 != 0 || j.n % 32 != 0)))
             return set_error(SVTAD_ERR_UNSUPPORTED, "adapter_prep: shape without a layout");
-        if ((int64_t)j.off * j.n * j.k >= (int64_t)INT32_MAX)
+        if (prep_outputs(j) >= (int64_t)INT32_MAX)
             return set_error(SVTAD_ERR_UNSUPPORTED, "adapter_prep: 2^31 values or more");
         pj.j[q] = j;
         pj.first[q] = (int)blocks;
-        blocks += cdiv((int64_t)j.off * j.n * j.k, 2048);
+        blocks += cdiv(prep_outputs(j), 2048);
     }
     pj.first[count] = (int)blocks;
     if (blocks == 0) return SVTAD_OK;

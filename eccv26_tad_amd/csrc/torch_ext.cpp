@@ -1018,10 +1018,18 @@ struct PrepList {
         push(SVTAD_PREP_WIDEN, g, dst, 1, 1, g.numel(), false, nullptr);
         return dst;
     }
-    void launch() {
+    // row of the [B * N, .] matrix of each special token, then of each patch token (patch_only: of those)
+    at::Tensor token_rows(int64_t B, int64_t N, int64_t S, bool patch_only) {
+        const int64_t count = B * (patch_only ? N - S : N);
+        at::Tensor rows = at::empty({count}, opt.dtype(at::kInt));
+        if (count > 0)
+            jobs.push_back(svtad_prep_job{nullptr, rows.data_ptr(), nullptr, SVTAD_PREP_TOKEN_ROWS, (int)B, (int)N, (int)S, 0, 0,
+                                          patch_only});
+        return rows;
+    }
+    void launch(void* stream) {
         if (!jobs.empty())
-            check_status(svtad_adapter_prep(jobs.data(), (int)jobs.size(), t == at::kHalf ? SVTAD_F16 : SVTAD_BF16,
-                                            stream_of(keep[0])),
+            check_status(svtad_adapter_prep(jobs.data(), (int)jobs.size(), t == at::kHalf ? SVTAD_F16 : SVTAD_BF16, stream),
                          "adapter_prep");
     }
 };
@@ -1075,8 +1083,20 @@ std::vector<at::Tensor> op_adapter_prep(const at::Tensor& w_d, const c10::option
     c10::DeviceGuard g(w_d.device());
     PrepList L(w_d, bf16);
     auto out = adapter_prep_jobs(L, w_d, b_d, w_c, b_c, w_u, b_u, gamma, train, pack_conv);
-    L.launch();
+    L.launch(stream_of(w_d));
     return out;
+}
+
+// patch_rows(like, B, N, S) -> int32 [B * (N - S)]: the row of like's [B * N, .]
+// matrix of each patch token, in the order of the SparseConv2D rows
+at::Tensor op_patch_rows(const at::Tensor& like, int64_t B, int64_t N, int64_t S) {
+    check_gpu(like, "like");
+    TORCH_CHECK(B >= 0 && S >= 0 && S <= N && N < (int64_t)INT32_MAX && B * N < (int64_t)INT32_MAX, "patch_rows: bad sizes");
+    c10::DeviceGuard g(like.device());
+    PrepList L(like, true);
+    at::Tensor rows = L.token_rows(B, N, S, true);
+    L.launch(stream_of(like));
+    return rows;
 }
 
 // x contiguous; a float32 x (whose cast once gave a fresh buffer) on 16 bytes
@@ -1307,7 +1327,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> op_key_attention_bwd(const at::Te
 // ---------------------------------------------------------------------------
 
 enum { A_NW, A_NB, A_DW, A_DB, A_QW, A_QB, A_QNW, A_QNB, A_KNW, A_KNB, A_PW, A_PB, A_GAMMA, A_COUNT };
-enum { S_X, S_PRE, S_CBUF, S_PA, S_WC, S_WU, S_BU, S_WDT, S_WUT, S_PB, S_COUNT };
+enum { S_X, S_PRE, S_CBUF, S_PA, S_WC, S_WU, S_BU, S_WDT, S_WUT, S_PB, S_ROWS, S_COUNT };
 enum { S_COMB = S_COUNT, S_STATS, S_XN, S_DW, S_XA, S_QW, S_Q, S_KV, S_ATT, S_PW, S_PBIAS, S_X2, S_DWT, S_QWT, S_PWT, S_ACOUNT };
 
 // x [M, k] W^T + bias, [M, n] in x's type (W in fragment order, pair columns)
@@ -1369,7 +1389,10 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
         }
         pbias = L.cast(attn[A_PB]);
     }
-    L.launch();
+    TORCH_CHECK(N < (int64_t)INT32_MAX && M < (int64_t)INT32_MAX, "adapter_forward: 2^31 rows or more");
+    // with attention the up projection's operand is in token order
+    at::Tensor rows = train && !a ? L.token_rows(B, N, S, false) : at::empty({0}, L.opt.dtype(at::kInt));
+    L.launch(stream_of(x));
     // special rows first, then the patch rows' SparseConv2D output: the up
     // projection's operand, and its weight gradient's in one row list
     at::Tensor cbuf = at::empty({M, h}, L.opt);
@@ -1432,22 +1455,21 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
                        : op_adapter_rows_res(sp, conv, P[2], P[3], gamma, xin, out32);
     std::vector<at::Tensor> ret{out, pf, pb};
     if (!train) return ret;
-    for (const at::Tensor& t : {xc, pre, cbuf, pa, P[5], P[6], P[3], P[7], P[8], pb}) ret.push_back(t);
+    for (const at::Tensor& t : {xc, pre, cbuf, pa, P[5], P[6], P[3], P[7], P[8], pb, rows}) ret.push_back(t);
     if (a)
         for (const at::Tensor& t : {comb, stats, xn, dw, xa, qw, q, kv, att, pw, pbias, x2, dwt, qwt, pwt})
             ret.push_back(t.defined() ? t : at::empty({0}, L.opt));
     return ret;
 }
 
-// adapter_backward(go, saved, gamma, neighbor_indices, hm_rows, hm_gate, rows, attn, n_special, tokens_per_batch, nk, eps_head,
+// adapter_backward(go, saved, gamma, neighbor_indices, hm_rows, hm_gate, attn, n_special, tokens_per_batch, nk, eps_head,
 //                  symmetric, has_bd, has_bc, need_x, need_wd, param types [w_d, b_d, w_c, b_c, w_u, b_u], x_float32)
 //   -> [gx, gw_d, gb_d, gw_c, gb_c, gw_u, gb_u, g_gamma, g_gate, attention parameters]
-// rows: the row of go of each row of the saved special / patch buffer.
 // Gradients that are not wanted or do not exist are empty.
 std::vector<at::Tensor> op_adapter_backward(const at::Tensor& go_in, const std::vector<at::Tensor>& saved,
                                             const at::Tensor& gamma, const at::Tensor& nbr,
                                             const c10::optional<at::Tensor>& hm_rows,
-                                            const c10::optional<at::Tensor>& hm_gate, const at::Tensor& rows,
+                                            const c10::optional<at::Tensor>& hm_gate,
                                             const std::vector<at::Tensor>& attn, int64_t S, int64_t tpb, int64_t nk,
                                             double eps_head, bool symmetric, bool has_bd, bool has_bc, bool need_x,
                                             bool need_wd, const std::vector<bool>& f32, bool x_f32) {
@@ -1487,7 +1509,7 @@ std::vector<at::Tensor> op_adapter_backward(const at::Tensor& go_in, const std::
     if (go.scalar_type() == t) goc = go;
     at::Tensor go2 = goc.view({M, E});
     at::Tensor G = with_attn ? op_linear_wgrad(go2, no_rows, saved[S_X2].view({M, h}), true)
-                             : op_linear_wgrad(go2, rows, saved[S_CBUF], true);
+                             : op_linear_wgrad(go2, saved[S_ROWS], saved[S_CBUF], true);
     at::Tensor gsum = b_u.numel() ? op_column_sums(go2) : none, gw_u, gb_u;
     at::Tensor g_gamma = up_grads(w_u, G, b_u, gsum, gamma, nullptr, &gw_u, &gb_u);
     std::vector<at::Tensor> ag;
@@ -1564,7 +1586,7 @@ std::vector<at::Tensor> op_adapter_backward(const at::Tensor& go_in, const std::
     at::Tensor gb_d = has_bd ? L.grad(op_column_sums(du2), want(1)) : none;
     std::vector<at::Tensor> ret{gx, gw_d, gb_d, L.grad(gw_c, want(2)), has_bc ? L.grad(gb_c, want(3)) : none,
                                 L.grad(gw_u, want(4)), b_u.numel() ? L.grad(gb_u, want(5)) : none, g_gamma, g_gate};
-    L.launch();
+    L.launch(st);
     ret.insert(ret.end(), ag.begin(), ag.end());
     return ret;
 }
@@ -1662,6 +1684,8 @@ PYBIND11_MODULE(opentad_sparse_ops, m) {
     m.def("adapter_prep", &op_adapter_prep, "Adapter parameters cast and laid out for adapter_rows_*, one launch",
           py::arg("w_d"), py::arg("b_d"), py::arg("w_c"), py::arg("b_c"), py::arg("w_u"), py::arg("b_u"),
           py::arg("gamma"), py::arg("bf16"), py::arg("train"), py::arg("pack_conv"));
+    m.def("patch_rows", &op_patch_rows, "Rows of the patch tokens of [B, N, .]", py::arg("like"), py::arg("batch"),
+          py::arg("n_tokens"), py::arg("n_special"));
     m.def("adapter_rows_down", &op_adapter_rows_down, "adapter_down over whole token tiles (weight of adapter_prep)",
           py::arg("x"), py::arg("w"), py::arg("bias"), py::arg("n"), py::arg("n_special"), py::arg("copy"));
     m.def("adapter_rows_split", &op_adapter_rows_split, "go W^T split into special and patch rows",

@@ -568,6 +568,9 @@ int svtad_gamma_grad_mixed(const void* w, const void* g, int64_t count, const vo
  *   SVTAD_PREP_COLS      the same of its transpose, src [k, n]
  *   SVTAD_PREP_CONV_FWD  svtad_pack_weight's packed_fwd of src [9, k, n]
  *   SVTAD_PREP_CONV_BWD  svtad_pack_weight's packed_bwd of src [9, n, k]
+ *   SVTAD_PREP_TOKEN_ROWS  (no src, dst int32) row b * n + r of every token r of
+ *                        every sample b of [off, n]: the first k tokens of all
+ *                        samples, then the others (with pair only the others)
  * n and k are multiples of 32 in the layouts. `pair` is 0 for the weight of
  * SVTAD_ROWS_RES and 1 for those of the other kinds (column order).
  */
@@ -577,7 +580,8 @@ enum svtad_prep_kind {
     SVTAD_PREP_COLS = 2,
     SVTAD_PREP_CONV_FWD = 3,
     SVTAD_PREP_CONV_BWD = 4,
-    SVTAD_PREP_WIDEN = 5
+    SVTAD_PREP_WIDEN = 5,
+    SVTAD_PREP_TOKEN_ROWS = 6
 };
 enum { SVTAD_MAX_PREP_JOBS = 28 };
 typedef struct svtad_prep_job {

@@ -125,7 +125,7 @@ def test_inference_prepares_no_backward(mode, attn, monkeypatch):
 
     def forward(x, *args):
         seen.append(args[16])
-        return x.clone(), x.new_empty(0), x.new_empty(0), *[x.new_empty(0)] * (25 if attn else 10)
+        return x.clone(), x.new_empty(0), x.new_empty(0), *[x.new_empty(0)] * (26 if attn else 11)
 
     m = sv.SparseConvAdapter(768, 0.25, use_attn=attn, n_key_tokens=3)
     m.sparse_conv.packed_weight_cache = None  # keyed by the stream of a GPU

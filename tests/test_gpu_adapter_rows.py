@@ -195,3 +195,58 @@ def test_no_grad_matches_grad_mode(dev, embed, attn, amp):
     assert torch.equal(call(torch.enable_grad), cold) and cache._packed[1] is not None
     kept = cache._packed
     assert torch.equal(call(torch.no_grad), cold) and cache._packed is kept
+
+
+@pytest.mark.parametrize("B,N,S", [(1, 1, 0), (1, 9, 1), (3, 7, 7), (2, 1025, 0), (3, 683, 4), (4, 513, 512)])
+def test_patch_rows(dev, B, N, S):
+    import eccv26_tad_amd as sv
+
+    want = torch.arange(B * N, device=dev).view(B, N)[:, S:].reshape(-1)
+    got = sv.ops.patch_rows(torch.empty(0, device=dev), B, N, S)
+    assert got.dtype == torch.int32 and torch.equal(got.long(), want)
+
+
+@pytest.mark.parametrize("embed", [384, 512])
+def test_first_backward_of_a_shape_in_a_capture(dev, embed):
+    """Nothing of a backward that ran only inside a graph capture, or on another
+    stream, is read by a later one."""
+    import eccv26_tad_amd as sv
+
+    g = torch.Generator(device=dev).manual_seed(embed)
+    mod = sv.SparseConvAdapter(embed, 0.25).to(dev, torch.float16)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.add_(0.1 * torch.randn(p.shape, generator=g, device=dev))
+    params = list(mod.parameters())
+
+    def inputs(T):
+        idx = torch.arange(20 * T, device=dev).expand(2, -1)
+        table = sv.build_neighbor_table(torch.ones(2, T, 4, 5, dtype=torch.uint8, device=dev), batched=True, n=40 * T)
+        x = torch.randn(2, 2 + 20 * T, embed, generator=g, device=dev).half().requires_grad_(True)
+        return x, (4, 5, idx, 20 * T, table), torch.randn(2, 2 + 20 * T, embed, generator=g, device=dev).half()
+
+    def step(x, args, go):
+        return torch.autograd.grad(mod(x, *args), [x] + params, go)
+
+    def same(a, b):
+        return all(torch.equal(s, t) for s, t in zip(a, b))
+
+    warm, case = inputs(3), inputs(5)
+    side = torch.cuda.Stream(dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        step(*warm)
+    torch.cuda.current_stream(dev).wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step(*case)
+    eager = step(*case)  # before any replay
+    with torch.cuda.stream(side):
+        side.wait_stream(torch.cuda.current_stream(dev))
+        other = step(*case)
+    torch.cuda.current_stream(dev).wait_stream(side)
+    assert same(eager, other)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize(dev)
+        assert same(captured, eager) and same(step(*case), eager)
