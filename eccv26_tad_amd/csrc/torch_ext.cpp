@@ -1417,13 +1417,14 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
     at::Tensor tab = table_i32(nbr, pa.size(0));
     int mode = P[4].numel() ? (int)bias_mode : SVTAD_BIAS_NONE;
     if (mode == SVTAD_BIAS_FP32) mode = SVTAD_BIAS_PRE;  // the bias in the compute type, widened exactly
+    int packed_st = SVTAD_ERR_UNSUPPORTED;
     if (pf.numel())
-        check_status(svtad_fwd_packed(pa.data_ptr(), tab.data_ptr<int32_t>(), pf.data_ptr(),
-                                      mode ? P[4].data_ptr() : nullptr, mode, conv.data_ptr(), pa.size(0), (int)h, (int)h,
-                                      tpb, dt, st),
-                     "adapter_forward");
-    else
+        packed_st = svtad_fwd_packed(pa.data_ptr(), tab.data_ptr<int32_t>(), pf.data_ptr(), mode ? P[4].data_ptr() : nullptr,
+                                     mode, conv.data_ptr(), pa.size(0), (int)h, (int)h, tpb, dt, st);
+    if (packed_st == SVTAD_ERR_UNSUPPORTED)  // no packed layout, or operands of 2^31 bytes: as op_fwd_packed
         conv.copy_(conv_fwd(pa, tab, P[5], P[4], tpb, (int)bias_mode, -1));
+    else
+        check_status(packed_st, "adapter_forward");
     at::Tensor comb, stats, xn, xa, q, kv, att, x2;
     if (a) {
         TORCH_CHECK(svtad_key_attention_ok(4, (int)a / 4, N, (int)nk), "adapter_forward: attention size");

@@ -250,3 +250,34 @@ def test_first_backward_of_a_shape_in_a_capture(dev, embed):
         graph.replay()
         torch.cuda.synchronize(dev)
         assert same(captured, eager) and same(step(*case), eager)
+
+
+def test_patch_rows_of_2_gib(dev):
+    """Inference where the convolution's operand reaches 2^31 bytes, beyond the
+    32-bit offsets of its packed kernel: sampled rows against float32."""
+    import eccv26_tad_amd as sv
+
+    n, E, h, S = 2 ** 31 // 512, 768, 256, 1
+    g = torch.Generator(device=dev).manual_seed(3)
+    mod = sv.SparseConvAdapter(E, 0.25).to(dev, torch.float16)
+    with torch.no_grad():
+        mod.up_proj.weight.copy_(0.05 * torch.randn(E, h, generator=g, device=dev))
+    x = torch.randn(1, S + n, E, generator=g, device=dev, dtype=torch.float16)
+    step = torch.arange(9, device=dev, dtype=torch.int32) - 4
+    table = torch.arange(n, device=dev, dtype=torch.int32).view(n, 1) + step
+    table = torch.where((table >= 0) & (table < n), table, -1)
+    idx = torch.arange(n, device=dev).view(1, n)
+    with torch.no_grad():
+        y = mod(x, 1, n, idx, n, table.view(1, n, 9))
+    rows = torch.cat([torch.tensor([0, 1, 2, 3, n // 2, n - 4, n - 2, n - 1], device=dev),
+                      torch.randint(0, n, (200,), generator=g, device=dev)])
+    p = {k: v.detach().float() for k, v in mod.named_parameters()}
+    near = table[rows].long()
+    src = x[0, S + near.clamp_min(0)].float()
+    u = F.gelu(F.linear(src, p["down_proj.weight"], p["down_proj.bias"])) * (near >= 0).unsqueeze(-1)
+    conv = p["sparse_conv.bias"] + u.flatten(1) @ p["sparse_conv.weight"].reshape(9 * h, h)
+    want = F.linear(conv, p["up_proj.weight"], p["up_proj.bias"]) * p["gamma"] + x[0, S + rows].float()
+    got = y[0, S + rows].float()
+    # the parts' roundings to float16 (hidden rows, convolution, z, output), each 2^-11 of its value
+    assert float((got - want).norm() / want.norm()) <= 4 * 2.0 ** -11
+    assert float((got - want).abs().max()) <= 8 * 2.0 ** -11 * float(want.abs().max())
