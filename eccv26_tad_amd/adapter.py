@@ -581,9 +581,11 @@ class SparseConvAdapter(nn.Module):
                 nbr = nbr.to(torch.int32)
             nbr = _keep_symmetric(neighbor_indices, nbr)
         conv = self.sparse_conv
-        # with attention sparse_conv is called, unless a call would only read its parameters
-        key_attn = self.use_attn == 2 and _is_plain(conv, SparseConv2d) and self._key_attention_ok(B, N)
-        if not self.use_attn or key_attn:
+        attn = ()
+        if self.use_attn == 2 and _is_plain(conv, SparseConv2d):
+            # with attention sparse_conv is called, unless a call would only read its parameters
+            attn = self._key_attention_layers(B, N)
+        if not self.use_attn or attn:
             hm_rows = hm_gate = None
             if self._uses_heatmap():
                 H_hm, W_hm = self.heatmap_grid_size
@@ -602,10 +604,9 @@ class SparseConvAdapter(nn.Module):
                     # packed with the other parameters' preparation when not current
                     packed = cache.peek(conv.weight, cd, grad_mode)
                     keep_packed = functools.partial(cache.put, conv.weight, cd)
-                attn, nk, eps = (), 0, (0.0, 0.0)
-                if key_attn:
-                    attn, nk = self._attention_parameters(), self.n_key_tokens
-                    eps = (self.attn_norm.eps, self.q_norm.eps)
+                nk, eps = 0, (0.0, 0.0)
+                if attn:
+                    nk, eps = self.n_key_tokens, (self.attn_norm.eps, self.q_norm.eps)
                 return AdapterRowsFunction.apply(x, self.down_proj.weight, self.down_proj.bias, conv.weight, conv.bias,
                                                  self.up_proj.weight, self.up_proj.bias, self.gamma, nbr, hm_rows,
                                                  hm_gate, packed, keep_packed,
@@ -630,26 +631,25 @@ class SparseConvAdapter(nn.Module):
                 self.qkv.bias, self.q_norm.weight, self.q_norm.bias, self.k_norm.weight, self.k_norm.bias,
                 self.attn_proj.weight, self.attn_proj.bias, self.attn_gamma)
 
-    def _key_attention_ok(self, batch, n_tokens):
-        """Whether ``KeyTokenAttentionFunction`` takes this module: its widths
-        and key count, norms with weight and bias and one eps, biased Linear
-        layers, one parameter type for the norms of a kernel, and layers that a
-        call runs as they are; the kernels' grids take 1 to 65535 samples."""
+    def _key_attention_layers(self, batch, n_tokens):
+        """The parameters for the native key-token attention, or () when it does
+        not take this module: layers that a call runs as they are, of the widths,
+        types and key count of ``key_attention_layers_ok``, and one eps for the
+        head norms; the kernels' grids take 1 to 65535 samples."""
         if not 1 <= batch <= 65535:
-            return False
-        norms = (self.attn_norm, self.q_norm, self.k_norm)
-        if not all(_is_plain(m, nn.LayerNorm) for m in norms):
-            return False
+            return ()
+        if not all(_is_plain(m, nn.LayerNorm) for m in (self.attn_norm, self.q_norm, self.k_norm)):
+            return ()
         if not (_is_plain(self.down_attn, nn.Linear) and _is_plain(self.qkv, nn.Linear)):
-            return False
-        if any(m.weight is None or m.bias is None or m.weight.dtype != m.bias.dtype for m in norms):
-            return False
-        if self.q_norm.eps != self.k_norm.eps or self.q_norm.weight.dtype != self.k_norm.weight.dtype:
-            return False
-        if self.down_attn.bias is None or self.qkv.bias is None or self.attn_proj.bias is None or self.hidden_dims not in (128, 256):
-            return False
-        return _ops.key_attention_ok(self.num_heads, self.hidden_dims // 2 // self.num_heads, n_tokens,
-                                     self.n_key_tokens)
+            return ()
+        if self.q_norm.eps != self.k_norm.eps:
+            return ()
+        attn = self._attention_parameters()
+        ok = _ops.key_attention_layers_ok(attn, self.down_proj.weight.shape[0], self.num_heads, n_tokens, self.n_key_tokens)
+        return attn if ok else ()
+
+    def _key_attention_ok(self, batch, n_tokens):
+        return bool(self._key_attention_layers(batch, n_tokens))
 
     def _attention_branch(self, x_comb, S, indices, h, w, total_num_patches, fused, cd=None):
         """The ``use_attn`` branch on ``x_combined`` (vit_sparse_adapter_poguise.py:
@@ -688,11 +688,10 @@ class SparseConvAdapter(nn.Module):
             fr_out = coarse[:, S:]
             pa_out = torch.gather(fr_out.float(), 1, idx).to(fr_out.dtype) if fused else torch.gather(fr_out, 1, idx)
             return shortcut + torch.cat([sp_out, pa_out], dim=1)
-        if fused and self.use_attn == 2 and self._key_attention_ok(B, N):
-            xa = KeyTokenAttentionFunction.apply(
-                x_comb, self.attn_norm.weight, self.attn_norm.bias, self.down_attn.weight, self.down_attn.bias,
-                self.qkv.weight, self.qkv.bias, self.q_norm.weight, self.q_norm.bias, self.k_norm.weight,
-                self.k_norm.bias, self.n_key_tokens, (self.attn_norm.eps, self.q_norm.eps), cd)
+        attn = self._key_attention_layers(B, N) if fused and self.use_attn == 2 else ()
+        if attn:
+            xa = KeyTokenAttentionFunction.apply(x_comb, *attn[:10], self.n_key_tokens,
+                                                 (self.attn_norm.eps, self.q_norm.eps), cd)
             return AdapterUpFunction.apply(xa.new_empty(B, 0, xa.shape[-1]), xa.view(B * N, -1), self.attn_proj.weight,
                                            self.attn_proj.bias, self.attn_gamma, shortcut, False, cd)
         xa = self.down_attn(self.attn_norm(x_comb))

@@ -1229,6 +1229,29 @@ at::Tensor op_adapter_rows_res(const c10::optional<at::Tensor>& sp_in, const at:
 // attention to the key tokens
 // ---------------------------------------------------------------------------
 
+enum { A_NW, A_NB, A_DW, A_DB, A_QW, A_QB, A_QNW, A_QNB, A_KNW, A_KNB, A_PW, A_PB, A_GAMMA, A_COUNT };
+
+// key_attention_layers_ok(parameters in the order above or None, hidden, heads, n, nk): whether the
+// kernels take them: every one there, of the widths that hidden gives (the
+// kernels read that many values), norm parameters contiguous and of one type
+// per kernel, and svtad_key_attention_ok's sizes
+bool op_key_attention_layers_ok(const std::vector<c10::optional<at::Tensor>>& p, int64_t h, int64_t heads, int64_t n, int64_t nk) {
+    if (p.size() != A_COUNT || (h != 128 && h != 256) || heads != 4 || nk >= 1024) return false;
+    const int64_t a = h / 2, hd = a / 4;
+    if (!svtad_key_attention_ok(4, (int)hd, n, (int)nk)) return false;
+    for (const auto& t : p)
+        if (!t.has_value() || !t->defined()) return false;
+    auto rows = [&](int i, int64_t r) { return p[i]->dim() == 1 && p[i]->size(0) == r; };
+    auto mat = [&](int i, int64_t r, int64_t c) { return p[i]->dim() == 2 && p[i]->size(0) == r && p[i]->size(1) == c; };
+    if (!mat(A_DW, a, h) || !rows(A_DB, a) || !mat(A_QW, 3 * a, a) || !rows(A_QB, 3 * a) || !mat(A_PW, h, a) || !rows(A_PB, h))
+        return false;
+    for (int i : {A_NW, A_NB, A_QNW, A_QNB, A_KNW, A_KNB}) {
+        const int first = i <= A_NB ? A_NW : A_QNW;
+        if (!rows(i, i <= A_NB ? h : hd) || !p[i]->is_contiguous() || p[i]->scalar_type() != p[first]->scalar_type()) return false;
+    }
+    return true;
+}
+
 static void attn_params(const at::Tensor& like, std::initializer_list<const at::Tensor*> ps, int64_t n) {
     const at::ScalarType t = (*ps.begin())->scalar_type();
     TORCH_CHECK(t == like.scalar_type() || t == at::kFloat, "norm parameters take the row type or float32");
@@ -1326,7 +1349,6 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> op_key_attention_bwd(const at::Te
 // the adapter's forward and backward as one call each (widths of adapter_rows_ok)
 // ---------------------------------------------------------------------------
 
-enum { A_NW, A_NB, A_DW, A_DB, A_QW, A_QB, A_QNW, A_QNB, A_KNW, A_KNB, A_PW, A_PB, A_GAMMA, A_COUNT };
 enum { S_X, S_PRE, S_CBUF, S_PA, S_WC, S_WU, S_BU, S_WDT, S_WUT, S_PB, S_ROWS, S_COUNT };
 enum { S_COMB = S_COUNT, S_STATS, S_XN, S_DW, S_XA, S_QW, S_Q, S_KV, S_ATT, S_PW, S_PBIAS, S_X2, S_DWT, S_QWT, S_PWT, S_ACOUNT };
 
@@ -1362,6 +1384,8 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
     c10::DeviceGuard g(x.device());
     const int64_t B = x.size(0), N = x.size(1), h = w_d.size(0), M = B * N;
     TORCH_CHECK(S >= 0 && S <= N, "n_special out of range");
+    TORCH_CHECK(attn.empty() || op_key_attention_layers_ok({attn.begin(), attn.end()}, h, 4, N, nk),
+                "adapter_forward: attention parameters or sizes without a kernel");
     PrepList L(x, bf16);
     const bool pack = !pf_in.has_value();
     auto P = adapter_prep_jobs(L, w_d, b_d, w_c, b_c, w_u, b_u, gamma, train, pack);
@@ -1427,7 +1451,6 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
         check_status(packed_st, "adapter_forward");
     at::Tensor comb, stats, xn, xa, q, kv, att, x2;
     if (a) {
-        TORCH_CHECK(svtad_key_attention_ok(4, (int)a / 4, N, (int)nk), "adapter_forward: attention size");
         attn_params(cbuf, {&attn[A_NW], &attn[A_NB]}, h);
         comb = S ? at::empty({B, N, h}, L.opt) : conv.view({B, N, h});
         xn = at::empty({M, h}, L.opt);
@@ -1601,6 +1624,8 @@ PYBIND11_MODULE(opentad_sparse_ops, m) {
           py::arg("stats"), py::arg("w"));
     m.def("key_attention_ok", &op_key_attention_ok, "Whether key_attention takes these sizes", py::arg("heads"),
           py::arg("head_dim"), py::arg("n"), py::arg("nk"));
+    m.def("key_attention_layers_ok", &op_key_attention_layers_ok, "Whether the key-token attention takes these parameters",
+          py::arg("parameters"), py::arg("hidden"), py::arg("heads"), py::arg("n"), py::arg("nk"));
     m.def("key_attention", &op_key_attention, "Normalised attention of the visual tokens to the key tokens", py::arg("q"),
           py::arg("kv"), py::arg("qn_w"), py::arg("qn_b"), py::arg("kn_w"), py::arg("kn_b"), py::arg("eps"));
     m.def("key_attention_bwd", &op_key_attention_bwd, "Its gradients (dq, dkv, norm parameters)", py::arg("dout"),

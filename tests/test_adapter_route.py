@@ -68,8 +68,9 @@ class _Route(Exception):
 
 
 def _route(m, monkeypatch):
-    """Which route a 16-bit call takes: "one node", or "layers" when the
-    modules' calls (sparse_conv among them) run."""
+    """Which route a 16-bit call takes: "one node" for AdapterRowsFunction,
+    "chain" for the node of other widths, or "layers" when the modules' calls
+    (sparse_conv among them) run."""
     from eccv26_tad_amd import adapter
 
     def take(name):
@@ -79,6 +80,7 @@ def _route(m, monkeypatch):
 
     monkeypatch.setattr(adapter.SparseConvAdapter, "_fused_dtype", lambda self, x: torch.bfloat16)
     monkeypatch.setattr(adapter.AdapterRowsFunction, "apply", take("one node"))
+    monkeypatch.setattr(adapter.SparseConvAdapterFunction, "apply", take("chain"))
     monkeypatch.setattr(adapter.AdapterDownFunction, "apply", take("layers"))
     with pytest.raises(_Route) as route:
         m(torch.zeros(2, 8, 768), 1, 5, torch.arange(5).expand(2, -1), 5, torch.full((2, 5, 9), -1, dtype=torch.int32))
@@ -135,3 +137,33 @@ def test_inference_prepares_no_backward(mode, attn, monkeypatch):
     with {"no_grad": torch.no_grad, "inference_mode": torch.inference_mode}.get(mode, torch.enable_grad)():
         y = m(torch.zeros(2, 8, 768), 1, 5, torch.arange(5).expand(2, -1), 5, torch.full((2, 5, 9), -1, dtype=torch.int32))
     assert seen == [mode == "grad"] and y.requires_grad == (mode == "grad")
+
+
+def _strided(norm):
+    norm.weight = torch.nn.Parameter(torch.ones(2 * norm.weight.numel())[::2])
+
+
+SHAPES = {
+    "qkv_in": lambda m: setattr(m, "qkv", torch.nn.Linear(64, 384)),
+    "qkv_out": lambda m: setattr(m, "qkv", torch.nn.Linear(128, 256)),
+    "down": lambda m: setattr(m, "down_attn", torch.nn.Linear(256, 64)),
+    "down_in": lambda m: setattr(m, "down_attn", torch.nn.Linear(128, 128)),
+    "proj": lambda m: setattr(m, "attn_proj", torch.nn.Linear(128, 128)),
+    "proj_bias": lambda m: setattr(m, "attn_proj", torch.nn.Linear(128, 256, bias=False)),
+    "norm": lambda m: setattr(m, "attn_norm", torch.nn.LayerNorm(128)),
+    "no_affine": lambda m: setattr(m, "attn_norm", torch.nn.LayerNorm(256, elementwise_affine=False)),
+    "head_norm": lambda m: setattr(m, "q_norm", torch.nn.LayerNorm(16)),
+    "strided_norm": lambda m: _strided(m.attn_norm),
+    "strided_head_norm": lambda m: _strided(m.k_norm),
+    "norm_types": lambda m: m.k_norm.half(),
+    "hidden": lambda m: setattr(m, "down_proj", torch.nn.Linear(768, 128)),
+}
+
+
+@pytest.mark.parametrize("change", sorted(SHAPES))
+def test_layers_of_other_shapes_are_called(change):
+    """The kernels read as many values as their widths give: layers of other
+    shapes and strides stay with PyTorch, which takes or refuses them."""
+    m = _module()
+    SHAPES[change](m)
+    assert not m._key_attention_ok(2, 4)
