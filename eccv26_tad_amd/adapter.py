@@ -598,7 +598,8 @@ class SparseConvAdapter(nn.Module):
             cache = conv.packed_weight_cache
             packed = None
             grad_mode = torch.is_grad_enabled()
-            if _ops.adapter_rows_ok(self.embed_dims, self.hidden_dims):
+            hidden, embed = self.down_proj.weight.shape  # of the layers in place, which may have been exchanged
+            if _ops.adapter_rows_ok(embed, hidden):
                 keep_packed = None
                 if cache is not None:
                     # packed with the other parameters' preparation when not current

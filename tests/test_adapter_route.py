@@ -167,3 +167,10 @@ def test_layers_of_other_shapes_are_called(change):
     m = _module()
     SHAPES[change](m)
     assert not m._key_attention_ok(2, 4)
+
+
+def test_exchanged_widths_take_their_own_route(monkeypatch):
+    m = sv.SparseConvAdapter(768, 0.25)
+    assert _route(m, monkeypatch) == "one node"
+    m.down_proj, m.up_proj, m.sparse_conv = torch.nn.Linear(768, 64), torch.nn.Linear(64, 768), sv.SparseConv2d(64, 64)
+    assert _route(m, monkeypatch) == "chain"
