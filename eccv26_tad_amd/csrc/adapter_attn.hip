@@ -330,18 +330,24 @@ __global__ __launch_bounds__(256) void k_key_attn_sum(const float* __restrict__ 
     sums[(int64_t)blockIdx.y * count + e] = s;
 }
 
-// The keys' LayerNorm backward and the small sums, one workgroup of A threads:
-// dkv [B, nk, 2 A] and dn [4][HD] (qn_w, qn_b, kn_w, kn_b gradients).
+// The keys' LayerNorm backward and the small sums: dkv [B, nk, 2 A] and, per
+// workgroup of A threads and `per` samples, dn [4][HD] (qn_w, qn_b, kn_w, kn_b
+// gradients). A key is a chain of loads and lane sums, 0.53 us: up to
+// kKeysInOne keys run in one workgroup (6 keys 4.7 us, 16 keys 10.1), more in
+// up to kKeyGroups, whose sums a reduction adds (20 keys 11.8 -> 3.9 + 2.1 us,
+// 256 samples of 16 keys 2162 -> 10.6 + 4.4).
+constexpr int kKeysInOne = 8, kKeyGroups = 256;
 template <typename T, int HD>
 __global__ __launch_bounds__(4 * HD) void k_key_attn_keys(KeyAttnArgs p, const float* __restrict__ sums, int batch,
-                                                          T* __restrict__ dkv, float* __restrict__ dn) {
+                                                          int per, T* __restrict__ dkv, float* __restrict__ dn) {
     constexpr int A = 4 * HD;
     __shared__ float red[4][A];
     const int c = threadIdx.x, j = c % HD;
     const int nr = 2 * p.nk + 2;
     const float kw = load_param<T>(p.kn_w, j, p.p32);
     float dqw = 0.f, dqb = 0.f, dkw = 0.f, dkb = 0.f;
-    for (int b = 0; b < batch; ++b) {
+    const int b1 = min(batch, ((int)blockIdx.x + 1) * per);
+    for (int b = (int)blockIdx.x * per; b < b1; ++b) {
         const float* const s = sums + (int64_t)b * nr * A;
         const T* const kv = (const T*)p.kv + (int64_t)b * p.nk * 2 * A;
         for (int t = 0; t < p.nk; ++t) {
@@ -367,7 +373,7 @@ __global__ __launch_bounds__(4 * HD) void k_key_attn_keys(KeyAttnArgs p, const f
     __syncthreads();
     for (int e = c; e < 4 * HD; e += A) {
         const float* r = red[e / HD] + e % HD;
-        dn[e] = r[0] + r[HD] + r[2 * HD] + r[3 * HD];
+        dn[blockIdx.x * 4 * HD + e] = r[0] + r[HD] + r[2 * HD] + r[3 * HD];
     }
 }
 
@@ -539,9 +545,16 @@ static int64_t key_attn_part(int64_t batch, int64_t n, int nk, int hd) {
     return batch * cdiv(n, kAttnRows) * (2 * nk + 2) * 4 * hd;
 }
 
+// Samples per workgroup of k_key_attn_keys.
+static int key_samples(int64_t batch, int nk) {
+    return (int)(batch * nk <= kKeysInOne ? batch : cdiv(batch, std::min<int64_t>(batch, kKeyGroups)));
+}
+
 extern "C" size_t svtad_key_attention_bwd_workspace_bytes(int64_t batch, int64_t n, int nk, int head_dim) {
     if (batch < 1 || n < 1 || nk < 1 || head_dim < 1) return 0;
-    return (size_t)(key_attn_part(batch, n, nk, head_dim) + batch * (2 * nk + 2) * 4 * head_dim) * 4;
+    const int64_t groups = cdiv(batch, key_samples(batch, nk));
+    return (size_t)(key_attn_part(batch, n, nk, head_dim) + batch * (2 * nk + 2) * 4 * head_dim +
+                    (groups > 1 ? groups * 4 * head_dim : 0)) * 4;
 }
 
 extern "C" int svtad_key_attention_bwd(const void* dout, const void* q, const void* kv, const void* qn_w, const void* qn_b,
@@ -564,8 +577,10 @@ extern "C" int svtad_key_attention_bwd(const void* dout, const void* q, const vo
     const int count = (2 * nk + 2) * 4 * head_dim;
     hipLaunchKernelGGL(k_key_attn_sum, dim3((unsigned)cdiv(count, 32), (unsigned)batch), dim3(256), 0, s, part, sums,
                        (int)cdiv(n, kAttnRows), count);
+    const int per = key_samples(batch, nk), groups = (int)cdiv(batch, per);
+    float* const dn = groups > 1 ? sums + batch * count : dnorm;
 #define SVTAD_KK(T, H) \
-    hipLaunchKernelGGL((k_key_attn_keys<T, H>), dim3(1), dim3(4 * H), 0, s, p, (const float*)sums, (int)batch, (T*)dkv, dnorm)
+    hipLaunchKernelGGL((k_key_attn_keys<T, H>), dim3((unsigned)groups), dim3(4 * H), 0, s, p, (const float*)sums, (int)batch, per, (T*)dkv, dn)
     if (dtype == SVTAD_F16) {
         if (head_dim == 16) SVTAD_KK(f16, 16);
         else SVTAD_KK(f16, 32);
@@ -574,6 +589,7 @@ extern "C" int svtad_key_attention_bwd(const void* dout, const void* q, const vo
         else SVTAD_KK(bf16, 32);
     }
 #undef SVTAD_KK
+    if (groups > 1) split_reduce(SVTAD_F32, dn, 4 * head_dim, groups, dnorm, s);
     return launch_status();
 }
 

@@ -82,3 +82,11 @@ def test_key_attention(dev, hd, B, N, nk, cd, param):
         assert float(dq.double().abs().max()) <= 1e-5 and float(dn[:3].abs().max()) <= 1e-3
     # the key bias moves every score of a query alike: zero but for rounding
     assert float(dn[3].abs().max()) <= 1e-4 * (1 + float(dn[2].abs().max())) * N ** 0.5
+
+
+@pytest.mark.parametrize("hd", [16, 32])
+@pytest.mark.parametrize("B,N,nk", [(8, 3, 1), (9, 3, 1), (3, 20, 6), (256, 5, 2), (257, 5, 2), (700, 19, 16)])
+@pytest.mark.parametrize("cd,param", TYPES[:2])
+def test_key_attention_of_many_samples(dev, hd, B, N, nk, cd, param):
+    """Up to 8 keys in one workgroup, more in up to 256 of whole samples."""
+    test_key_attention(dev, hd, B, N, nk, cd, param)
