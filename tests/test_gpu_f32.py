@@ -110,3 +110,28 @@ def test_layer_matches_float64(sv, n, ci, co, one_way):
     if not one_way:
         empty = torch.empty(0, dtype=torch.uint8, device="cuda")
         _check("gi", sv.ops.bwd_in_packed(GO, tab, W, empty, n, ci, 0, symmetric=True), gi, mgi, 9 * co)
+
+
+@pytest.mark.parametrize("n,ci,co", [(3601, 512, 512), (15001, 256, 256)])
+def test_backward_weight_of_long_splits(sv, n, ci, co):
+    """Splits of more rows than the kernel lists at once (1024), the last one
+    and its last list uneven; the workspace holds one partial per split."""
+    import ctypes
+    import os
+
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(sv.__file__), "libsvtad_sparse.so"))
+    lib.svtad_bwd_w_workspace_bytes.restype = ctypes.c_size_t
+    lib.svtad_bwd_w_workspace_bytes.argtypes = [ctypes.c_int64] + [ctypes.c_int] * 3
+    splits = lib.svtad_bwd_w_workspace_bytes(n, ci, co, 0) // ((9 * ci * co + co) * 4)
+    assert 1 <= splits and -(-n // splits) > 1024
+    terms = -(-n // splits) + 32 + splits  # a split's rows one after another, then the splits
+    rng = np.random.default_rng(n)
+    t = torch.from_numpy(_table(rng, n, 2)).cuda()
+    x, go = (torch.from_numpy(rng.standard_normal((n, c)).astype(np.float32)).cuda() for c in (ci, co))
+    got_w, got_b = sv.ops.bwd_w_bias(go, x, t, ci, 0, True)
+    for k in range(9):
+        i = (t[:, k] >= 0).nonzero()[:, 0]
+        xs, gs = x[t[i, k].long()].double(), go[i].double()
+        _check("gw", got_w[k], (xs.t() @ gs).cpu().numpy(), (xs.abs().t() @ gs.abs()).cpu().numpy(), terms)
+    g = go.double()
+    _check("gb", got_b, g.sum(0).cpu().numpy(), g.abs().sum(0).cpu().numpy(), terms)
