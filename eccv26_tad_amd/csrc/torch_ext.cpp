@@ -1125,6 +1125,25 @@ static void rows_check(const at::Tensor& a, const at::Tensor& w, int64_t k, int6
                 "adapter_rows: ", what, " takes the type of w or float32");
 }
 
+// Down projection and GELU of the rows of x [B, N, k] (contiguous): the
+// pre-activation, GELU's special rows in sp and patch rows in pa (empty: none),
+// and x in the compute type in xc where it is another tensor than x.
+static void rows_down(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bias, const at::Tensor& pre,
+                      const at::Tensor& sp, const at::Tensor& pa, const at::Tensor& xc, int64_t S, const char* what) {
+    const int64_t k = x.size(2), n = pre.size(2);
+    rows_check(x, w, k, n, "x");
+    svtad_rows_args a = rows_args(SVTAD_ROWS_GELU, x.size(0), x.size(1), S, k, n);
+    a.a0 = x.data_ptr();
+    a.w = w.data_ptr();
+    a.bias = opt_ptr(bias, n, w);
+    a.a_copy = xc.numel() && !xc.is_same(x) ? xc.data_ptr() : nullptr;
+    a.out0 = pre.data_ptr();
+    a.out1 = sp.numel() ? sp.data_ptr() : nullptr;
+    a.out2 = pa.numel() ? pa.data_ptr() : nullptr;
+    a.a_f32 = x.scalar_type() == at::kFloat;
+    check_status(svtad_adapter_rows(&a, dtype_code(w), stream_of(x)), what);
+}
+
 // adapter_rows_down(x [B, N, k], wd, bias or empty, n, n_special, copy) ->
 //   (pre_act [B, N, n], act_special [B, S, n], act_patch [B * (N - S), n], x in the compute type if copy, else empty)
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> op_adapter_rows_down(const at::Tensor& x_in, const at::Tensor& w,
@@ -1132,24 +1151,14 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> op_adapter_rows_down(
                                                                                 int64_t S, bool copy) {
     TORCH_CHECK(x_in.dim() == 3, "x must be [B, N, C]");
     const int64_t B = x_in.size(0), N = x_in.size(1), k = x_in.size(2);
-    rows_check(x_in, w, k, n, "x");
+    rows_check(x_in, w, k, n, "x");  // before n and S size any buffer
     TORCH_CHECK(S >= 0 && S <= N, "n_special out of range");
     at::Tensor x = rows_input(x_in);
     c10::DeviceGuard g(x.device());
     const auto opt = w.options();
     at::Tensor pre = at::empty({B, N, n}, opt), sp = at::empty({B, S, n}, opt), pa = at::empty({B * (N - S), n}, opt);
-    const bool f32 = x.scalar_type() == at::kFloat;
-    at::Tensor xc = copy && f32 ? at::empty({B, N, k}, opt) : at::empty({0}, opt);
-    svtad_rows_args a = rows_args(SVTAD_ROWS_GELU, B, N, S, k, n);
-    a.a0 = x.data_ptr();
-    a.w = w.data_ptr();
-    a.bias = opt_ptr(bias, n, w);
-    a.a_copy = xc.numel() ? xc.data_ptr() : nullptr;
-    a.out0 = pre.data_ptr();
-    a.out1 = sp.numel() ? sp.data_ptr() : nullptr;
-    a.out2 = pa.numel() ? pa.data_ptr() : nullptr;
-    a.a_f32 = f32;
-    check_status(svtad_adapter_rows(&a, dtype_code(w), stream_of(x)), "adapter_rows_down");
+    at::Tensor xc = copy && x.scalar_type() == at::kFloat ? at::empty({B, N, k}, opt) : at::empty({0}, opt);
+    rows_down(x, w, bias, pre, sp, pa, xc, S, "adapter_rows_down");
     return {pre, sp, pa, xc};
 }
 
@@ -1422,21 +1431,10 @@ std::vector<at::Tensor> op_adapter_forward(const at::Tensor& x, const at::Tensor
     at::Tensor cbuf = at::empty({M, h}, L.opt);
     at::Tensor sp = cbuf.narrow(0, 0, B * S).view({B, S, h}), conv = cbuf.narrow(0, B * S, M - B * S);
     at::Tensor xin = rows_input(x), pre = at::empty({B, N, h}, L.opt), pa = at::empty({M - B * S, h}, L.opt);
-    rows_check(xin, P[0], x.size(2), h, "x");
-    const bool f32 = xin.scalar_type() == at::kFloat;
-    at::Tensor xc = train && f32 ? at::empty(x.sizes(), L.opt) : xin;
+    at::Tensor xc = train && xin.scalar_type() == at::kFloat ? at::empty(x.sizes(), L.opt) : xin;
     void* const st = stream_of(x);
     const int dt = L.t == at::kHalf ? SVTAD_F16 : SVTAD_BF16;
-    svtad_rows_args r = rows_args(SVTAD_ROWS_GELU, B, N, S, x.size(2), h);
-    r.a0 = xin.data_ptr();
-    r.w = P[0].data_ptr();
-    r.bias = P[1].numel() ? P[1].data_ptr() : nullptr;
-    r.a_copy = train && f32 ? xc.data_ptr() : nullptr;
-    r.out0 = pre.data_ptr();
-    r.out1 = S ? sp.data_ptr() : nullptr;
-    r.out2 = pa.numel() ? pa.data_ptr() : nullptr;
-    r.a_f32 = f32;
-    check_status(svtad_adapter_rows(&r, dt, st), "adapter_forward");
+    rows_down(xin, P[0], P[1], pre, sp, pa, xc, S, "adapter_forward");
     if (hm_rows.has_value()) op_heatmap_add_(pa, sp, *hm_rows, *hm_gate);
     at::Tensor tab = table_i32(nbr, pa.size(0));
     int mode = P[4].numel() ? (int)bias_mode : SVTAD_BIAS_NONE;
