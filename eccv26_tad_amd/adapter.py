@@ -18,37 +18,50 @@ adapter tokens (1: all tokens, 2: visual tokens attend to the key tokens,
 3: key tokens attend to the visual tokens; ``shortcut + attn_proj(.) *
 attn_gamma``), 4 and above the temporal attention over frame-pooled tokens.
 
-Without attention the module runs as one autograd node
-(``SparseConvAdapterFunction``); its forward is the down GEMM
-(``opentad_sparse_ops.adapter_down``), the heatmap gather-add when it
-applies (``heatmap_add_``), the SparseConv2D forward (weight pack +
-gathered GEMM) and the up GEMM (``opentad_sparse_ops.adapter_up``):
+Without attention, and with the attention to the key tokens (``use_attn`` 2),
+the module runs as one autograd node with one native call each way
+(``AdapterRowsFunction``) where its widths have token-tile kernels
+(``adapter_rows_ok``: embed 384, 768 or 1024, hidden 128 or 256):
 
-* the down GEMM's epilogue adds the bias, rounds the Linear output, applies
-  GELU and writes the special tokens and the (contiguous) SparseConv2D input
-  directly: no GELU pass and no slice copy;
+* one launch casts the parameters and lays them out for the GEMMs, packs the
+  SparseConv2D weight when its cache is not current, and with a backward to
+  come writes the row list of its weight gradients;
+* the down GEMM reads x in its own type and writes the rounded Linear output,
+  GELU of the special tokens and the (contiguous) SparseConv2D input: no cast
+  pass, no GELU pass, no slice copy; the heatmap gather-add follows when it
+  applies;
 * the up GEMM reads the special tokens and the SparseConv2D output in place of
   the concatenation and applies bias, ``gamma`` and the residual before its
-  single store: no cat, no scale pass, no add pass;
-* ``tokens_per_batch`` defaults to 0 (the tables the backbone builds are
-  global), so there is no host sync; ``None`` restores the reference's
-  ``max()`` heuristic (``sparse_conv_layer.py:174-177``).
+  single store; with attention the row LayerNorm, the projections and the
+  attention kernels come before it (``KeyTokenAttentionFunction`` describes
+  them), and ``shortcut + attn_proj(.) * attn_gamma`` is an up GEMM too;
+* the backward's input gradients are GEMMs of the same kind: the gradient of
+  the up projection's operand leaves as special and patch rows, and ``grad_x``
+  adds the residual's gradient.
 
-With attention the adapter is a chain of nodes: the fused down GEMM
-(``AdapterDownFunction``), SparseConv2D, the concatenation and the
-reference's attention ops (LayerNorm, Linear, attention), then the same up
-GEMM epilogue for both ``shortcut + attn_proj(.) * attn_gamma`` and
-``up_proj(c) * gamma + x`` (``AdapterUpFunction`` with no special tokens: the
-A rows are the ``[B, N, .]`` input itself). The attention is evaluated in
-float32 (``_attention``).
+Other widths without attention take ``SparseConvAdapterFunction``: the same
+computation as separate calls (``opentad_sparse_ops.adapter_down``,
+``heatmap_add_``, ``fwd_packed``, ``adapter_up``), with library GEMMs for the
+input gradients, one of them ``addmm(go, du, W_d)`` with the residual's term as
+its addend. ``tokens_per_batch`` defaults to 0 (the tables the backbone builds
+are global), so there is no host sync; ``None`` restores the reference's
+``max()`` heuristic (``sparse_conv_layer.py:174-177``).
+
+With any other attention, other widths beside it, or layers that a call would
+not run as they are (hooks, a replaced ``forward``, another class) the adapter
+is a chain of nodes: the fused down GEMM (``AdapterDownFunction``),
+SparseConv2D, the concatenation and the reference's attention ops (LayerNorm,
+Linear, attention) or ``KeyTokenAttentionFunction``, then the up GEMM epilogue
+for both ``shortcut + attn_proj(.) * attn_gamma`` and ``up_proj(c) * gamma + x``
+(``AdapterUpFunction`` with no special tokens: the A rows are the ``[B, N, .]``
+input itself). PyTorch's attention is evaluated in float32 (``_attention``).
 
 The backward's weight gradients (sums over every token row) run on the
 split-row kernel of SparseConv2D's backward-weight pass with one offset
 (``opentad_sparse_ops.linear_wgrad``: deterministic, and a grid that fills the
-chip where a library GEMM with a 17k-long reduction gets a dozen workgroups);
-the input gradients use library GEMMs (``torch.matmul``). The GELU backward
-reads the special-token and patch-token gradients in place of their
-concatenation (``opentad_sparse_ops.gelu_backward_split``). ``gamma``'s
+chip where a library GEMM with a 17k-long reduction gets a dozen workgroups).
+The GELU backward reads the special-token and patch-token gradients in place of
+their concatenation (``opentad_sparse_ops.gelu_backward_split``). ``gamma``'s
 gradient needs ``z = cat(...) W_u^T + b_u``, which the fused forward never
 stores: ``sum(go * z) = <W_u, go^T c> + <b_u, sum(go)>``, and ``go^T c`` is
 the up-projection's weight-gradient reduction anyway; one launch adds both
@@ -56,11 +69,6 @@ products (``opentad_sparse_ops.gamma_grad``). The bias gradients (column sums
 over the token rows) use ``opentad_sparse_ops.column_sums``. The heatmap
 injection's backward is the gather's: a scatter-add of ``g * gate`` into the
 special-token gradient and ``sum(g * sampled)`` for the gate, in PyTorch.
-
-The input gradient is one GEMM with the residual's term as its addend
-(``addmm(go, du, W_d)``), which the single node makes possible.
-``AdapterDownFunction`` and ``AdapterUpFunction`` are the same kernels as two
-separate nodes around a ``SparseConv2d``.
 
 The fused path runs in a compute dtype ``cd`` of float16 / bfloat16:
 
