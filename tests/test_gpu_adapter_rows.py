@@ -281,3 +281,34 @@ def test_patch_rows_of_2_gib(dev):
     # the parts' roundings to float16 (hidden rows, convolution, z, output), each 2^-11 of its value
     assert float((got - want).norm() / want.norm()) <= 4 * 2.0 ** -11
     assert float((got - want).abs().max()) <= 8 * 2.0 ** -11 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("embed", [384, 768])
+def test_hooked_sparse_conv_with_key_attention(dev, embed):
+    """The layer is called, and the chain around it agrees with the one node
+    within the roundings of either; a doubling hook changes the result."""
+    import eccv26_tad_amd as sv
+
+    g = torch.Generator(device=dev).manual_seed(embed)
+    mod = sv.SparseConvAdapter(embed, 0.25, use_attn=2, n_key_tokens=2).to(dev, torch.float16)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.add_(0.1 * torch.randn(p.shape, generator=g, device=dev))
+    idx = torch.arange(40, device=dev).expand(2, -1)
+    table = sv.build_neighbor_table(torch.ones(2, 2, 4, 5, dtype=torch.uint8, device=dev), batched=True, n=80)
+    x = torch.randn(2, 42, embed, generator=g, device=dev).half().requires_grad_(True)
+    go = torch.randn(2, 42, embed, generator=g, device=dev).half()
+    wrt = [x] + [p for n, p in mod.named_parameters() if n != "k_norm.bias"]
+    scale = [1]
+
+    def step():
+        y = mod(x, 4, 5, idx, 40, table)
+        return [y.detach(), *torch.autograd.grad(y, wrt, go)]
+
+    plain = step()
+    mod.sparse_conv.register_forward_hook(lambda m, args, out: out * scale[0])
+    for a, b in zip(plain, step()):
+        # a few float16 roundings of each chain; single gains sum products that cancel
+        assert float((a - b).float().norm()) <= (4e-3 if a.numel() > 1 else 5e-2) * float(a.float().norm())
+    scale[0] = 2
+    assert float((step()[0] - plain[0]).float().norm()) > 0.05 * float(plain[0].float().norm())
